@@ -798,7 +798,7 @@ KERNELS = {  # kind -> (kernel, bound, peak FLOP/s, work unit)
     11: ("gemm3_kernel/gemm3x_kernel (split planes)", "mfma", PEAK_BF16,
          "3*M*N*rank fp16 MFMA flops executed (three fp16 products per fp32-equivalent "
          "product of one triangular operand)"),
-    3: ("leaf_kernel", "latency", PEAK_F32, "2*n^3/3"),
+    3: ("node_kernel", "latency", PEAK_F32, "2*n^3/3"),
     4: ("gptq_block_kernel", "latency", PEAK_F32, "rows*L*(L-1)"),
     5: ("refine GEMMs (refine_gradient_kernel + gptq_trailing_kernel)", "mfma", PEAK_F32,
         "2*rows*rank*cols"),

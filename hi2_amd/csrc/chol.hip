@@ -8,9 +8,7 @@
 // is needed, never L: 2K^3/3 flops.
 //
 // L^-1 is built recursively on P = J H J, in place in its lower triangle:
-//   leaf (n <= 128): one workgroup runs the same recursion on the block in LDS down to
-//     16 x 16 bases, each one wave's fused factor-and-invert sweep in registers; a node
-//     of up to 256 columns (two leaves and its four products) is one workgroup too;
+//   n <= 256: one workgroup sweeps the block's 16-column tiles in registers (node_kernel);
 //   node [A11 0; A21 A22], n1 + n2 = n, after inv_chol(A11) left A11 = L11^-1:
 //     T1  = A21 A11^T               (= L21)
 //     A22 = A22 - T1 T1^T           (lower triangle)
@@ -29,7 +27,7 @@
 namespace hi2x {
 namespace {
 
-constexpr int NB = 128;  // leaf size
+constexpr int NB = 128;  // column granule of the recursion (a node kernel takes up to two)
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_u16(const uint16_t* base, int64_t n) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), (short)0, (int)(n * 2),
@@ -1289,481 +1287,333 @@ __global__ __launch_bounds__(256) void reverse_damp4_kernel(const float* __restr
   }
 }
 
-// ---- leaf: L^-1 of chol(P[r0:r0+n, r0:r0+n]) in place (lower triangle) ---------------------
-// One workgroup of 4 waves holds the 128 x 128 block in LDS (identity beyond n, zeros
-// above the diagonal) and runs the same recursion as the host on it, down to 16 x 16:
-//   node [A11 0; A21 A22]: leaf(A11); T1 = A21 A11^T; A22 -= T1 T1^T (lower);
-//                          leaf(A22); T2 = T1 A11; A21 = -A22 T2
-// with the products on v_mfma_f32_16x16x4f32 (each product is read into registers,
-// then written back in place after a barrier).
+// ---- node: L^-1 of chol(P[r0:r0+m, r0:r0+m]) in place (lower triangle), m <= 256 ---------
+// One workgroup of 16 waves, wave w owning block column w of the block's 16 x 16 tiles, sweeps
+// the block columns c = 0, 1, ...:
 //
-// The 16 x 16 base is one wave's fused factor-and-invert sweep, lane i (< 16) holding row
-// i of the symmetric block in 16 registers (the upper triangle mirrored from the lower one
-// on load).  For c = 0..15, with d = M[c][c], r = 1/sqrt(d) and g_i = -M[i][c] r^2 on
-// the rows i > c (0 on the others):
+//   X       = inv(chol(D)), D the diagonal tile (c, c): its wave's sweep in registers (below)
+//   P_w     = X T(c, w)            every wave w != c; published in LDS where w > c
+//   T(k, w) -= P_k^T P_w           k > c (k < w where w > c; the diagonal tile is kept apart)
+//   T(k, c)  = -P_k^T X            k > c, wave c
+//
+// For c < w, T(k, w) is the Schur complement's block A[w][k] transposed; from c = w on it is
+// block (k, w) of L^-1 before row k's scaling, and final at c = k, as P_w.  So the Schur update
+// and the forward substitution of L^-1 are one product, every wave needs from the others only
+// the P_k past c, and every operand is the registers of a tile as the MFMA that made it left
+// them (the C layout: lane l holds rows 4 (l / 16) .. + 3 of column l % 16, register s being the
+// operand of k-step s of the transposed tile on the left and of the tile on the right): tiles
+// go through LDS without a transpose or a bank conflict, and only once per block column.
+//
+// What bounds it is the chain of the diagonal tiles (sweep, P of the next column, its own
+// update, a barrier on each side): the wave that owns the next one runs its sweep while the
+// others apply the update.  A 256-column node takes 39 us and a 128-column one 27 (84-88
+// and 31 us as recursive 16/32/64/128-column halves in 135 KB of LDS, whose sweeps, small
+// products and barriers followed one another); with 26 KB of LDS it also finds a CU beside
+// another stream's GEMM workgroups.
+//
+// The 16 x 16 sweep is one wave's fused factor-and-invert of the symmetric tile, lane 16 g + i
+// holding columns 4g .. 4g + 3 of row i (the C layout, by symmetry).  For c = 0..15, with
+// d = M[c][c] and g_i = -M[i][c] / d on the rows i > c (0 on the others):
 //   every j != c:  M[i][j] += g_i M[c][j]
-//     (j > c: the Schur update T[i][j] -= l_i l_j, l_k = T[k][c] r, with T[j][c] = T[c][j]
-//      by symmetry; j < c: the forward substitution B[i][j] -= l_i X[c][j], where row c of
-//      L^-1 is X[c][j] = B[c][j] r)
-//   rows i > c:    M[i][c] = g_i   (= -l_i r, column c of L^-1 before row i's scaling).
-// Row c is then final up to its scale, which is applied once after the sweep:
-// X[c][j] = M[c][j] r_c (j < c), X[c][c] = r_c.  Every multiplier is one of lane c's own
-// registers, broadcast to each row of 16 lanes by DPP (row_newbcast) inside
-// v_fmac_f32_dpp: one instruction per register and column, no barrier and no LDS traffic
-// in the sweep.  The reciprocal and square root are the hardware approximations (the
-// factor is compared to a tolerance, not bit for bit).
-constexpr int LP = NB + 4;  // LDS pitch of the leaf block (floats)
-#ifndef HI2X_LEAF_SPLIT
-#define HI2X_LEAF_SPLIT 1
-#endif
-constexpr bool LEAF_SPLIT = HI2X_LEAF_SPLIT;
+//     (j > c: the Schur update T[i][j] -= l_i l_j, l_k = T[k][c] / sqrt(d), with
+//      T[j][c] = T[c][j] by symmetry; j < c: the forward substitution)
+//   rows i > c:    M[i][c] = g_i   (column c of L^-1 before row i's scaling).
+// Row c is then final up to its scale r_c = 1/sqrt(d), which is applied once after the
+// sweep: X[c][j] = M[c][j] r_c (j < c), X[c][c] = r_c.  Row c reaches the other rows by DPP
+// (row_newbcast) inside v_fmac_f32_dpp, column c the other lane rows by two lane swaps: no
+// barrier and no LDS traffic.  The reciprocal and reciprocal square root are the hardware
+// approximations (1 ulp, the second refined once; the factor is compared to a tolerance, not
+// bit for bit).
+constexpr int ND_B = 16;             // tile edge
+constexpr int ND_N = 2 * NB / ND_B;  // block columns of the largest node, one wave each
+constexpr int ND_G = 2;              // tiles updated at a time
 
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 
-// v[j] += bcast_C(v[j]) * g for the 15 registers j != C, bcast_C = lane C of each row of 16
-// lanes.  The compiler does not fold a DPP move into an FMA (v_fma_f32 has no DPP form on
-// this target), so the fused instructions are written out.  The leading s_nop 4 gives the
-// five wait states a DPP instruction needs after a VALU write of its source VGPR (two) or
-// of EXEC (five); inside the block no instruction reads a register another one writes.
-#define HI2X_FMAC_DPP(k, C) \
-  "v_fmac_f32_dpp %" #k ", %" #k ", %15 row_newbcast:" #C " row_mask:0xf bank_mask:0xf\n\t"
-#define HI2X_FMAC15(C)                                                                     \
-  "s_nop 4\n\t" HI2X_FMAC_DPP(0, C) HI2X_FMAC_DPP(1, C) HI2X_FMAC_DPP(2, C)              \
-      HI2X_FMAC_DPP(3, C) HI2X_FMAC_DPP(4, C) HI2X_FMAC_DPP(5, C) HI2X_FMAC_DPP(6, C)     \
-          HI2X_FMAC_DPP(7, C) HI2X_FMAC_DPP(8, C) HI2X_FMAC_DPP(9, C) HI2X_FMAC_DPP(10, C) \
-              HI2X_FMAC_DPP(11, C) HI2X_FMAC_DPP(12, C) HI2X_FMAC_DPP(13, C)               \
-                  HI2X_FMAC_DPP(14, C)
-#define HI2X_J(k) ((k) < C ? (k) : (k) + 1)
-#define HI2X_ROW_OPS                                                                   \
-  "+v"(v[HI2X_J(0)]), "+v"(v[HI2X_J(1)]), "+v"(v[HI2X_J(2)]), "+v"(v[HI2X_J(3)]),     \
-      "+v"(v[HI2X_J(4)]), "+v"(v[HI2X_J(5)]), "+v"(v[HI2X_J(6)]), "+v"(v[HI2X_J(7)]), \
-      "+v"(v[HI2X_J(8)]), "+v"(v[HI2X_J(9)]), "+v"(v[HI2X_J(10)]),                    \
-      "+v"(v[HI2X_J(11)]), "+v"(v[HI2X_J(12)]), "+v"(v[HI2X_J(13)]),                  \
-      "+v"(v[HI2X_J(14)])
-template <int C>
-__device__ __forceinline__ void fmac_row(float (&v)[16], float g) {
-  static_assert(C >= 0 && C < 16, "column of the 16 x 16 base");
-  if constexpr (C == 0) asm(HI2X_FMAC15(0) : HI2X_ROW_OPS : "v"(g));
-  else if constexpr (C == 1) asm(HI2X_FMAC15(1) : HI2X_ROW_OPS : "v"(g));
-  else if constexpr (C == 2) asm(HI2X_FMAC15(2) : HI2X_ROW_OPS : "v"(g));
-  else if constexpr (C == 3) asm(HI2X_FMAC15(3) : HI2X_ROW_OPS : "v"(g));
-  else if constexpr (C == 4) asm(HI2X_FMAC15(4) : HI2X_ROW_OPS : "v"(g));
-  else if constexpr (C == 5) asm(HI2X_FMAC15(5) : HI2X_ROW_OPS : "v"(g));
-  else if constexpr (C == 6) asm(HI2X_FMAC15(6) : HI2X_ROW_OPS : "v"(g));
-  else if constexpr (C == 7) asm(HI2X_FMAC15(7) : HI2X_ROW_OPS : "v"(g));
-  else if constexpr (C == 8) asm(HI2X_FMAC15(8) : HI2X_ROW_OPS : "v"(g));
-  else if constexpr (C == 9) asm(HI2X_FMAC15(9) : HI2X_ROW_OPS : "v"(g));
-  else if constexpr (C == 10) asm(HI2X_FMAC15(10) : HI2X_ROW_OPS : "v"(g));
-  else if constexpr (C == 11) asm(HI2X_FMAC15(11) : HI2X_ROW_OPS : "v"(g));
-  else if constexpr (C == 12) asm(HI2X_FMAC15(12) : HI2X_ROW_OPS : "v"(g));
-  else if constexpr (C == 13) asm(HI2X_FMAC15(13) : HI2X_ROW_OPS : "v"(g));
-  else if constexpr (C == 14) asm(HI2X_FMAC15(14) : HI2X_ROW_OPS : "v"(g));
-  else asm(HI2X_FMAC15(15) : HI2X_ROW_OPS : "v"(g));
+// x += bcast_C(x) * g, bcast_C = lane C of each row of 16 lanes.  The compiler does not fold
+// a DPP move into an FMA (v_fma_f32 has no DPP form on this target), so the fused
+// instructions are written out.  A DPP instruction needs two wait states after a VALU write
+// of its source VGPR: the leading s_nop 1 gives them, and inside a block no instruction reads
+// a register another one writes.
+#define HI2X_FMAC_DPP(k, g, c) \
+  "v_fmac_f32_dpp %" #k ", %" #k ", %" #g " row_newbcast:" #c " row_mask:0xf bank_mask:0xf\n\t"
+#define HI2X_FMAC_CASE(c)                                                                    \
+  if constexpr (C == c) {                                                                    \
+    asm("s_nop 1\n\t" HI2X_FMAC_DPP(0, 1, c) : "+v"(x) : "v"(g));                            \
+    then();                                                                                  \
+    asm("s_nop 1\n\t" HI2X_FMAC_DPP(0, 3, c) HI2X_FMAC_DPP(1, 3, c) HI2X_FMAC_DPP(2, 3, c)   \
+        : "+v"(y0), "+v"(y1), "+v"(y2) : "v"(g));                                            \
+  }
+// x first, then() and the three others
+template <int C, class Then>
+__device__ __forceinline__ void fmac_bcast(float& x, float& y0, float& y1, float& y2, float g,
+                                           Then then) {
+  static_assert(C >= 0 && C < 16, "lane of a 16-lane row");
+  HI2X_FMAC_CASE(0) HI2X_FMAC_CASE(1) HI2X_FMAC_CASE(2) HI2X_FMAC_CASE(3)
+  HI2X_FMAC_CASE(4) HI2X_FMAC_CASE(5) HI2X_FMAC_CASE(6) HI2X_FMAC_CASE(7)
+  HI2X_FMAC_CASE(8) HI2X_FMAC_CASE(9) HI2X_FMAC_CASE(10) HI2X_FMAC_CASE(11)
+  HI2X_FMAC_CASE(12) HI2X_FMAC_CASE(13) HI2X_FMAC_CASE(14) HI2X_FMAC_CASE(15)
 }
-#undef HI2X_ROW_OPS
-#undef HI2X_J
-#undef HI2X_FMAC15
+#undef HI2X_FMAC_CASE
 #undef HI2X_FMAC_DPP
 
-// Column C of the sweep.  Lane i keeps its own pivot in pv (rows below C take theirs at
-// their own column, so i >= C is the previous column's i > C).  M[i][C] becomes g on every
-// row: the rows below need it, and lane C's and the finished rows' registers C are not
-// read again before the final scaling overwrites them.
+// Lane l's copy of lane 16 G + l % 16: the 16-lane row G in every row.
+template <int G>
+__device__ __forceinline__ float row_all(float x) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  const auto h = __builtin_amdgcn_permlane32_swap(u, u, false, false);  // rows {0, 1} / {2, 3} twice
+  const uint32_t y = h[G >> 1];
+  const auto r = __builtin_amdgcn_permlane16_swap(y, y, false, false);  // the even / the odd row
+  return __builtin_bit_cast(float, (uint32_t)r[G & 1]);
+}
+
+// Column C of the sweep (v[e] = M[i][4g + e] in lane 16 g + i), d its pivot and rc about 1/d.
+// The column's multipliers go to all four lane rows by two lane swaps; the register of column
+// C + 1 is updated first, and the next pivot's reciprocal runs beside the other updates.
+// M[i][C] becomes g on every row: the rows below C need it, and the others are overwritten by
+// the final scaling.
 template <int C>
-__device__ __forceinline__ void base_step(float (&v)[16], int i, float& pv) {
-  const float d = __builtin_bit_cast(
-      float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v[C]), C));  // pivot M[c][c]
-  const float rp = __builtin_amdgcn_rcpf(__builtin_amdgcn_sqrtf(d));
-  const float gv = v[C] * -(rp * rp);
-  fmac_row<C>(v, i > C ? gv : 0.0f);
-  v[C] = gv;
-  pv = i >= C ? d : pv;
+__device__ __forceinline__ void base_step(float (&v)[4], int i, int lg, float& pv, float& d,
+                                          float& rc) {
+  constexpr int G = C >> 2, E = C & 3, N = (C + 1) & 15;
+  const float gv = row_all<G>(v[E]) * -rc;
+  const float g = i > C ? gv : 0.0f;
+  pv = i == C ? d : pv;
+  fmac_bcast<C>(v[(E + 1) & 3], v[(E + 2) & 3], v[(E + 3) & 3], v[E], g, [&]() {
+    if constexpr (C < 15) {
+      d = __builtin_bit_cast(
+          float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v[(E + 1) & 3]), 16 * (N >> 2) + N));
+      rc = __builtin_amdgcn_rcpf(d);
+    }
+  });
+  v[E] = lg == G ? gv : v[E];
 }
 
 template <int... Cs>
-__device__ __forceinline__ void base_steps(float (&v)[16], int i, float& pv,
+__device__ __forceinline__ void base_steps(float (&v)[4], int i, int lg, float& pv,
                                            std::integer_sequence<int, Cs...>) {
-  (base_step<Cs>(v, i, pv), ...);
+  float d = __builtin_bit_cast(float,
+                               __builtin_amdgcn_readlane(__builtin_bit_cast(int, v[0]), 0));
+  float rc = __builtin_amdgcn_rcpf(d);
+  (base_step<Cs>(v, i, lg, pv, d, rc), ...);
 }
 
-// 16 x 16 block at (o, o): one wave (the caller's wave 0), lane i holds row i % 16 (lanes
-// 16..63 repeat rows 0..15 and do not write back).  Only the block's lower triangle is
-// read: row i below the diagonal, column i (M[j][i] for j > i) as the upper half.
-__device__ __forceinline__ void leaf_base16(float* S, int o, bool& bad) {
-  const int l = threadIdx.x & 63, i = l & 15;
-  float* row = &S[(o + i) * LP + o];
-  float v[16], t[16];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const float4 x = *reinterpret_cast<const float4*>(row + 4 * q);
-    v[4 * q] = x.x;
-    v[4 * q + 1] = x.y;
-    v[4 * q + 2] = x.z;
-    v[4 * q + 3] = x.w;
-  }
-#pragma unroll
-  for (int j = 0; j < 16; ++j) t[j] = S[(o + j) * LP + o + i];
-#pragma unroll
-  for (int j = 0; j < 16; ++j) v[j] = j > i ? t[j] : v[j];
+// X = inv(chol(D)) of the symmetric tile d (C layout, so lane 16 g + i holds columns
+// 4g .. 4g + 3 of row i): one wave.  xs receives X in the same layout, which is the left MFMA
+// operand's, and rows < rows of X go to byte offset off + 4 i ld of rs.  True when a pivot
+// was not positive (or NaN).
+__device__ __forceinline__ bool node_base(const f32x4v& d, f32x4v* xs, __amdgpu_buffer_rsrc_t rs,
+                                          uint32_t off, int64_t ld, int rows) {
+  int l = threadIdx.x & 63;
+  asm volatile("" : "+v"(l));
+  const int i = l & 15, lg = l >> 4;
+  float v[4] = {d[0], d[1], d[2], d[3]};
   float pv = 0.0f;
-  base_steps(v, i, pv, std::make_integer_sequence<int, 16>{});
-  // a pivot not positive (or NaN) anywhere in the block; the same r_i as in the sweep
-  bad = bad || __builtin_amdgcn_ballot_w64(!(pv > 0.0f)) != 0;
-  const float r = __builtin_amdgcn_rcpf(__builtin_amdgcn_sqrtf(pv));
-  // row i of L^-1: X[i][j] = M[i][j] r_i (j < i), X[i][i] = r_i; the block stays lower
+  base_steps(v, i, lg, pv, std::make_integer_sequence<int, 16>{});
+  const bool bad = __builtin_amdgcn_ballot_w64(!(pv > 0.0f)) != 0;
+  float r = __builtin_amdgcn_rsqf(pv);
+  r = __builtin_fmaf(0.5f * r, __builtin_fmaf(-pv * r, r, 1.0f), r);  // one Newton step
+  // row i of L^-1: X[i][j] = M[i][j] r_i (j < i), X[i][i] = r_i, zeros above
+  f32x4v x;
 #pragma unroll
-  for (int j = 0; j < 16; ++j) v[j] = j < i ? v[j] * r : (j == i ? r : 0.0f);
-  if (l < 16) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      *reinterpret_cast<float4*>(row + 4 * q) =
-          make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+  for (int e = 0; e < 4; ++e) {
+    const int j = 4 * lg + e;
+    x[e] = j < i ? v[e] * r : (j == i ? r : 0.0f);
   }
+  xs[l] = x;
+  // rows and columns past rows are identity padding (rows is a multiple of 4)
+  const uint32_t o = (i < rows && 4 * lg < rows) ? off + (uint32_t)((i * ld + 4 * lg) * 4) : MG_OOB;
+  __builtin_amdgcn_raw_buffer_store_b128(
+      __builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned, x), rs, (int)o, 0, 0);
+  return bad;
 }
 
-// C[H x H] at (cr, cc) = alpha * A (at (ar, ac)) * op(B) (at (br, bc)), op(B) = B^T when
-// TB; with LOWER, C += alpha * A op(B) on the lower triangle of C only.  Every block is in
-// the leaf's LDS; the result is written after all inputs have been read (C may alias).
-// For each 16 k: lane group g = l/16 supplies k = 16 kb + 4 g + s at MFMA step s, so a
-// lane reads its 4 k of A (and of B^T) as one 16-byte vector.
-template <int H>
-struct ProdAcc {  // this wave's tiles of an H x H product (tile t = wave + 4p, p < PER)
-  static constexpr int NT = H / 16, TILES = NT * NT, PER = (TILES + 3) / 4;
-  f32x4v acc[PER];
-};
+// A^T B of two tiles in the C layout
+__device__ __forceinline__ f32x4v tile_mma(const f32x4v& a, const f32x4v& b) {
+  f32x4v p = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+    p = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], p, 0, 0, 0);
+  return p;
+}
 
-// Three bf16 planes of 8 consecutive k of one lane's fragment: x1 = bf16(x),
-// x2 = bf16(x - x1), x3 = bf16(x - x1 - x2) (the differences are exact in fp32; bf16 has
-// fp32's exponent range, so no row scale is needed).  Pairs go through
-// v_cvt_pk_bf16_f32; a bf16 back to fp32 is its bits in the upper half of the word.
+// Three bf16 planes of four values, x1 = bf16(x), x2 = bf16(x - x1), x3 = bf16(x - x1 - x2)
+// (the differences are exact in fp32; bf16 has fp32's exponent range, so no scale is needed).
+// Pairs go through v_cvt_pk_bf16_f32; a bf16 back to fp32 is its bits in the upper half.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2v __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void split8(const float4 x0, const float4 x1, bf16x8 (&o)[3]) {
-  const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-  uint32_t w[3][4];
+__device__ __forceinline__ void split4(const f32x4v& x, uint2 (&o)[3]) {
+  uint32_t u[2][3];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    float lo = x[2 * e], hi = x[2 * e + 1];
+  for (int h = 0; h < 2; ++h) {
+    float a = x[2 * h], b = x[2 * h + 1];
 #pragma unroll
     for (int pl = 0; pl < 3; ++pl) {
-      const uint32_t u =
-          __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2v){lo, hi}, bf16x2));
-      w[pl][e] = u;
+      u[h][pl] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2v){a, b}, bf16x2));
       if (pl < 2) {
-        lo = lo - __builtin_bit_cast(float, u << 16);
-        hi = hi - __builtin_bit_cast(float, u & 0xffff0000u);
+        a = a - __builtin_bit_cast(float, u[h][pl] << 16);
+        b = b - __builtin_bit_cast(float, u[h][pl] & 0xffff0000u);
       }
     }
   }
 #pragma unroll
-  for (int pl = 0; pl < 3; ++pl)
-    o[pl] = __builtin_bit_cast(bf16x8, (uint4){w[pl][0], w[pl][1], w[pl][2], w[pl][3]});
+  for (int pl = 0; pl < 3; ++pl) o[pl] = make_uint2(u[0][pl], u[1][pl]);
+}
+__device__ __forceinline__ bf16x8 plane_pair(const uint2& a, const uint2& b) {
+  return __builtin_bit_cast(bf16x8, make_uint4(a.x, a.y, b.x, b.y));
 }
 
-// acc = A op(B) for the node's 128 x 128 blocks on bf16 MFMA through the three-way split
-// (the six terms x_i y_j with i + j <= 2, small terms first; the big products' scaled
-// two-plane fp16 split measured slower here, its row maxima and conversions back to
-// fp32 costing the VALU time its halved MFMAs save):
-// v_mfma_f32_16x16x32_bf16 (lane l: row or column l % 16, k 8 (l / 16) .. + 7; the
-// accumulator layout of the fp32 16x16x4 MFMA), six 16-cycle MFMAs per 32 k where the
-// fp32 MFMA takes eight of 32 cycles.  The wave's tiles t = wave + 4p are tile row p / 2,
-// column wave + 4 (p % 2): per 32 k its two column fragments are split first, then the
-// eight row fragments two at a time, each pair's 24 MFMAs (four accumulators in turn)
-// covering the split of the next pair.  fp32-level rounding, not bit-identical to the
-// fp32 MFMA.  (Blocks of 64 and below stay on fp32 MFMA: with a row fragment used by
-// one tile, the split costs more VALU time than the MFMA time it saves.)
-template <bool TB>
-__device__ __forceinline__ void node_mma3(const float* S, int ar, int ac, int br, int bc,
-                                          ProdAcc<128>& P) {
-  constexpr int PER = ProdAcc<128>::PER;
-  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
-  const int lr = l & 15, lg = l >> 4;
+// P^T Q of two tiles in the C layout on bf16 MFMA through their planes, six of the nine terms
+// (p_i q_j with i + j <= 4, the dropped ones below 2^-24 |p q|), small ones first: the 16 k of
+// a tile take half of a 32-k step, so two terms share one (lane group g holds k = 4g .. 4g + 3
+// of one plane in the lower and of another in the upper half of its eight).  48 cycles of the
+// matrix core instead of the fp32 MFMA's 128.  a: P's planes 2 | 1, a3 its plane 3;
+// b1 = 1 | 1, b2 = 2 | 2 and b3 = 3 | 1 of Q.
+__device__ __forceinline__ f32x4v plane_mma(const uint4& a, const uint2& a3, const bf16x8& b1,
+                                            const bf16x8& b2, const bf16x8& b3) {
+  const bf16x8 a21 = __builtin_bit_cast(bf16x8, a);
+  const bf16x8 a13 = __builtin_bit_cast(bf16x8, make_uint4(a.z, a.w, a3.x, a3.y));
+  f32x4v q = {0.0f, 0.0f, 0.0f, 0.0f};
+  q = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a13, b3, q, 0, 0, 0);
+  q = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a21, b2, q, 0, 0, 0);
+  q = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a21, b1, q, 0, 0, 0);
+  return q;
+}
+
+// d -= q with the rounding error of every subtraction carried to the next one in dc.  A
+// diagonal tile takes one subtraction per block column before its sweep; compensated, the
+// whole factor is as close to 64 bits as with one subtraction per 64 or 128 columns (K = 1024:
+// 3.6e-6 of U, 4.4e-6 without).
+__device__ __forceinline__ void sub_comp(f32x4v& d, f32x4v& dc, const f32x4v& q) {
+  const f32x4v y = -q - dc, t = d + y;
+  dc = (t - d) - y;
+  d = t;
+}
+
+// A workgroup barrier that orders LDS accesses only: __syncthreads() would also wait for the
+// wave's stores of finished blocks to reach memory, about a microsecond each time.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+struct NodeSmem {
+  uint4 A[ND_N][64];   // planes 2 and 1 of P_j of the current block column
+  uint2 A3[ND_N][64];  // its plane 3
+  f32x4v X[2][64];     // inverse of the diagonal tile's factor
+};
+
+__global__ __launch_bounds__(64 * ND_N) void node_kernel(float* __restrict__ P, int64_t K,
+                                                         int64_t r0, int m,
+                                                         int* __restrict__ status, int64_t sP) {
+  __shared__ NodeSmem sm;
+  P += (int64_t)blockIdx.z * sP + r0 * K + r0;
+  status += blockIdx.z;
+  int l = threadIdx.x & 63, ln = l & 15, lg = l >> 4;
+  // the block column of this wave: each SIMD's four waves (id % 4) get columns s, 7 - s,
+  // 8 + s and 15 - s, which share the updates evenly
+  const int id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), sid = id & 3;
+  const int w = (id >> 2) == 0 ? sid : (id >> 2) == 1 ? 7 - sid : (id >> 2) == 2 ? 8 + sid : 15 - sid;
+  const int nb = (m + ND_B - 1) / ND_B;
+  // tile (k, w), k <= w: register j of lane l is A[16 w + l % 16][16 k + 4 (l / 16) + j], zeros
+  // past m.
+  // m and K are multiples of 4 (the entry points require it of K), so a 16-byte vector is all
+  // in or all out.
+  const __amdgpu_buffer_rsrc_t rs = mg_rsrc(P, (int64_t)(m - 1) * K + m);
+  // the diagonal tile first (wave 0's sweep waits for nothing else): its upper half from its
+  // lower one, identity past m
+  f32x4v d, dc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-  for (int p = 0; p < PER; ++p) P.acc[p] = (f32x4v){0.0f, 0.0f, 0.0f, 0.0f};
-  constexpr int PA[6] = {2, 1, 0, 1, 0, 0}, PB[6] = {0, 1, 2, 0, 1, 0};
+  for (int j = 0; j < 4; ++j) {
+    const int r = ND_B * w + 4 * lg + j, c = ND_B * w + ln;
+    const uint32_t off = (uint32_t)((r > c ? (int64_t)r * K + c : (int64_t)c * K + r) * 4);
+    const float u = __builtin_bit_cast(
+        float, __builtin_amdgcn_raw_buffer_load_b32(rs, (int)(r < m && c < m ? off : MG_OOB), 0, 0));
+    d[j] = r < m && c < m ? u : (r == c ? 1.0f : 0.0f);
+  }
+  float acc[ND_N][4];
+#pragma unroll
+  for (int k = 0; k < ND_N; ++k) {
+    const int r = ND_B * w + ln, c = ND_B * k + 4 * lg;
+    const uint32_t off = (k < w && r < m && c < m) ? (uint32_t)(((int64_t)r * K + c) * 4) : MG_OOB;
+    const f32x4 x = mg_load4(rs, off);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[k][j] = x[j];
+  }
+  float nxt[4] = {acc[0][0], acc[0][1], acc[0][2], acc[0][3]};  // the wave's tile c of the next c
+  bool bad = false;
 #pragma unroll 1
-  for (int kb = 0; kb < 128; kb += 32) {
-    const int k = kb + 8 * lg;
-    bf16x8 b[2][3];
-#pragma unroll
-    for (int ci = 0; ci < 2; ++ci) {
-      const int tc = wave + 4 * ci;
-      float4 x0, x1;
-      if (TB) {
-        const float* bp = &S[(br + tc * 16 + lr) * LP + bc + k];
-        x0 = *reinterpret_cast<const float4*>(bp);
-        x1 = *reinterpret_cast<const float4*>(bp + 4);
-      } else {
-        const float* bp = &S[(br + k) * LP + bc + tc * 16 + lr];
-        x0 = make_float4(bp[0], bp[LP], bp[2 * LP], bp[3 * LP]);
-        x1 = make_float4(bp[4 * LP], bp[5 * LP], bp[6 * LP], bp[7 * LP]);
+  for (int c = -1; c < nb; ++c) {
+    // the lane's addresses are rebuilt at each use instead of being held across the loop
+    // (the tiles take half of the 128 registers that sixteen waves leave a lane)
+    asm volatile("" : "+v"(l));
+    ln = l & 15, lg = l >> 4;
+    f32x4v p;    // P_w
+    uint2 y[3];  // its planes
+    if (c >= 0) {
+      lds_barrier();  // X is there and the update of column c - 1 is complete
+      if (w > c) {
+        p = tile_mma(sm.X[c & 1][l], (f32x4v){nxt[0], nxt[1], nxt[2], nxt[3]});
+        split4(p, y);
+        sm.A[w][l] = make_uint4(y[1].x, y[1].y, y[0].x, y[0].y);
+        sm.A3[w][l] = y[2];
+        if (w == c + 1) sub_comp(d, dc, tile_mma(p, p));
       }
-      split8(x0, x1, b[ci]);
+      lds_barrier();  // every P_j, j > c, is there
     }
+    if (w == c + 1 && w < nb) {  // the sweep of its diagonal tile, beside the other updates
+      __builtin_amdgcn_s_setprio(3);
+      const uint32_t o = (uint32_t)((int64_t)ND_B * w * (K + 1) * 4);
+      bad = node_base(d, sm.X[w & 1], rs, o, K, m - ND_B * w);
+      __builtin_amdgcn_s_setprio(0);
+    }
+    if (c < 0 || w == c + 1) continue;
+    if (w > c) {
+      sub_comp(d, dc, tile_mma(p, p));
+    } else if (w < c) {  // block (c, w) of L^-1 is final
+      p = tile_mma(sm.X[c & 1][l], (f32x4v){nxt[0], nxt[1], nxt[2], nxt[3]});
+      const int r = ND_B * c + 4 * lg, cc = ND_B * w + ln;
 #pragma unroll
-    for (int rp = 0; rp < 4; ++rp) {
-      bf16x8 a[2][3];
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const float* ap = &S[(ar + (2 * rp + q) * 16 + lr) * LP + ac + k];
-        split8(*reinterpret_cast<const float4*>(ap), *reinterpret_cast<const float4*>(ap + 4),
-               a[q]);
+      for (int j = 0; j < 4; ++j) {
+        const float x = p[j];
+        const uint32_t off = r + j < m ? (uint32_t)(((int64_t)(r + j) * K + cc) * 4) : MG_OOB;
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), rs, (int)off, 0, 0);
       }
-#pragma unroll
-      for (int pr = 0; pr < 6; ++pr)
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-#pragma unroll
-          for (int ci = 0; ci < 2; ++ci) {
-            const int p = 2 * (2 * rp + q) + ci;
-            P.acc[p] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[q][PA[pr]], b[ci][PB[pr]],
-                                                                P.acc[p], 0, 0, 0);
-          }
+      split4(p, y);
+    } else {  // X as the right operand: register s is X[4 (l / 16) + s][l % 16]
+      const float* x = reinterpret_cast<const float*>(&sm.X[c & 1][16 * (ln >> 2) + 4 * lg]) + (ln & 3);
+      split4((f32x4v){x[0], x[4], x[8], x[12]}, y);
     }
-  }
-}
-
-// acc = A (at (ar, ac)) * op(B) (at (br, bc)), H x H blocks of the leaf's LDS, op(B) = B^T
-// when TB (the 128 blocks take the split product above).  For each 16 k: lane group g = l/16 supplies k = 16 kb + 4 g + s at MFMA step
-// s, so a lane reads its 4 k of A (and of B^T) as one 16-byte vector.
-template <int H, bool TB>
-__device__ __forceinline__ void leaf_mma(const float* S, int ar, int ac, int br, int bc,
-                                         ProdAcc<H>& P) {
-  if constexpr (H == 128 && LEAF_SPLIT) {
-    node_mma3<TB>(S, ar, ac, br, bc, P);
-    return;
-  }
-  constexpr int NT = ProdAcc<H>::NT, TILES = ProdAcc<H>::TILES, PER = ProdAcc<H>::PER;
-  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
-  const int lr = l & 15, lg = l >> 4;
+    const bf16x8 b1 = plane_pair(y[0], y[0]), b2 = plane_pair(y[1], y[1]), b3 = plane_pair(y[2], y[0]);
+    // tile k loses P_k^T P_w (on wave c: becomes -P_k^T X), k below w where w > c (its diagonal
+    // tile is d, and the tiles past it do not exist yet).  A few tiles at a time, so that their
+    // operand reads and chains of MFMAs overlap; the ones at or before c or past the end among
+    // them are dead.
+    const int kend = w > c ? w : nb;
 #pragma unroll
-  for (int p = 0; p < PER; ++p) {
-    const int t = wave + 4 * p;
-    P.acc[p] = (f32x4v){0.0f, 0.0f, 0.0f, 0.0f};
-    if (t < TILES) {
-      const int tr = t / NT, tc = t % NT;
+    for (int k0 = 0; k0 < ND_N; k0 += ND_G) {
+      if (k0 + ND_G - 1 > c && k0 < kend) {
+        f32x4v q[ND_G];
 #pragma unroll
-      for (int kb = 0; kb < H; kb += 16) {
-        const int k = kb + 4 * lg;
-        const float4 a = *reinterpret_cast<const float4*>(&S[(ar + tr * 16 + lr) * LP + ac + k]);
-        float4 b;
-        if (TB) {
-          b = *reinterpret_cast<const float4*>(&S[(br + tc * 16 + lr) * LP + bc + k]);
-        } else {
-          const float* bp = &S[(br + k) * LP + bc + tc * 16 + lr];
-          b = make_float4(bp[0], bp[LP], bp[2 * LP], bp[3 * LP]);
+        for (int e = 0; e < ND_G; ++e)
+          q[e] = plane_mma(sm.A[k0 + e][l], sm.A3[k0 + e][l], b1, b2, b3);
+#pragma unroll
+        for (int e = 0; e < ND_G; ++e)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[k0 + e][j] = (w == c ? 0.0f : acc[k0 + e][j]) - q[e][j];
+        if (k0 <= c + 1) {  // the group of tile c + 1 (at most one that updates can hold it)
+#pragma unroll
+          for (int e = 0; e < ND_G; ++e)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) nxt[j] = k0 + e == c + 1 ? acc[k0 + e][j] : nxt[j];
         }
-        P.acc[p] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, P.acc[p], 0, 0, 0);
-        P.acc[p] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, P.acc[p], 0, 0, 0);
-        P.acc[p] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, P.acc[p], 0, 0, 0);
-        P.acc[p] = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, P.acc[p], 0, 0, 0);
       }
     }
   }
-}
-
-// (row, col) within the H x H product of register j of tile p of this lane
-template <int H>
-__device__ __forceinline__ int prod_row(int p, int j) {
-  const int t = (threadIdx.x >> 6) + 4 * p;
-  return (t / ProdAcc<H>::NT) * 16 + 4 * ((threadIdx.x & 63) >> 4) + j;
-}
-template <int H>
-__device__ __forceinline__ int prod_col(int p) {
-  const int t = (threadIdx.x >> 6) + 4 * p;
-  return (t % ProdAcc<H>::NT) * 16 + (threadIdx.x & 15);
-}
-template <int H>
-__device__ __forceinline__ bool prod_live(int p) {
-  return (threadIdx.x >> 6) + 4 * p < ProdAcc<H>::TILES;
-}
-
-// C[H x H] at (cr, cc) = alpha * A op(B); with LOWER, C += alpha * A op(B) on the lower
-// triangle of C only.  The result is written after all inputs have been read (C may
-// alias an input).
-template <int H, bool TB, bool LOWER>
-__device__ __forceinline__ void leaf_prod(float* S, int ar, int ac, int br, int bc, int cr,
-                                          int cc, float alpha) {
-  ProdAcc<H> P;
-  leaf_mma<H, TB>(S, ar, ac, br, bc, P);
-  __syncthreads();
-#pragma unroll
-  for (int p = 0; p < ProdAcc<H>::PER; ++p) {
-    if (!prod_live<H>(p)) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int r = prod_row<H>(p, j), c = prod_col<H>(p);
-      const float x = P.acc[p][j];
-      float* d = &S[(cr + r) * LP + cc + c];
-      if (LOWER) {
-        if (c <= r) *d = *d + alpha * x;
-      } else {
-        *d = alpha * x;
-      }
-    }
-  }
-  __syncthreads();
-}
-
-// returns true when a pivot of this block was not positive (wave 0's view)
-template <int N>
-__device__ __forceinline__ bool leaf_rec(float* S, int o) {
-  if constexpr (N == 16) {
-    bool bad = false;
-    if ((threadIdx.x >> 6) == 0) leaf_base16(S, o, bad);
-    __syncthreads();
-    return bad;
-  } else {
-    constexpr int H = N / 2;
-    bool bad = leaf_rec<H>(S, o);
-    leaf_prod<H, true, false>(S, o + H, o, o, o, o + H, o, 1.0f);             // T1
-    leaf_prod<H, true, true>(S, o + H, o, o + H, o, o + H, o + H, -1.0f);      // A22 -= T1 T1^T
-    bad = leaf_rec<H>(S, o + H) || bad;
-    leaf_prod<H, false, false>(S, o + H, o, o, o, o + H, o, 1.0f);            // T2 = T1 A11
-    leaf_prod<H, false, false>(S, o + H, o + H, o + H, o, o + H, o, -1.0f);   // -A22 T2
-    return bad;
-  }
-}
-
-// Rows [0, n) x columns [0, n) of the n x n diagonal block at P (row stride K) into the
-// LDS block at row offset so of S: lower triangle, zeros above, identity beyond n.  The
-// buffer ends at the block's last element: rows past n read zero; n and K are multiples
-// of 4 (the entry points require it of K), so every 16-byte vector is all in or all out.
-__device__ __forceinline__ void leaf_load(float* S, int so, const float* P, int64_t K, int n) {
-  const __amdgpu_buffer_rsrc_t rs = mg_rsrc(P, (int64_t)(n - 1) * K + n);
-  constexpr int V = NB / 4;  // float4 per row
-  const int tid = threadIdx.x;
-  float4 x[NB * V / 256];
-#pragma unroll
-  for (int q = 0; q < NB * V / 256; ++q) {
-    const int idx = tid + 256 * q, i = idx / V, j = 4 * (idx % V);
-    const uint32_t off = (i < n && j < n) ? (uint32_t)(((int64_t)i * K + j) * 4) : MG_OOB;
-    x[q] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
-  }
-#pragma unroll
-  for (int q = 0; q < NB * V / 256; ++q) {
-    const int idx = tid + 256 * q, i = idx / V, j = 4 * (idx % V);
-    float e[4] = {x[q].x, x[q].y, x[q].z, x[q].w};
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int jj = j + t;
-      e[t] = (i < n && jj < n) ? (jj <= i ? e[t] : 0.0f) : (i == jj ? 1.0f : 0.0f);
-    }
-    *reinterpret_cast<float4*>(&S[(so + i) * LP + j]) = make_float4(e[0], e[1], e[2], e[3]);
-  }
-}
-
-// The LDS block at row offset so back to rows [0, n) x columns [0, n) at P in full
-// vectors: the zeros above the diagonal land in P's upper triangle, which nothing reads
-// before the final reflection overwrites it.
-__device__ __forceinline__ void leaf_store(const float* S, int so, float* P, int64_t K, int n) {
-  const __amdgpu_buffer_rsrc_t rs = mg_rsrc(P, (int64_t)(n - 1) * K + n);
-  constexpr int V = NB / 4;
-  const int tid = threadIdx.x;
-#pragma unroll
-  for (int q = 0; q < NB * V / 256; ++q) {
-    const int idx = tid + 256 * q, i = idx / V, j = 4 * (idx % V);
-    const uint32_t off = (i < n && j < n) ? (uint32_t)(((int64_t)i * K + j) * 4) : MG_OOB;
-    const float4 v = *reinterpret_cast<const float4*>(&S[(so + i) * LP + j]);
-    __builtin_amdgcn_raw_buffer_store_b128(
-        __builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned, v), rs, (int)off, 0, 0);
-  }
-}
-
-__global__ __launch_bounds__(256) void leaf_kernel(float* __restrict__ P, int64_t K, int64_t r0,
-                                                   int n, int* __restrict__ status, int64_t sP) {
-  __shared__ float S[NB * LP];
-  P += (int64_t)blockIdx.z * sP;
-  status += blockIdx.z;
-  float* blk = P + r0 * K + r0;
-  leaf_load(S, 0, blk, K, n);
-  __syncthreads();
-  const bool bad = leaf_rec<NB>(S, 0);
-  if (threadIdx.x == 0 && bad) atomicMin(status, (int)(r0 + 1));
-  leaf_store(S, 0, blk, K, n);
-}
-
-// A whole recursion node of m = 128 + m2 columns (0 < m2 <= 128) in one workgroup: both
-// diagonal blocks live in LDS (rows 0..127 and 128..255 of S), so the node's two leaves
-// and four 128 x 128 products run without a launch in between:
-//   S_A = leaf(A11) -> A11;  S_B = A21;  T1 = S_B S_A^T -> S_B;  T2 = T1 S_A -> S_A;
-//   S_B = A22 - T1 T1^T (lower);  S_B = leaf(S_B) -> A22;  A21 = -S_B T2.
-__global__ __launch_bounds__(256) void node_kernel(float* __restrict__ P, int64_t K, int64_t r0,
-                                                   int m2, int* __restrict__ status, int64_t sP) {
-  __shared__ float S[2 * NB * LP];
-  P += (int64_t)blockIdx.z * sP;
-  status += blockIdx.z;
-  float* a11 = P + r0 * K + r0;
-  float* a21 = P + (r0 + NB) * K + r0;
-  float* a22 = P + (r0 + NB) * K + (r0 + NB);
-  leaf_load(S, 0, a11, K, NB);
-  {  // A21 [m2 x 128] into S_B (rows past m2 zero)
-    const __amdgpu_buffer_rsrc_t rs = mg_rsrc(a21, (int64_t)(m2 - 1) * K + NB);
-    constexpr int V = NB / 4;
-    const int tid = threadIdx.x;
-    float4 x[NB * V / 256];
-#pragma unroll
-    for (int q = 0; q < NB * V / 256; ++q) {
-      const int idx = tid + 256 * q, i = idx / V, j = 4 * (idx % V);
-      const uint32_t off = i < m2 ? (uint32_t)(((int64_t)i * K + j) * 4) : MG_OOB;
-      x[q] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
-    }
-#pragma unroll
-    for (int q = 0; q < NB * V / 256; ++q) {
-      const int idx = tid + 256 * q, i = idx / V, j = 4 * (idx % V);
-      *reinterpret_cast<float4*>(&S[(NB + i) * LP + j]) = x[q];
-    }
-  }
-  __syncthreads();
-  bool bad1 = leaf_rec<NB>(S, 0);
-  leaf_store(S, 0, a11, K, NB);
-  leaf_prod<NB, true, false>(S, NB, 0, 0, 0, NB, 0, 1.0f);   // T1 = A21 A11^T
-  leaf_prod<NB, false, false>(S, NB, 0, 0, 0, 0, 0, 1.0f);   // T2 = T1 A11 (over S_A)
-  {  // S_B = A22 - T1 T1^T: lower triangle, zeros above, identity beyond m2
-    // (A22 is requested from memory first, so that its loads are in flight during the
-    // product)
-    const __amdgpu_buffer_rsrc_t rs = mg_rsrc(a22, (int64_t)(m2 - 1) * K + m2);
-    float g[ProdAcc<NB>::PER][4];
-#pragma unroll
-    for (int p = 0; p < ProdAcc<NB>::PER; ++p)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int r = prod_row<NB>(p, j), c = prod_col<NB>(p);
-        const uint32_t off = (r < m2 && c <= r) ? (uint32_t)(((int64_t)r * K + c) * 4) : MG_OOB;
-        g[p][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, (int)off, 0, 0));
-      }
-    ProdAcc<NB> Q;
-    leaf_mma<NB, true>(S, NB, 0, NB, 0, Q);
-    __syncthreads();  // T1 has been read
-#pragma unroll
-    for (int p = 0; p < ProdAcc<NB>::PER; ++p)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int r = prod_row<NB>(p, j), c = prod_col<NB>(p);
-        const float x = Q.acc[p][j];
-        const float v = (r < m2 && c < m2) ? (c <= r ? g[p][j] - x : 0.0f) : (r == c ? 1.0f : 0.0f);
-        S[(NB + r) * LP + c] = v;
-      }
-    __syncthreads();
-  }
-  bool bad2 = leaf_rec<NB>(S + NB * LP, 0);
-  if (threadIdx.x == 0 && (bad1 || bad2)) atomicMin(status, (int)(r0 + (bad1 ? 1 : NB + 1)));
-  leaf_store(S, NB, a22, K, m2);
-  {  // A21 = -S_B T2 (rows < m2)
-    ProdAcc<NB> Q;
-    leaf_mma<NB, false>(S, NB, 0, 0, 0, Q);
-    const __amdgpu_buffer_rsrc_t rs = mg_rsrc(a21, (int64_t)(m2 - 1) * K + NB);
-#pragma unroll
-    for (int p = 0; p < ProdAcc<NB>::PER; ++p)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int r = prod_row<NB>(p, j), c = prod_col<NB>(p);
-        const uint32_t off = r < m2 ? (uint32_t)(((int64_t)r * K + c) * 4) : MG_OOB;
-        const float x = Q.acc[p][j];
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(-x), rs, (int)off, 0, 0);
-      }
-  }
+  // the half of the block whose pivot failed, as 128-column blocks
+  if (bad && l == 0) atomicMin(status, (int)(r0 + w * ND_B / NB * NB + 1));
 }
 
 // U[i][j] = Linv[K-1-i][K-1-j] for j >= i, 0 below: in place over pairs
@@ -1844,7 +1694,7 @@ static bool pair_small(int64_t m1, int64_t m2) {
 }
 
 void plan_sizes(int64_t m, int depth, std::vector<int64_t>& t12) {
-  if (m <= 2 * NB) return;  // nodes and leaves work in LDS
+  if (m <= 2 * NB) return;  // one workgroup, no workspace
   const int64_t nbk = (m + NB - 1) / NB;
   const int64_t m1 = ((nbk + 1) / 2) * NB, m2 = m - m1;
   if ((int)t12.size() <= depth) t12.resize(depth + 1, 0);
@@ -1954,16 +1804,10 @@ int product_pair(const Ctx& c, GemmArgs upd, GemmArgs t2) {
 
 int inv_chol(const Ctx& c, int64_t r0, int64_t m, int depth) {
   const int64_t K = c.K;
-  if (m <= NB) {
+  if (m <= 2 * NB) {
     LaunchTimer timer(HI2X_TIME_CHOL_LEAF, 2.0 * m * m * m / 3.0 * c.batch, c.s);
-    hipLaunchKernelGGL(leaf_kernel, dim3(1, 1, (unsigned)c.batch), dim3(256), 0, c.s, c.P, K, r0,
-                       (int)m, c.status, c.sP);
-    return launch_status("leaf_kernel");
-  }
-  if (m <= 2 * NB) {  // the node's split is 128 + (m - 128): one fused kernel
-    LaunchTimer timer(HI2X_TIME_CHOL_LEAF, 2.0 * m * m * m / 3.0 * c.batch, c.s);
-    hipLaunchKernelGGL(node_kernel, dim3(1, 1, (unsigned)c.batch), dim3(256), 0, c.s, c.P, K, r0,
-                       (int)(m - NB), c.status, c.sP);
+    hipLaunchKernelGGL(node_kernel, dim3(1, 1, (unsigned)c.batch), dim3(64 * ND_N), 0, c.s, c.P, K,
+                       r0, (int)m, c.status, c.sP);
     return launch_status("node_kernel");
   }
   const int64_t nbk = (m + NB - 1) / NB;
