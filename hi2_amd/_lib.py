@@ -49,6 +49,7 @@ SIGNATURES = {
     "hi2x_hessian_syrk_grouped": [_P, _I64, _I, _P, _P, _I64, _I64, _I64, _P, _I64, _I, _P,
                                   _I64, _P],
     "hi2x_hessian_syrk_upper": [_P, _I, _I64, _I64, _P, _P, _I64, _P],
+    "hi2x_hessian_accumulate": [_P, _I, _I64, _I64, _P, _I, _P, _I64, _P],
     "hi2x_hessian_mirror": [_P, _I64, _P],
     "hi2x_hessian_blend": [_P, _I64, _I64, _I64, _P, _P, _I, _P],
     "hi2x_sigma_transform_upper_batched": [_P, _I64, _P, _I64, _P, _P, _I64, _P, _I64, _P],
@@ -85,6 +86,7 @@ SIGNATURES["hi2x_assemble_batch"] = [_P, _I64, _P, _P]
 # workspace sizes (int64 bytes, -1 for bad arguments): name -> argtypes
 SIZES = {
     "hi2x_hessian_workspace_bytes": [_I, _I64, _I64],
+    "hi2x_hessian_accumulate_workspace_bytes": [_I, _I64, _I64],
     "hi2x_hessian_grouped_workspace_bytes": [_I64, _I64, _I64],
     "hi2x_chol_workspace_bytes": [_I64],
     "hi2x_chol_batched_workspace_bytes": [_I64, _I64],

@@ -15,9 +15,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int HT = 128;  // output tile (features x features)
-constexpr int TCB = 32;  // tokens per LDS stage (bf16): two 32x32x16 steps
 constexpr int TCF = 8;   // tokens per LDS stage (f32): four 32x32x2 steps
-constexpr int XSB = TCB + 8;  // LDS row stride in bf16 elements (bank spread)
 
 __device__ __forceinline__ void upper_tile(int nT, int idx, int& ta, int& tb) {
   int a = 0;
@@ -31,10 +29,11 @@ __device__ __forceinline__ void upper_tile(int nT, int idx, int& ta, int& tb) {
 
 // Adds the accumulator tiles of one 128 x 128 output tile (rows a0.., cols b0..) into S,
 // mirrored so that S stays exactly symmetric: a diagonal tile writes (i, j) and (j, i)
-// from the i <= j element; an off-diagonal tile writes both (i, j) and (j, i).
+// from the i <= j element; an off-diagonal tile writes both (i, j) and (j, i).  first: S is
+// taken as zero.
 __device__ __forceinline__ void store_sym(float* __restrict__ s, int64_t K, int64_t a0,
                                           int64_t b0, bool diag, int wr, int wcn, int lane,
-                                          const f32x16 (&acc)[2][2]) {
+                                          bool first, const f32x16 (&acc)[2][2]) {
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -45,82 +44,22 @@ __device__ __forceinline__ void store_sym(float* __restrict__ s, int64_t K, int6
         const int64_t col = b0 + wcn * 64 + b * 32 + (lane & 31);
         if (row >= K || col >= K) continue;
         if (diag && row > col) continue;
-        const float v = s[row * K + col] + acc[a][b][j];
+        const float v = (first ? 0.0f : s[row * K + col]) + acc[a][b][j];
         s[row * K + col] = v;
         if (row != col) s[col * K + row] = v;
       }
 }
 
-// bf16 X [T, K]: one workgroup per upper 128 x 128 tile; the two feature slabs of a
-// 32-token stage are staged feature-major in LDS so every lane reads its 8 tokens as
-// one 16-byte vector; v_mfma_f32_32x32x16_bf16 accumulates in f32 (products exact).
-__global__ __launch_bounds__(256) void syrk_bf16_kernel(const uint16_t* __restrict__ x,
-                                                        int64_t T, int64_t K, int nT,
-                                                        float* __restrict__ s) {
-  __shared__ __attribute__((aligned(16))) uint16_t Xa[HT * XSB];
-  __shared__ __attribute__((aligned(16))) uint16_t Xb[HT * XSB];
-  int ta, tb;
-  upper_tile(nT, blockIdx.x, ta, tb);
-  const bool diag = ta == tb;
-  const int64_t a0 = (int64_t)ta * HT, b0 = (int64_t)tb * HT;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wr = wave >> 1, wcn = wave & 1;
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) acc[a][b][j] = 0.0f;
-
-  const int f = tid & (HT - 1), tg = tid >> 7;  // feature, 16-token half
-  for (int64_t t0 = 0; t0 < T; t0 += TCB) {
-    __syncthreads();
-    {
-      u16x8 va0, va1, vb0, vb1;
-      const int64_t fa = a0 + f, fb = b0 + f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int64_t t1 = t0 + tg * 16 + e, t2 = t1 + 8;
-        va0[e] = (t1 < T && fa < K) ? x[t1 * K + fa] : (uint16_t)0;
-        va1[e] = (t2 < T && fa < K) ? x[t2 * K + fa] : (uint16_t)0;
-        if (!diag) {
-          vb0[e] = (t1 < T && fb < K) ? x[t1 * K + fb] : (uint16_t)0;
-          vb1[e] = (t2 < T && fb < K) ? x[t2 * K + fb] : (uint16_t)0;
-        }
-      }
-      *reinterpret_cast<u16x8*>(&Xa[f * XSB + tg * 16]) = va0;
-      *reinterpret_cast<u16x8*>(&Xa[f * XSB + tg * 16 + 8]) = va1;
-      if (!diag) {
-        *reinterpret_cast<u16x8*>(&Xb[f * XSB + tg * 16]) = vb0;
-        *reinterpret_cast<u16x8*>(&Xb[f * XSB + tg * 16 + 8]) = vb1;
-      }
-    }
-    __syncthreads();
-    const uint16_t* XB = diag ? Xa : Xb;
-#pragma unroll
-    for (int ks = 0; ks < TCB; ks += 16) {
-      const int ko = ks + 8 * (lane >> 5);
-      bf16x8 av[2], bv[2];
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-        av[a] = __builtin_bit_cast(
-            bf16x8, *reinterpret_cast<const u16x8*>(&Xa[(wr * 64 + a * 32 + (lane & 31)) * XSB + ko]));
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-        bv[b] = __builtin_bit_cast(
-            bf16x8, *reinterpret_cast<const u16x8*>(&XB[(wcn * 64 + b * 32 + (lane & 31)) * XSB + ko]));
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-          acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[a], bv[b], acc[a][b], 0, 0, 0);
-    }
-  }
-  store_sym(s, K, a0, b0, diag, wr, wcn, lane, acc);
-}
-
-// ---- bf16 SYRK on the feature-major copy Xt [K, T] -----------------------------------
+// ---- 16-bit SYRK on the feature-major copy Xt [K, T] -----------------------------------
+// Three inputs run it: bf16 tokens on the bf16 MFMA, fp16 tokens on the fp16 MFMA (products of
+// either are exact in fp32; K=2560, 3 x 1777 fp16 tokens 197 us with the transform, 1715 us
+// converted to fp32 and multiplied on the fp32 MFMA), and
+// fp32 tokens as three bf16 planes x1 = bf16(x), x2 = bf16(x - x1), x3 = bf16(x - x1 - x2)
+// (the differences are exact in fp32, so the planes hold x to 2^-24 of itself whatever the
+// other tokens are), six of the nine plane products on the bf16 MFMA, small ones first: 96
+// cycles of the matrix core per 16 tokens of a 32 x 32 tile where the fp32 MFMA takes 512.
+// K=4096, 2 x 2048 fp32 tokens: 558 us with the transform, 2750 us on the fp32 MFMA (263
+// against 1250 us a batch); error against float64 2.6e-7 and 7.3e-7.
 // X [T, K] is first transposed once (one HBM pass) so that every MFMA operand (8
 // consecutive tokens of one feature) is a 16-byte vector in memory and in LDS.  A
 // workgroup (4 waves) computes a 256 x 256 upper tile of S; each wave owns 128 x 128 as
@@ -253,6 +192,75 @@ __global__ __launch_bounds__(256) void transpose8_bf16_kernel(const uint16_t* __
   }
 }
 
+// The three bf16 planes of f32 X [T, K], transposed: row k of xt [K, 3 Tp] is plane 1, 2, 3 of
+// feature k, zeros from T on.  One pass: 4 bytes read and 6 written per element.  A value whose
+// first plane would round to infinity (or is not finite) sets *bad, and the caller's products
+// run on the fp32 MFMA instead.  VEC: K a multiple of 4 and x 16-byte aligned.
+template <bool VEC>
+__global__ __launch_bounds__(256) void transpose_planes_kernel(const float* __restrict__ x,
+                                                               int64_t T, int64_t K, int64_t Tp,
+                                                               uint16_t* __restrict__ xt,
+                                                               uint32_t* __restrict__ bad) {
+  __shared__ float tile[64][65];
+  const int64_t t0 = (int64_t)blockIdx.y * 64, k0 = (int64_t)blockIdx.x * 64;
+  const int tid = threadIdx.x;
+  bool wide = false;
+  // the largest fp32 magnitude that rounds to a finite bf16 is below 0x7f7f8000
+  auto put = [&](int r, int c, float v) {
+    tile[r][c] = v;
+    wide = wide || (__float_as_uint(v) & 0x7fffffffu) >= 0x7f7f8000u;
+  };
+  if constexpr (VEC) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int r = (tid >> 4) + 16 * p, c = 4 * (tid & 15);
+      const int64_t t = t0 + r, k = k0 + c;
+      float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (t < T && k < K) v = *reinterpret_cast<const float4*>(x + t * K + k);
+      put(r, c, v.x);
+      put(r, c + 1, v.y);
+      put(r, c + 2, v.z);
+      put(r, c + 3, v.w);
+    }
+  } else {
+    for (int r = tid >> 6; r < 64; r += 4) {
+      const int64_t t = t0 + r, k = k0 + (tid & 63);
+      put(r, tid & 63, (t < T && k < K) ? x[t * K + k] : 0.0f);
+    }
+  }
+  if (__syncthreads_or(wide) && tid == 0) atomicOr(bad, 1u);
+  const int c = tid & 7;  // 8 tokens of feature kk: one 16-byte vector per plane
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const int kk = (tid >> 3) + 32 * p;
+    const int64_t k = k0 + kk;
+    if (k >= K) continue;
+    uint32_t w[3][4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float lo = tile[8 * c + 2 * e][kk], hi = tile[8 * c + 2 * e + 1][kk];
+#pragma unroll
+      for (int pl = 0; pl < 3; ++pl) {
+        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+        typedef float f32x2 __attribute__((ext_vector_type(2)));
+        const uint32_t u =
+            __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){lo, hi}, bf16x2));
+        w[pl][e] = u;
+        lo = lo - __uint_as_float(u << 16);
+        hi = hi - __uint_as_float(u & 0xffff0000u);
+      }
+    }
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl)
+      *reinterpret_cast<uint4*>(xt + k * 3 * Tp + pl * Tp + t0 + 8 * c) =
+          make_uint4(w[pl][0], w[pl][1], w[pl][2], w[pl][3]);
+  }
+}
+
+__global__ void clear_word_kernel(uint32_t* w) {
+  if (threadIdx.x == 0) *w = 0;
+}
+
 // ---- routed (grouped) accumulation: one launch for every group of a token batch --------
 // Group e is the tokens j in [offs[e], offs[e+1]) of a routed batch (the rows an MoE
 // router sent to expert e, hi2/moe.py:83-100); token j is row rows[j] of x (rows NULL:
@@ -343,22 +351,41 @@ __global__ __launch_bounds__(256) void grouped_transpose_kernel(
 
 // Operands of one k-step (16 tokens) of the current stage: XA / XB point at this lane's
 // operand row (tile t adds 32 rows), so its 16-byte slot.
-__device__ __forceinline__ void syrk_read(bf16x8 (&av)[4], bf16x8 (&bv)[4], const uint16_t* XA,
+__device__ __forceinline__ void syrk_read(u16x8 (&av)[4], u16x8 (&bv)[4], const uint16_t* XA,
                                           const uint16_t* XB, int so) {
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
-    av[t] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u16x8*>(&XA[32 * t * S2C + so]));
-    bv[t] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u16x8*>(&XB[32 * t * S2C + so]));
+    av[t] = *reinterpret_cast<const u16x8*>(&XA[32 * t * S2C + so]);
+    bv[t] = *reinterpret_cast<const u16x8*>(&XB[32 * t * S2C + so]);
   }
 }
-__device__ __forceinline__ void syrk_mma(f32x16 (&acc)[4][4], const bf16x8 (&av)[4],
-                                         const bf16x8 (&bv)[4]) {
+
+// What the 16-bit values are: bf16, fp16, or the three bf16 planes of fp32.
+enum SyrkKind { SYRK_BF16 = 0, SYRK_F16 = 1, SYRK_PLANES = 2 };
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+template <int KIND>
+__device__ __forceinline__ f32x16 syrk_mfma(const u16x8& a, const u16x8& b, const f32x16& c) {
+  if constexpr (KIND == SYRK_F16)
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
+                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+template <int KIND>
+__device__ __forceinline__ void syrk_mma(f32x16 (&acc)[4][4], const u16x8 (&av)[4],
+                                         const u16x8 (&bv)[4]) {
 #pragma unroll
   for (int a = 0; a < 4; ++a)
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
-      acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[a], bv[b], acc[a][b], 0, 0, 0);
+    for (int b = 0; b < 4; ++b) acc[a][b] = syrk_mfma<KIND>(av[a], bv[b], acc[a][b]);
 }
+
+// The plane products of fp32 tokens in the order they are summed: A's plane in bits 2i, B's in
+// the same bits of the second word (planes 0, 1, 2 for x1, x2, x3).
+constexpr int SYRK_TERMS = 6;
+constexpr uint32_t SYRK_PA = 2u | 0u << 2 | 1u << 4 | 1u << 6 | 0u << 8 | 0u << 10;
+constexpr uint32_t SYRK_PB = 0u | 2u << 2 | 1u << 4 | 0u << 6 | 1u << 8 | 0u << 10;
 
 // 16 bytes per lane from a buffer straight into LDS: lane L writes lds + 16 L (lds is
 // wave-uniform).  Issued as inline assembly so that the compiler does not treat the
@@ -384,7 +411,10 @@ constexpr int waitcnt_imm(int vm, int lgkm) {
   return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | (lgkm << 8);
 }
 
-// T is xt's row stride (its padded token count); with grouped (gr.order not null) item
+// T is xt's row stride: its padded token count Tp, or 3 Tp for planes (a feature's row is its
+// plane 1, then 2, then 3), whose token range is the SYRK_TERMS plane products one after the
+// other, SYRK_TERMS Tp virtual tokens.  skip (when not null): a nonzero word there ends the
+// launch at once (fp32 tokens that the planes cannot hold).  first: S is taken as zero.  With grouped (gr.order not null) item
 // blockIdx.x is tile (id % ntiles) of the group of rank id / ntiles, over its window.
 //
 // mode 0: every upper tile (row-major id = blockIdx / splits, dealt to the XCDs in
@@ -392,12 +422,17 @@ constexpr int waitcnt_imm(int vm, int lgkm) {
 // split (or S itself with one split); mode 1 (super): XCD blockIdx % 8 runs tile
 // blockIdx / 8 of its list in sched, into S; mode 2 (tail): tail tile blockIdx / splits
 // of sched, split over the tokens, each (tile, split) partial a 256 x 256 block of out.
-__global__ __launch_bounds__(256) void syrk2_bf16_kernel(const uint16_t* __restrict__ xt,
-                                                         int64_t T, int64_t K, int nT,
-                                                         int64_t ntiles, int splits,
-                                                         int64_t tchunk, float* __restrict__ out,
-                                                         int64_t out_stride, int mode,
-                                                         SyrkGroups gr, const SyrkSched sched) {
+template <int KIND>
+__global__ __launch_bounds__(256) void syrk2_kernel(const uint16_t* __restrict__ xt,
+                                                    int64_t T, int64_t K, int nT,
+                                                    int64_t ntiles, int splits,
+                                                    int64_t tchunk, float* __restrict__ out,
+                                                    int64_t out_stride, int mode, int first,
+                                                    const uint32_t* __restrict__ skip,
+                                                    SyrkGroups gr, const SyrkSched sched) {
+  if (KIND == SYRK_PLANES && *skip != 0) return;
+  const int64_t Tp = KIND == SYRK_PLANES ? T / 3 : T;
+  const int64_t Tv = KIND == SYRK_PLANES ? SYRK_TERMS * Tp : T;  // virtual tokens
   __shared__ __attribute__((aligned(1024))) uint16_t Xa[S2NB][S2T * S2C];
   __shared__ __attribute__((aligned(1024))) uint16_t Xb[S2NB][S2T * S2C];
   const int64_t id = (int64_t)blockIdx.x;
@@ -432,7 +467,7 @@ __global__ __launch_bounds__(256) void syrk2_bf16_kernel(const uint16_t* __restr
       upper_tile(nT, (int)tile, ta, tb);
     }
     tbeg = (int64_t)sp * tchunk;
-    tend = (tbeg + tchunk < T) ? tbeg + tchunk : T;
+    tend = (tbeg + tchunk < Tv) ? tbeg + tchunk : Tv;
     if (mode == 2) {
       so = out + (tile * splits + sp) * (int64_t)S2T * S2T;
       ldo = S2T;
@@ -473,25 +508,42 @@ __global__ __launch_bounds__(256) void syrk2_bf16_kernel(const uint16_t* __restr
   // byte offset of the stage in its first row
   // (live = false: a load that reads nothing and writes zeros, for stages past the end,
   // so that every stage issues the same number of loads)
-  auto dma_one = [&](int j, uint32_t b, int buf, bool live) {
+  struct Off {
+    uint32_t a, b;
+  };
+  auto dma_one = [&](int j, Off f, int buf, bool live) {
     const int i = j >> 1, c = NC * wv + i, row = 16 * c + prow;
-    const uint32_t o = b + (uint32_t)((int64_t)16 * i * T * 2);
+    const uint32_t o = (uint32_t)((int64_t)16 * i * T * 2);
     if ((j & 1) == 0) {
-      lds_dma16(rsa, (live && row < rowsA) ? o : MG_OOB, &Xa[buf][c * 512]);
+      lds_dma16(rsa, (live && row < rowsA) ? f.a + o : MG_OOB, &Xa[buf][c * 512]);
     } else {  // diagonal tiles load the A panel twice (uniform count of loads per stage)
-      lds_dma16(diag ? rsa : rsb, (live && row < (diag ? rowsA : rowsB)) ? o : MG_OOB,
+      lds_dma16(diag ? rsa : rsb, (live && row < (diag ? rowsA : rowsB)) ? f.b + o : MG_OOB,
                 &Xb[buf][c * 512]);
     }
   };
+  // planes: the term and first token of the next stage to be requested (stages are requested
+  // in order, and Tp is a multiple of the stage)
+  int term = KIND == SYRK_PLANES ? (int)(tbeg / Tp) : 0;
+  int64_t tt = KIND == SYRK_PLANES ? tbeg - term * Tp : 0;
   auto stage_off = [&](int64_t t0) {
-    uint32_t b = (uint32_t)(((int64_t)(16 * NC * wv + prow)) * T * 2 + t0 * 2 + 16 * piece);
-    asm volatile("" : "+v"(b));
-    return b;
+    uint32_t b = (uint32_t)(((int64_t)(16 * NC * wv + prow)) * T * 2 + 16 * piece);
+    if constexpr (KIND == SYRK_PLANES) {
+      asm volatile("" : "+v"(b));
+      const uint32_t ba = (uint32_t)((((SYRK_PA >> (2 * term)) & 3) * Tp + tt) * 2);
+      const uint32_t bb = (uint32_t)((((SYRK_PB >> (2 * term)) & 3) * Tp + tt) * 2);
+      tt += S2C;
+      if (tt == Tp) tt = 0, ++term;
+      return Off{b + ba, b + bb};
+    } else {
+      b += (uint32_t)(t0 * 2);
+      asm volatile("" : "+v"(b));
+      return Off{b, b};
+    }
   };
   auto dma = [&](int64_t t0, int buf, bool live) {
-    const uint32_t b = stage_off(t0);
+    const Off f = stage_off(t0);
 #pragma unroll
-    for (int j = 0; j < 2 * NC; ++j) dma_one(j, b, buf, live);
+    for (int j = 0; j < 2 * NC; ++j) dma_one(j, f, buf, live);
   };
   constexpr int PER_STAGE = 2 * NC;  // load instructions per wave and stage
   static_assert(S2C == 32 && S2NB == 4, "the loop below reads two k-steps per stage");
@@ -512,7 +564,7 @@ __global__ __launch_bounds__(256) void syrk2_bf16_kernel(const uint16_t* __restr
     __builtin_amdgcn_s_barrier();
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
   };
-  bf16x8 oa0[4], ob0[4], oa1[4], ob1[4];
+  u16x8 oa0[4], ob0[4], oa1[4], ob1[4];
   if (nst > 0) {
 #pragma unroll
     for (int p = 0; p < S2NB; ++p) dma(tbeg + (int64_t)p * S2C, p, p < nst);
@@ -524,7 +576,7 @@ __global__ __launch_bounds__(256) void syrk2_bf16_kernel(const uint16_t* __restr
     const int cb = st % S2NB, nb = (st + 1) % S2NB;
     syrk_read(oa1, ob1, &Xa[cb][rowA * S2C], &Xb[cb][rowB * S2C], so1);
     __builtin_amdgcn_sched_barrier(0);
-    syrk_mma(acc, oa0, ob0);
+    syrk_mma<KIND>(acc, oa0, ob0);
     __builtin_amdgcn_sched_barrier(0);
     // this wave's reads of stage st are done and stage st + 1 has landed; after the
     // barrier no wave reads buffer cb any more (past the end: reads of unused zeros)
@@ -534,15 +586,15 @@ __global__ __launch_bounds__(256) void syrk2_bf16_kernel(const uint16_t* __restr
     __builtin_amdgcn_sched_barrier(0);
     // stage st + 4 into buffer cb, one load after every second MFMA (a single wave per
     // SIMD issues in order: a block of loads would leave the MFMA pipe idle)
-    const uint32_t b = stage_off(tbeg + (int64_t)(st + S2NB) * S2C);
+    const Off f = stage_off(tbeg + (int64_t)(st + S2NB) * S2C);
     const bool live = st + S2NB < nst;
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        acc[a][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(oa1[a], ob1[q], acc[a][q], 0, 0, 0);
+        acc[a][q] = syrk_mfma<KIND>(oa1[a], ob1[q], acc[a][q]);
         if (q & 1) {
-          dma_one(2 * a + (q >> 1), b, cb, live);
+          dma_one(2 * a + (q >> 1), f, cb, live);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -570,7 +622,7 @@ __global__ __launch_bounds__(256) void syrk2_bf16_kernel(const uint16_t* __restr
                      : MG_OOB;
         cur[j] = 0.0f;
       }
-      if (splits == 1) {
+      if (splits == 1 && !first) {
 #pragma unroll
         for (int j = 0; j < 16; ++j)
           cur[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rss, (int)offs[j], 0, 0));
@@ -590,15 +642,19 @@ __global__ __launch_bounds__(256) void syrk2_bf16_kernel(const uint16_t* __restr
 template <bool VEC>
 __global__ __launch_bounds__(256) void split_sum_kernel(float* __restrict__ s,
                                                         const float* __restrict__ parts,
-                                                        int splits, int64_t K) {
+                                                        int splits, int64_t K, int first,
+                                                        const uint32_t* __restrict__ skip) {
+  if (skip != nullptr && *skip != 0) return;
   const int64_t i = blockIdx.x;
   constexpr int W = VEC ? 4 : 1;
   const int64_t j = ((int64_t)blockIdx.y * 256 + threadIdx.x) * W;
   if (j >= K || j + W - 1 < i) return;
   const int64_t idx = i * K + j;
   if constexpr (VEC) {
-    f32x4 v = *reinterpret_cast<const f32x4*>(s + idx);
+    f32x4 v = (f32x4)(0.0f);
+    if (!first || j < i) v = *reinterpret_cast<const f32x4*>(s + idx);
     const f32x4 v0 = v;
+    if (first) v = (f32x4)(0.0f);
     for (int p = 0; p < splits; ++p) {
       const f32x4 q = *reinterpret_cast<const f32x4*>(parts + (int64_t)p * K * K + idx);
 #pragma unroll
@@ -608,7 +664,7 @@ __global__ __launch_bounds__(256) void split_sum_kernel(float* __restrict__ s,
     for (int e = 0; e < 4; ++e) v[e] = j + e < i ? v0[e] : v[e];
     *reinterpret_cast<f32x4*>(s + idx) = v;
   } else {
-    float v = s[idx];
+    float v = first ? 0.0f : s[idx];
     for (int p = 0; p < splits; ++p) v = v + parts[(int64_t)p * K * K + idx];
     s[idx] = v;
   }
@@ -619,7 +675,10 @@ __global__ __launch_bounds__(256) void split_sum_kernel(float* __restrict__ s,
 // each tile.  Four workgroups per tile, 64 rows each; thread c walks column c of its rows.
 __global__ __launch_bounds__(256) void syrk_tail_sum_kernel(float* __restrict__ s, int64_t K,
                                                             const SyrkSched sched, int splits,
-                                                            const float* __restrict__ parts) {
+                                                            const float* __restrict__ parts,
+                                                            int first,
+                                                            const uint32_t* __restrict__ skip) {
+  if (skip != nullptr && *skip != 0) return;
   const int64_t t = blockIdx.x / 4;
   const int r0 = (int)(blockIdx.x % 4) * 64, c = threadIdx.x;
   const int ta = sched.tail[t] >> 8, tb = sched.tail[t] & 0xff;
@@ -628,7 +687,7 @@ __global__ __launch_bounds__(256) void syrk_tail_sum_kernel(float* __restrict__ 
   const float* pt = parts + t * splits * (int64_t)S2T * S2T;
   for (int r = r0; r < r0 + 64; ++r) {
     if (a0 + r >= K || (ta == tb && r > c)) break;  // rows only grow: the rest is out too
-    float v = s[(a0 + r) * K + b0 + c];
+    float v = first ? 0.0f : s[(a0 + r) * K + b0 + c];
     for (int p = 0; p < splits; ++p) v = v + pt[((int64_t)p * S2T + r) * S2T + c];
     s[(a0 + r) * K + b0 + c] = v;
   }
@@ -680,10 +739,14 @@ __global__ __launch_bounds__(256) void mirror_kernel(float* __restrict__ s, int6
   }
 }
 
-// f32 X [T, K]: same tiling on v_mfma_f32_32x32x2_f32.
+// f32 X [T, K] on v_mfma_f32_32x32x2_f32, 128 x 128 tiles: for callers without a workspace and
+// for tokens that the bf16 planes cannot hold (only: when not null, the launch does nothing
+// unless the word there is nonzero).  Writes both triangles; first: S is taken as zero.
 __global__ __launch_bounds__(256) void syrk_f32_kernel(const float* __restrict__ x, int64_t T,
-                                                       int64_t K, int nT,
-                                                       float* __restrict__ s) {
+                                                       int64_t K, int nT, float* __restrict__ s,
+                                                       int first,
+                                                       const uint32_t* __restrict__ only) {
+  if (only != nullptr && *only == 0) return;
   __shared__ float Xa[TCF][HT];
   __shared__ float Xb[TCF][HT];
   int ta, tb;
@@ -726,7 +789,7 @@ __global__ __launch_bounds__(256) void syrk_f32_kernel(const float* __restrict__
           acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[a], bv[b], acc[a][b], 0, 0, 0);
     }
   }
-  store_sym(s, K, a0, b0, diag, wr, wcn, lane, acc);
+  store_sym(s, K, a0, b0, diag, wr, wcn, lane, first != 0, acc);
 }
 
 // transform_sigma in three coalesced passes over HBM, evaluating what the reference's
@@ -961,15 +1024,17 @@ __global__ __launch_bounds__(256) void st_upper_kernel(const float* __restrict__
 // the tail tiles (the last tiles in row-major order past the last whole round of 256,
 // each split over the token range so that they fill one round of the CUs).
 struct SyrkPlan {
-  int64_t tp = 0, tchunk = 0, ntiles = 0;
+  int64_t tp = 0;  // padded tokens
+  int64_t tv = 0;  // tokens the products run over (SYRK_TERMS tp for planes)
+  int64_t tchunk = 0, ntiles = 0;
   int nT = 0, splits = 1;
   int super = 0;
   int64_t main_grid = 0;             // super: workgroups of the main launch
   int tail_splits = 1;
   int64_t tail_tchunk = 0;
   SyrkSched sched{};
-  size_t xt_bytes = 0, parts_bytes = 0;
-  size_t total() const { return xt_bytes + parts_bytes; }
+  size_t xt_bytes = 0, parts_bytes = 0, flag_bytes = 0;
+  size_t total() const { return xt_bytes + parts_bytes + flag_bytes; }
 };
 
 // Token chunk of s splits of tp tokens (a multiple of the stage), and the splits that
@@ -1024,7 +1089,7 @@ static bool syrk_schedule(SyrkPlan& p) {
   for (int x = 0; x < 8; ++x) tail += load[x] > main ? load[x] - main : 0;
   int ts = tail > 0 ? (int)(256 / tail) : 1;
   if (ts > 8) ts = 8;
-  if (tail == 0 || tail > SYRK_MAX_TAIL || ts < 2 || p.tp < 4 * S2C * ts) {
+  if (tail == 0 || tail > SYRK_MAX_TAIL || ts < 2 || p.tv < 4 * S2C * ts) {
     sc.main = (int32_t)maxl;  // no tail: every tile in the main launch
     sc.ntail = 0;
     p.main_grid = 8 * maxl;
@@ -1046,21 +1111,24 @@ static bool syrk_schedule(SyrkPlan& p) {
     }
   }
   p.main_grid = 8 * main;
-  syrk_chunk(p.tp, ts, p.tail_tchunk, p.tail_splits);
+  syrk_chunk(p.tv, ts, p.tail_tchunk, p.tail_splits);
   p.parts_bytes = (size_t)sc.ntail * p.tail_splits * S2T * S2T * sizeof(float);
   return true;
 }
 
-SyrkPlan syrk_plan(int dtype, int64_t t, int64_t k) {
+SyrkPlan syrk_plan(int kind, int64_t t, int64_t k) {
   SyrkPlan p;
-  if (dtype != 2 || t == 0) return p;
+  if (t == 0) return p;
   p.tp = (t + 63) / 64 * 64;
+  p.tv = kind == SYRK_PLANES ? SYRK_TERMS * p.tp : p.tp;
   p.nT = (int)((k + S2T - 1) / S2T);
   p.ntiles = (int64_t)p.nT * (p.nT + 1) / 2;
-  p.xt_bytes = ((size_t)p.tp * (size_t)k * 2 + 255) / 256 * 256;
+  const size_t row = (size_t)p.tp * (kind == SYRK_PLANES ? 3 : 1);
+  p.xt_bytes = (row * (size_t)k * 2 + 255) / 256 * 256;
+  p.flag_bytes = kind == SYRK_PLANES ? 256 : 0;
   if (p.ntiles >= 512) {
     // super-tile schedule, one workgroup per CU (else every tile at once, no tail)
-    p.tchunk = p.tp;
+    p.tchunk = p.tv;
     p.super = syrk_schedule(p) ? 1 : 0;
     return p;
   }
@@ -1078,7 +1146,7 @@ SyrkPlan syrk_plan(int dtype, int64_t t, int64_t k) {
       if (c < cost - 1e-9) cost = c, best = sp;
     }
   }
-  syrk_chunk(p.tp, best, p.tchunk, p.splits);
+  syrk_chunk(p.tv, best, p.tchunk, p.splits);
   p.parts_bytes = p.splits > 1 ? (size_t)p.splits * k * k * sizeof(float) : 0;
   return p;
 }
@@ -1089,48 +1157,64 @@ int launch_mirror(float* s, int64_t k, hipStream_t st) {
   return launch_status("mirror_kernel");
 }
 
-// ws: device workspace of at least syrk_plan(...).total() bytes, 256-byte aligned.
-// mirror = false leaves the lower triangle of a bf16 accumulation stale (the f32 path
-// always writes both triangles).
-int launch_syrk(const void* x, int dtype, int64_t t, int64_t k, float* s, char* ws,
-                hipStream_t st, bool mirror = true) {
-  if (dtype != 2) {
-    const int nT = (int)((k + HT - 1) / HT);
-    const int64_t tiles = (int64_t)nT * (nT + 1) / 2;
-    LaunchTimer timer(HI2X_TIME_HESSIAN_SYRK, (double)t * k * (k + 1), st);  // upper triangle
-    hipLaunchKernelGGL(syrk_f32_kernel, dim3((unsigned)tiles), dim3(256), 0, st,
-                       (const float*)x, t, k, nT, s);
-    return launch_status("syrk_f32_kernel");
-  }
-  // bf16: transpose, tiles of 256 (token range split when the tiles are few), mirror
-  const SyrkPlan p = syrk_plan(dtype, t, k);
+int launch_syrk_f32(const float* x, int64_t t, int64_t k, float* s, int first,
+                    const uint32_t* only, hipStream_t st) {
+  const int nT = (int)((k + HT - 1) / HT);
+  const int64_t tiles = (int64_t)nT * (nT + 1) / 2;
+  hipLaunchKernelGGL(syrk_f32_kernel, dim3((unsigned)tiles), dim3(256), 0, st, x, t, k, nT, s,
+                     first, only);
+  return launch_status("syrk_f32_kernel");
+}
+
+// ws: device workspace of at least syrk_plan(KIND, ...).total() bytes, 256-byte aligned.
+// Transpose (fp32: into planes), tiles of 256 (token range split when the tiles are few), sums;
+// the lower triangle of s is left stale.
+template <int KIND>
+int launch_syrk16(const void* x, int64_t t, int64_t k, float* s, int first, char* ws,
+                  hipStream_t st) {
+  const SyrkPlan p = syrk_plan(KIND, t, k);
   uint16_t* xt = reinterpret_cast<uint16_t*>(ws);
   float* parts = p.parts_bytes > 0 ? reinterpret_cast<float*>(ws + p.xt_bytes) : nullptr;
+  uint32_t* bad = nullptr;
   const dim3 tg((unsigned)((k + 63) / 64), (unsigned)(p.tp / 64));
-  if (k % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0)
+  const bool al = (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+  if constexpr (KIND == SYRK_PLANES) {
+    bad = reinterpret_cast<uint32_t*>(ws + p.xt_bytes + p.parts_bytes);
+    hipLaunchKernelGGL(clear_word_kernel, dim3(1), dim3(64), 0, st, bad);
+    const int rc = launch_status("clear_word_kernel");
+    if (rc) return rc;
+    if (k % 4 == 0 && al)
+      hipLaunchKernelGGL(transpose_planes_kernel<true>, tg, dim3(256), 0, st, (const float*)x, t,
+                         k, p.tp, xt, bad);
+    else
+      hipLaunchKernelGGL(transpose_planes_kernel<false>, tg, dim3(256), 0, st, (const float*)x, t,
+                         k, p.tp, xt, bad);
+  } else if (k % 8 == 0 && al) {
     hipLaunchKernelGGL(transpose8_bf16_kernel, tg, dim3(256), 0, st, (const uint16_t*)x, t, k,
                        p.tp, xt);
-  else
+  } else {
     hipLaunchKernelGGL(transpose_bf16_kernel, tg, dim3(256), 0, st, (const uint16_t*)x, t, k, p.tp,
                        xt);
+  }
   int rc = launch_status("transpose_bf16_kernel");
+  const int64_t ld = KIND == SYRK_PLANES ? 3 * p.tp : p.tp;
   if (!rc) {
     // one workgroup per CU: super-tile rounds once the tiles fill several rounds
     LaunchTimer timer(HI2X_TIME_HESSIAN_SYRK, (double)t * k * (k + 1), st);  // upper triangle
     const int64_t grid = p.super ? p.main_grid : (p.ntiles + 7) / 8 * 8 * p.splits;
-    hipLaunchKernelGGL(syrk2_bf16_kernel, dim3((unsigned)grid), dim3(256), 0, st, xt, p.tp, k,
-                       p.nT, p.ntiles, p.splits, p.tchunk, p.splits > 1 ? parts : s, k * k,
-                       p.super, SyrkGroups{}, p.sched);
-    rc = launch_status("syrk2_bf16_kernel");
+    hipLaunchKernelGGL(syrk2_kernel<KIND>, dim3((unsigned)grid), dim3(256), 0, st, xt, ld, k, p.nT,
+                       p.ntiles, p.splits, p.tchunk, p.splits > 1 ? parts : s, k * k, p.super,
+                       first, bad, SyrkGroups{}, p.sched);
+    rc = launch_status("syrk2_kernel");
     const int ntail = p.super ? p.sched.ntail : 0;
     if (!rc && ntail > 0) {  // the tail tiles, token-split, then summed in split order
-      hipLaunchKernelGGL(syrk2_bf16_kernel, dim3((unsigned)(ntail * p.tail_splits)), dim3(256), 0,
-                         st, xt, p.tp, k, p.nT, (int64_t)ntail, p.tail_splits, p.tail_tchunk,
-                         parts, (int64_t)0, 2, SyrkGroups{}, p.sched);
-      rc = launch_status("syrk2_bf16_kernel");
+      hipLaunchKernelGGL(syrk2_kernel<KIND>, dim3((unsigned)(ntail * p.tail_splits)), dim3(256), 0,
+                         st, xt, ld, k, p.nT, (int64_t)ntail, p.tail_splits, p.tail_tchunk, parts,
+                         (int64_t)0, 2, 1, bad, SyrkGroups{}, p.sched);
+      rc = launch_status("syrk2_kernel");
       if (!rc) {
         hipLaunchKernelGGL(syrk_tail_sum_kernel, dim3((unsigned)(4 * ntail)), dim3(256), 0, st, s,
-                           k, p.sched, p.tail_splits, parts);
+                           k, p.sched, p.tail_splits, parts, first, bad);
         rc = launch_status("syrk_tail_sum_kernel");
       }
     }
@@ -1141,14 +1225,32 @@ int launch_syrk(const void* x, int dtype, int64_t t, int64_t k, float* s, char* 
     const int64_t w = vec ? 4 : 1;
     const dim3 grid((unsigned)k, (unsigned)((k + 256 * w - 1) / (256 * w)));
     if (vec)
-      hipLaunchKernelGGL(split_sum_kernel<true>, grid, dim3(256), 0, st, s, parts, p.splits, k);
+      hipLaunchKernelGGL(split_sum_kernel<true>, grid, dim3(256), 0, st, s, parts, p.splits, k,
+                         first, bad);
     else
-      hipLaunchKernelGGL(split_sum_kernel<false>, grid, dim3(256), 0, st, s, parts, p.splits, k);
+      hipLaunchKernelGGL(split_sum_kernel<false>, grid, dim3(256), 0, st, s, parts, p.splits, k,
+                         first, bad);
     rc = launch_status("split_sum_kernel");
   }
-  if (!rc && mirror) rc = launch_mirror(s, k, st);
+  if (!rc && KIND == SYRK_PLANES) rc = launch_syrk_f32((const float*)x, t, k, s, first, bad, st);
   return rc;
 }
+
+// The accumulations without a choice of workspace: bf16 through the transposed copy, f32 on
+// the fp32 MFMA (no workspace; both triangles).
+int launch_syrk(const void* x, int dtype, int64_t t, int64_t k, float* s, char* ws,
+                hipStream_t st, bool mirror = true) {
+  if (dtype != 2) {
+    LaunchTimer timer(HI2X_TIME_HESSIAN_SYRK, (double)t * k * (k + 1), st);  // upper triangle
+    return launch_syrk_f32((const float*)x, t, k, s, 0, nullptr, st);
+  }
+  const int rc = launch_syrk16<SYRK_BF16>(x, t, k, s, 0, ws, st);
+  return !rc && mirror ? launch_mirror(s, k, st) : rc;
+}
+
+// fp32 tokens run as planes unless a 256-feature panel of them would pass 32-bit offsets (1.4 M
+// tokens in one call).
+bool f32_planes(int64_t t, int64_t k) { return (t + 63) / 64 * 64 * 3 <= (int64_t(1) << 22); }
 
 // Workspace of the grouped accumulation: xt [k, cap] bf16 (cap = tokens + 64 per group,
 // the windows' worst case) and the plan tables.
@@ -1175,7 +1277,7 @@ using namespace hi2x;
 
 extern "C" int64_t hi2x_hessian_workspace_bytes(int dtype, int64_t t, int64_t k) {
   if ((dtype != 0 && dtype != 2) || k <= 0 || t < 0) return -1;
-  return (int64_t)syrk_plan(dtype, t, k).total();
+  return dtype == 2 ? (int64_t)syrk_plan(SYRK_BF16, t, k).total() : 0;
 }
 
 extern "C" int hi2x_hessian_syrk(const void* x, int dtype, int64_t t, int64_t k, float* s,
@@ -1186,7 +1288,8 @@ extern "C" int hi2x_hessian_syrk(const void* x, int dtype, int64_t t, int64_t k,
   if (t == 0) return HI2X_OK;
   hipStream_t st = as_stream(stream);
   Workspace w;
-  const int rc = take_workspace(w, ws, ws_bytes, syrk_plan(dtype, t, k).total(), st,
+  const int rc = take_workspace(w, ws, ws_bytes,
+                                dtype == 2 ? syrk_plan(SYRK_BF16, t, k).total() : 0, st,
                                 "hessian_syrk");
   if (rc) return rc;
   return launch_syrk(x, dtype, t, k, s, w.p, st);
@@ -1201,10 +1304,38 @@ extern "C" int hi2x_hessian_syrk_upper(const void* x, int dtype, int64_t t, int6
   if (t == 0) return HI2X_OK;
   hipStream_t st = as_stream(stream);
   Workspace w;
-  const int rc = take_workspace(w, ws, ws_bytes, syrk_plan(dtype, t, k).total(), st,
+  const int rc = take_workspace(w, ws, ws_bytes,
+                                dtype == 2 ? syrk_plan(SYRK_BF16, t, k).total() : 0, st,
                                 "hessian_syrk_upper");
   if (rc) return rc;
   return launch_syrk(x, dtype, t, k, s, w.p, st, false);
+}
+
+extern "C" int64_t hi2x_hessian_accumulate_workspace_bytes(int dtype, int64_t t, int64_t k) {
+  if (dtype < 0 || dtype > 2 || k <= 0 || t < 0) return -1;
+  if (dtype == 0) return f32_planes(t, k) ? (int64_t)syrk_plan(SYRK_PLANES, t, k).total() : 0;
+  return (int64_t)syrk_plan(SYRK_BF16, t, k).total();
+}
+
+extern "C" int hi2x_hessian_accumulate(const void* x, int dtype, int64_t t, int64_t k, float* s,
+                                       int first, void* ws, int64_t ws_bytes, void* stream) {
+  clear_error();
+  HI2X_REQUIRE(dtype >= 0 && dtype <= 2, "hessian_accumulate: dtype %d (0 = f32, 1 = f16, 2 = bf16)",
+               dtype);
+  HI2X_REQUIRE(k > 0 && t > 0 && x && s, "hessian_accumulate: bad arguments");
+  HI2X_REQUIRE(dtype != 1 || t <= (int64_t(1) << 22), "hessian_accumulate: %lld f16 tokens exceed 4M",
+               (long long)t);
+  hipStream_t st = as_stream(stream);
+  Workspace w;
+  const int rc = take_workspace(w, ws, ws_bytes,
+                                (size_t)hi2x_hessian_accumulate_workspace_bytes(dtype, t, k), st,
+                                "hessian_accumulate");
+  if (rc) return rc;
+  if (dtype == 2) return launch_syrk16<SYRK_BF16>(x, t, k, s, first, w.p, st);
+  if (dtype == 1) return launch_syrk16<SYRK_F16>(x, t, k, s, first, w.p, st);
+  if (f32_planes(t, k)) return launch_syrk16<SYRK_PLANES>(x, t, k, s, first, w.p, st);
+  LaunchTimer timer(HI2X_TIME_HESSIAN_SYRK, (double)t * k * (k + 1), st);
+  return launch_syrk_f32((const float*)x, t, k, s, first, nullptr, st);
 }
 
 extern "C" int hi2x_hessian_mirror(float* s, int64_t k, void* stream) {
@@ -1258,10 +1389,10 @@ extern "C" int hi2x_hessian_syrk_grouped(const void* x, int64_t x_rows, int dtyp
   const int64_t ntiles = (int64_t)nT * (nT + 1) / 2;
   {
     LaunchTimer timer(HI2X_TIME_HESSIAN_SYRK, (double)t_total * k * (k + 1), st);
-    hipLaunchKernelGGL(syrk2_bf16_kernel, dim3((unsigned)(ntiles * G)), dim3(256), 0, st, xt,
-                       p.cap, k, nT, ntiles, 1, (int64_t)0, s, (int64_t)0, 0,
-                       SyrkGroups{order, toff, tp, s_stride, ntiles}, SyrkSched{});
-    rc = launch_status("syrk2_bf16_kernel");
+    hipLaunchKernelGGL(syrk2_kernel<SYRK_BF16>, dim3((unsigned)(ntiles * G)), dim3(256), 0, st, xt,
+                       p.cap, k, nT, ntiles, 1, (int64_t)0, s, (int64_t)0, 0, 0,
+                       (const uint32_t*)nullptr, SyrkGroups{order, toff, tp, s_stride, ntiles}, SyrkSched{});
+    rc = launch_status("syrk2_kernel");
   }
   if (rc || upper_only) return rc;
   const unsigned nM = (unsigned)((k + MT - 1) / MT);

@@ -11,7 +11,7 @@ fit a linear's ladders while its input's factor is still being computed.
 
 Every arithmetic step runs in the hi2x HIP kernels (``libhi2x.so``):
 
-* ``HessianStats.update``: ``hi2x_hessian_syrk_upper`` (bf16 / f32 MFMA), with
+* ``HessianStats.update``: ``hi2x_hessian_accumulate`` (bf16 / fp16 MFMA), with
   ``hi2x_hessian_mirror`` when ``S`` is read (exactly symmetric);
 * ``transform_sigma``: ``hi2x_sigma_transform`` (bit-identical to the reference einsums);
   ``HessianStats.transformed`` fuses the mean and the transform over the upper triangle
@@ -79,10 +79,13 @@ __all__ = [
 ]
 
 
+_SYRK_DTYPE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
+
+
 class HessianStats:
     """Full second moment ``sum x x^T`` of a Linear's input (fp32, ``[K, K]``) on a HIP
-    device; ``update`` accumulates on MFMA (bf16 inputs exactly, fp32 inputs on f32
-    MFMA, other dtypes converted to fp32 first as the reference does).
+    device; ``update`` accumulates on MFMA (bf16 and fp16 inputs exactly, fp32 inputs as
+    three bf16 planes, other dtypes converted to fp32 first as the reference does).
 
     ``update`` brings only the upper triangle up to date; the lower one is mirrored when
     ``S`` is read (``S``, ``mean``, ``merge``), and ``transformed`` reads the upper
@@ -95,9 +98,20 @@ class HessianStats:
             raise RuntimeError(
                 f"hi2_amd.HessianStats accumulates on the MI355X; got device {dev}"
             )
-        self._S = torch.zeros(k, k, dtype=torch.float32, device=dev)
+        self._dev = dev
+        self._sum: torch.Tensor | None = None  # made by the first update (or read as zeros)
         self._upper_only = False
         self.n = 0
+
+    @property
+    def _S(self) -> torch.Tensor:
+        if self._sum is None:
+            self._sum = torch.zeros(self.k, self.k, dtype=torch.float32, device=self._dev)
+        return self._sum
+
+    @_S.setter
+    def _S(self, value: torch.Tensor) -> None:
+        self._sum = value
 
     @property
     def S(self) -> torch.Tensor:
@@ -116,18 +130,24 @@ class HessianStats:
         """``S += x^T x`` over all rows of ``x[..., K]`` (``chunk`` is accepted for
         interface compatibility; the kernel streams the rows itself)."""
         x = x.reshape(-1, self.k)
-        dev = self._S.device
-        if x.dtype not in (torch.bfloat16, torch.float32):
+        dev = self._dev if self._sum is None else self._sum.device
+        t = x.shape[0]
+        dtype = _SYRK_DTYPE.get(x.dtype, 0)
+        if dtype == 1 and t > 1 << 22:
+            dtype = 0
+        if not dtype and x.dtype != torch.float32:
             x = x.to(torch.float32)
         x = x.to(dev).contiguous()
-        t = x.shape[0]
         if t:
-            if self._S.dtype != torch.float32 or not self._S.is_contiguous():
+            first = self._sum is None  # nothing to add to: neither cleared nor read
+            if first:
+                self._sum = torch.empty(self.k, self.k, dtype=torch.float32, device=dev)
+            elif self._sum.dtype != torch.float32 or not self._sum.is_contiguous():
                 self._S = self.S.to(torch.float32).contiguous()
-            dtype = 2 if x.dtype == torch.bfloat16 else 0
-            ws = _lib.workspace(dev, "hi2x_hessian_workspace_bytes", dtype, t, self.k)
-            _lib.call("hi2x_hessian_syrk_upper", dev, _lib.ptr(x), dtype, t, self.k,
-                      _lib.ptr(self._S), _lib.ptr(ws), ws.numel())
+            s = self._sum
+            ws = _lib.workspace(dev, "hi2x_hessian_accumulate_workspace_bytes", dtype, t, self.k)
+            _lib.call("hi2x_hessian_accumulate", dev, _lib.ptr(x), dtype, t, self.k, _lib.ptr(s),
+                      int(first), _lib.ptr(ws), ws.numel())
             self._upper_only = True
         self.n += t
 

@@ -1,0 +1,102 @@
+"""``HessianStats`` on fp16 and fp32 tokens (``hi2x_hessian_accumulate``) against float64: the
+edges of the 256-feature tiles, 64-token padding and token splits, values the bf16 planes of
+fp32 cannot hold, and the first update's unread sum."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 16), (63, 40), (64, 250), (65, 256), (200, 257), (1000, 272), (129, 1544),
+          (4500, 512), (70, 8208)]
+
+
+def _x(t, k, dtype, dev, seed):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    x = torch.randn(t, k, generator=g, device=dev)
+    x[:, ::13] *= 20.0
+    x[::7, 1] *= 1e-3
+    return x.to(dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("t,k", SHAPES)
+def test_against_float64(t, k, dtype, dev):
+    from hi2_amd.hessian import HessianStats
+
+    print(f"hessian {dtype} t={t} k={k}", flush=True)
+    st = HessianStats(k, dev)
+    a, b = _x(t, k, dtype, dev, t + k), _x(t + 3, k, dtype, dev, t * k)
+    st.update(a)
+    st.update(b)
+    x = torch.cat([a, b]).double()
+    want, mag = x.T @ x, x.abs().T @ x.abs()
+    # every element: products exact (or to 3 x 2^-24 of themselves), then an fp32 sum of n
+    # terms in some order: at most (n + 4) 2^-24 of the sum of magnitudes
+    bound = (x.shape[0] + 4) * 2.0 ** -24
+    assert bool(((st.S.double() - want).abs() <= bound * mag + 1e-30).all())
+    assert torch.equal(st.S, st.S.T) and st.n == x.shape[0]
+
+
+def test_fp32_elements_keep_their_own_precision(dev):
+    """Rare tokens 1e5 times the others must not cost the others' products (a scaled fp16 split
+    would lose them: its error is relative to a feature's largest token)."""
+    from hi2_amd.hessian import HessianStats
+
+    t, k = 512, 64
+    x = _x(t, k, torch.float32, dev, 5)
+    x[3, 0] = 1e5
+    x[9, 1] = -1e5
+    st = HessianStats(k, dev)
+    st.update(x)
+    xd = x.double()
+    assert bool(((st.S.double() - xd.T @ xd).abs() <= (t + 4) * 2.0 ** -24
+                 * (xd.abs().T @ xd.abs())).all())
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.4e38])
+@pytest.mark.parametrize("first", [True, False])
+def test_fp32_values_beyond_the_planes(value, first, dev):
+    """Infinities, NaN and the largest fp32 values give what fp32 products and sums give."""
+    from hi2_amd.hessian import HessianStats
+
+    t, k = 96, 300
+    x = _x(t, k, torch.float32, dev, 11)
+    st = HessianStats(k, dev)
+    if not first:
+        st.update(x)
+    y = x.clone()
+    y[5, 7] = value
+    st.update(y)
+    s = st.S
+    want = (y.double().T @ y.double() + (0 if first else x.double().T @ x.double())).float()
+    fin = torch.isfinite(want)
+    assert torch.equal(torch.isnan(s), torch.isnan(want))
+    assert torch.equal(s[torch.isinf(want)], want[torch.isinf(want)])
+    assert torch.allclose(s[fin], want[fin], rtol=1e-4, atol=1e-4 * 400 * t)
+
+
+def test_fp16_specials(dev):
+    """fp16 infinities, NaN and subnormals multiply as their fp32 values do."""
+    from hi2_amd.hessian import HessianStats
+
+    t, k = 64, 64
+    x = torch.zeros(t, k, dtype=torch.float16, device=dev)
+    x[0, 0], x[0, 1], x[1, 2], x[2, 3] = float("inf"), 2.0, float("nan"), 6e-8
+    x[2, 4], x[3, 5] = 65504.0, 65504.0
+    st = HessianStats(k, dev)
+    st.update(x)
+    want = x.float().T @ x.float()
+    assert torch.equal(torch.isnan(st.S), torch.isnan(want))
+    m = ~torch.isnan(want)
+    assert torch.equal(st.S[m], want[m])
+
+
+def test_sum_without_an_update_is_zero(dev):
+    from hi2_amd.hessian import HessianStats
+
+    st = HessianStats(48, dev)
+    st.update(torch.empty(0, 48, device=dev))
+    assert st.n == 0 and not bool(st.S.any())
+    had = torch.ones(3, dtype=torch.uint8, device=dev)
+    assert not bool(HessianStats(48, dev).transformed(None, had).any())
