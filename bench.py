@@ -344,17 +344,6 @@ def _encode_block(xs, ws, masks, timer=None, lanes=None, keep=None, cfg=CFG3):
     return out
 
 
-def trailing_flops(cfg) -> float:
-    """Algorithmic flops of every cross-block update of a step: per linear,
-    sum over 128-column blocks of 2 N 128 (K - i2) on the real rows (no padding)."""
-    total = 0.0
-    for _, n, k, _ in cfg["linears"]:
-        for i1 in range(0, k, 128):
-            i2 = min(i1 + 128, k)
-            total += 2.0 * n * (i2 - i1) * (k - i2)
-    return total
-
-
 def stage_breakdown(xs, ws, masks, cfg=CFG3):
     """One step run serially on one stream with every stage timed: per input its Hessian,
     transform and factor (stream events), per linear its rotation, ladder fit, column
@@ -467,7 +456,7 @@ def block_leg(cfg, dev, steps, warmup):
     sp = _lib.timing_query(11)
     _lib.timing_enable([])
     per_input, per_linear, rates = stage_breakdown(xs, ws, masks, cfg)
-    flops = trailing_flops(cfg)
+    flops = tr[2]
     trail_ms = tr[1]  # one step's launches
     res = {
         "workload": f"{cfg['name']}: " + ", ".join(f"{n} {r}x{k}" for n, r, k, _ in cfg["linears"])
@@ -643,13 +632,7 @@ def moe_leg(dev, steps, warmup):
     encode_moe(*inp, timer=timer)
     stages = timer.summary()["moe"]
     counts = torch.bincount(inp[0].reshape(-1), minlength=E5).cpu().tolist()
-    # trailing flops on the real rows: per expert gate/up 2048 rows at K = 2048, down
-    # 2048 rows at K = 1024
-    flops = 0.0
-    for n, k in ((2 * I5, H5), (H5, I5)):
-        for i1 in range(0, k, 128):
-            i2 = min(i1 + 128, k)
-            flops += E5 * 2.0 * n * (i2 - i1) * (k - i2)
+    flops = tr[2]
     trail_ms = tr[1]  # one step's launches
     res = {
         "workload": "cfg5: OLMoE-shaped MoE layer, 64 experts (gate/up 1024x2048 sharing a "
@@ -799,7 +782,8 @@ KERNELS = {  # kind -> (kernel, bound, peak FLOP/s, work unit)
          "3*M*N*rank fp16 MFMA flops executed (three fp16 products per fp32-equivalent "
          "product of one triangular operand)"),
     3: ("node_kernel", "latency", PEAK_F32, "2*n^3/3"),
-    4: ("gptq_block_kernel", "latency", PEAK_F32, "rows*L*(L-1)"),
+    4: ("gptq_block_kernel/gptq_super_kernel", "latency", PEAK_F32,
+        "rows*L*(L-1), with the near updates' 2*rows*rank*L in the super-block kernel"),
     5: ("refine GEMMs (refine_gradient_kernel + gptq_trailing_kernel)", "mfma", PEAK_F32,
         "2*rows*rank*cols"),
     6: ("refine_block_kernel", "latency", PEAK_F32, "rows*L (column decisions)"),
@@ -851,12 +835,13 @@ def pmc_traffic(kernel):
 
 def trailing_roofline(steps, basis):
     """The trailing update's roofline over the last timing window: the algorithmic flops
-    of the block's cross-block updates on real rows (trailing_flops) divided by the summed
-    event-timed durations of its launches; ``traffic`` from the committed PMC summary."""
+    of its launches (the near updates of batches of up to 4096 rows run inside the column
+    loops' launches and are not among them) divided by their summed event-timed durations;
+    ``traffic`` from the committed PMC summary."""
     from hi2_amd import _lib
 
     n, ms, work = _lib.timing_query(DOMINANT)
-    flops = trailing_flops(CFG3) * steps
+    flops = work
     rate = flops / (ms / 1e3)
     traffic, split = pmc_traffic(KERNELS[DOMINANT][0])
     return {"bound": "mfma", "achieved": rate / 1e12, "peak": PEAK_F32 / 1e12,
@@ -864,9 +849,8 @@ def trailing_roofline(steps, basis):
             "traffic_split": split,
             "kernel": KERNELS[DOMINANT][0], "launches": n, "avg_ms": ms / n,
             "flops_per_launch": flops / n,
-            "work": "2*rows*rank*cols summed over the block's cross-block updates, real rows "
-                    "only (the launches also run the zero rows that align factor runs to "
-                    "128)", "timing": basis}
+            "work": "2*rows*rank*cols summed over the cross-block update launches",
+            "timing": basis}
 
 
 def _cpu_info():

@@ -29,9 +29,8 @@ namespace {
 //
 // Step i (fully unrolled): every lane runs the rounding chain on its own column m=i/16
 // (the two divisions are the bare reciprocal iteration on the lane's precomputed
-// reciprocals; the lanes whose operands leave the range where the iteration is exact are
-// collected in a wave mask, and the rare wave with any runs the block again with
-// div_rcp_code for the code and IEEE division for the error);
+// reciprocals; the range of the operands is recorded, and the rare wave where a lane's left the
+// one where the iteration is exact runs the block again with IEEE divisions);
 // only lane q = i%16 owns column i (its U value of row i is then U[i][i]), so its error e
 // is broadcast to the row with DPP row_newbcast, and the row applies
 // w[c] -= e * U[i][c] to the columns it holds.  Columns <= i of the other lanes are dead
@@ -69,10 +68,20 @@ template <bool COMP>
 struct RowRegs {
   float w[CPL], loc[CPL], stc[CPL], ys[CPL], yu[CPL], er[CPL], qc[CPL];
   float cm[COMP ? CPL : 1];  // value each owned column was rounded from
-  // lanes of the wave whose error quotient may fall outside the iteration's exact range
-  // (wave-uniform: scalar registers)
-  uint64_t inexact;
+  // what the fast loop's error numerators have to stay within (gptq_step): their sum of
+  // magnitudes, the least of them as signed integers and the least positive as unsigned ones
+  float nsum;
+  int32_t nneg;
+  uint32_t npos;
+  bool bounded;  // the block's own bounds hold in this lane (load_row_c)
 };
+
+// Whether a lane's numerators were all +0 or of magnitude in [2^-50, 2^50].
+template <bool COMP>
+__device__ __forceinline__ bool row_exact(const RowRegs<COMP>& R) {
+  constexpr int32_t lo = 0x26800000;  // 2^-50
+  return R.bounded && R.nsum <= 0x1p50f && R.nneg >= INT32_MIN + lo && R.npos >= (uint32_t)lo - 1;
+}
 
 // The live part of this lane's U row at p: columns mm >= M (earlier ones are dead at the
 // step that uses the row), each element loaded once.  A dead element brought in with its
@@ -104,24 +113,20 @@ __device__ __forceinline__ void load_urow(float (&u)[CPL], const float* p) {
 // Step I of the column loop, I a compile-time constant so that every register index
 // below is static (no dynamic VGPR indexing).  ub[I & 1] holds this lane's U row I;
 // the step fills ub[(I + 1) & 1] with row I + 1.  With FULL the block has LMAX columns
-// (no length test per step).  Both quotients are the bare reciprocal iteration, their
-// operand ranges recorded in the scalar mask R.inexact (a branch in the loop would
-// serialise it); EXACT uses div_rcp_code for the code and the IEEE division for the
-// error instead, for the rare block that has to be run again.
-template <int I, bool FULL, bool COMP, bool EXACT>
+// (no length test per step).  Both quotients are the bare reciprocal iteration; whether their
+// operands stayed where it is exact is recorded in R (a branch in the loop would serialise it),
+// and the rare wave where they did not runs the block again (gptq_rows_exact).
+template <int I, bool FULL, bool COMP>
 __device__ __forceinline__ void gptq_step(RowRegs<COMP>& R, int L, int q, float nm,
                                           const float* __restrict__ suq, float (&ub)[2][CPL]) {
   constexpr int m = I / QL, s = I % QL, cur = I & 1;
   if (!FULL && I >= L) return;
   if constexpr (I + 1 < LMAX) load_urow<(I + 1) / QL>(ub[cur ^ 1], suq + (I + 1) * USTR);
   const float col = R.w[m];
-  const float lo_j = R.loc[m], st_j = R.stc[m];
-  const float safe = (st_j == 0.0f) ? 1.0f : st_j;
+  const float lo_j = R.loc[m], st_j = R.stc[m];  // a zero step is held as 1 (load_row_c)
   const float dq = col - lo_j;
   float qv;
-  if constexpr (EXACT) {
-    qv = clamp_code(__builtin_rintf(div_rcp_code(dq, safe, R.ys[m])), nm);
-  } else {
+  {
     // div_rcp_code without its select: the iteration's quotient, whose code is the IEEE
     // quotient's while |q0| = |dq ys| <= 2^100.  That holds in every lane the wave keeps:
     // load_row_c marks the wave unless |ys| <= 2^40, |lo| <= 2^40 and |step| <= 2^32, and
@@ -129,35 +134,26 @@ __device__ __forceinline__ void gptq_step(RowRegs<COMP>& R, int L, int q, float 
     // |dq| <= |num| + |wq| + |lo| < 2^51 (NaN and infinities fail those tests).  Every
     // lane kept has a finite quotient, so the clamp is one median (clamp_code's NaN
     // propagation only matters in the waves the rerun redoes).  A zero step's column has
-    // ys = 0 (load_row_c): its quotient is +0 for every finite dq, the code 0 the
-    // reference gives it, without a select in the chain.
-    qv = __builtin_amdgcn_fmed3f(__builtin_rintf(div_rcp_fast(dq, safe, R.ys[m])), 0.0f, nm);
-  }
-  if constexpr (EXACT) {
-    if (st_j == 0.0f) qv = 0.0f;
+    // ys = 0 and step 1 (load_row_c): its quotient is +0 for every finite dq, the code 0 and
+    // the value lo that the reference gives it, without a select in the chain.
+    qv = __builtin_amdgcn_fmed3f(__builtin_rintf(div_rcp_fast(dq, st_j, R.ys[m])), 0.0f, nm);
   }
   const float wq = f16_round(lo_j + qv * st_j);
   const float ujj = ub[cur][m];  // U[I][I] in the owner lane
   const bool own = q == s;
   const float num = col - wq;
-  float e;
-  if constexpr (EXACT) {
-    e = num / ujj;
-  } else {
-    e = div_rcp_fast(num, ujj, R.yu[m]);
-    // div_rcp_ok(num, num yu) holds when |num| is in [2^-50, 2^50] (every column's yu is
-    // in [2^-50, 2^50], checked once per block) or num is +0: tested in every lane, owner
-    // or not (a false alarm only costs a rerun), the lanes that fail OR-ed into a wave
-    // mask in scalar registers
-    // (one ballot per comparison, each the comparison's own lane mask: no vector select)
-    const float an = __builtin_fabsf(num);
-    const uint64_t small = __builtin_amdgcn_ballot_w64(!(an >= 0x1p-50f));  // NaN too
-    const uint64_t large = __builtin_amdgcn_ballot_w64(!(an <= 0x1p50f));
-    // +0 passes (the iteration gives +0 there); -0 does not (it would give +0)
-    const uint64_t zero = __builtin_amdgcn_ballot_w64(num == 0.0f);
-    const uint64_t neg = __builtin_amdgcn_ballot_w64(__builtin_bit_cast(int32_t, num) < 0);
-    R.inexact |= (small | large) & ~(zero & ~neg);
-  }
+  const float e = div_rcp_fast(num, ujj, R.yu[m]);
+  // div_rcp_ok(num, num yu) holds when |num| is in [2^-50, 2^50] (every column's yu is in
+  // [2^-50, 2^50], checked once per block) or num is +0, where the iteration gives +0; -0 does
+  // not pass.  Tested in every lane, owner or not (a false alarm only costs a rerun), once
+  // after the loop, on three running values of four vector instructions a step: the sum of
+  // the magnitudes (at most 2^50 only if each is; NaN and infinities stay in it), the least
+  // bits as a signed integer (-0 and small negative numbers are the least of all) and the
+  // least bits less one as an unsigned one (+0 becomes the greatest of all).
+  const int32_t nb = __builtin_bit_cast(int32_t, num);
+  R.nsum = R.nsum + __builtin_fabsf(num);
+  R.nneg = nb < R.nneg ? nb : R.nneg;
+  R.npos = min(R.npos, (uint32_t)nb - 1u);
   const float eb = row_bcast<s>(e);
   // the selects are pinned here (empty asm): left free, the compiler keeps every step's
   // e and code in its own register until the end of the loop, which costs occupancy
@@ -172,11 +168,11 @@ __device__ __forceinline__ void gptq_step(RowRegs<COMP>& R, int L, int q, float 
   for (int mm = (I + 1) / QL; mm < CPL; ++mm) R.w[mm] = R.w[mm] - eb * ub[cur][mm];
 }
 
-template <bool FULL, bool COMP, bool EXACT, int... Is>
+template <bool FULL, bool COMP, int... Is>
 __device__ __forceinline__ void gptq_steps(std::integer_sequence<int, Is...>, RowRegs<COMP>& R,
                                            int L, int q, float nm, const float* __restrict__ suq,
                                            float (&ub)[2][CPL]) {
-  (gptq_step<Is, FULL, COMP, EXACT>(R, L, q, nm, suq, ub), ...);
+  (gptq_step<Is, FULL, COMP>(R, L, q, nm, suq, ub), ...);
 }
 
 // The state of this lane's 8 columns of row lr of the workgroup, in three parts so that
@@ -192,16 +188,23 @@ __device__ __forceinline__ void load_row_a(RowRegs<COMP>& R, int (&bix)[CPL],
                                            int q) {
   // this row's columns c = 16m + q: the working copy and each column's ladder block, the
   // latter from map gsel of the gspan + 1 block maps at blk (a run of groups sharing one
-  // factor, factor_run_end: gspan * K + L < 2^29, so the byte offsets fit in 32 bits)
-  const __amdgpu_buffer_rsrc_t wrs = mg_rsrc(wc + rbase * K + i1, (int64_t)(nrows - 1) * K + L);
+  // factor, factor_run_end: gspan * K + L < 2^29, so the byte offsets fit in 32 bits); wc
+  // NULL leaves R.w to the caller
+  if (wc != nullptr) {
+    const __amdgpu_buffer_rsrc_t wrs = mg_rsrc(wc + rbase * K + i1, (int64_t)(nrows - 1) * K + L);
+#pragma unroll
+    for (int m = 0; m < CPL; ++m) {
+      const int c = QL * m + q;
+      const uint32_t wo = c < L ? (uint32_t)(((int64_t)lr * K + c) * 4) : MG_OOB;
+      R.w[m] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (int)wo, 0, 0));
+    }
+  }
   const __amdgpu_buffer_rsrc_t brs = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<int32_t*>(blk + i1), (short)0, (int)(((int64_t)gspan * K + L) * 4), 0x00020000);
   const uint32_t boff = (uint32_t)gsel * (uint32_t)K;
 #pragma unroll
   for (int m = 0; m < CPL; ++m) {
     const int c = QL * m + q;
-    const uint32_t wo = c < L ? (uint32_t)(((int64_t)lr * K + c) * 4) : MG_OOB;
-    R.w[m] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(wrs, (int)wo, 0, 0));
     bix[m] = (int)__builtin_amdgcn_raw_buffer_load_b32(
         brs, (int)(c < L ? (boff + (uint32_t)c) * 4u : MG_OOB), 0, 0);
   }
@@ -241,8 +244,12 @@ __device__ __forceinline__ void load_row_c(RowRegs<COMP>& R, int L, const float*
     const float ay = __builtin_fabsf(R.yu[m]);
     yok = yok && ay >= 0x1p-50f && ay <= 0x1p50f && __builtin_fabsf(R.ys[m]) <= 0x1p40f &&
           __builtin_fabsf(R.loc[m]) <= 0x1p40f && __builtin_fabsf(R.stc[m]) <= 0x1p32f;
+    R.stc[m] = R.stc[m] == 0.0f ? 1.0f : R.stc[m];  // no step: code 0 (ys = 0), value lo
   }
-  R.inexact = __builtin_amdgcn_ballot_w64(!yok);
+  R.bounded = yok;
+  R.nsum = 0.0f;
+  R.nneg = INT32_MAX;
+  R.npos = UINT32_MAX;
 }
 template <bool COMP>
 __device__ __forceinline__ void load_row(RowRegs<COMP>& R, const float* __restrict__ wc,
@@ -287,9 +294,8 @@ __device__ __forceinline__ void exact_group(RowRegs<COMP>& R, int L, int q, floa
     if (i >= L) break;  // L is uniform: the whole wave leaves together
     const float col = R.w[M];
     const float lo_j = R.loc[M], st_j = R.stc[M];
-    const float safe = (st_j == 0.0f) ? 1.0f : st_j;
-    float qv = clamp_code(__builtin_rintf((col - lo_j) / safe), nm);
-    if (st_j == 0.0f) qv = 0.0f;
+    float qv = clamp_code(__builtin_rintf((col - lo_j) / st_j), nm);
+    if (R.ys[M] == 0.0f && st_j == 1.0f) qv = 0.0f;  // a zero step (load_row_c)
     const float wq = f16_round(lo_j + qv * st_j);
     const float* ui = suq + i * USTR;
     const float e = (col - wq) / ui[M];  // U[i][i] in the owner lane
@@ -309,7 +315,15 @@ __device__ __forceinline__ void exact_groups(std::integer_sequence<int, Ms...>,
   (exact_group<Ms, COMP>(R, L, q, nm, suq, lane), ...);
 }
 
-// The block for this lane's row again, from the working copy, with IEEE division, then
+// This lane's columns of its row of the workgroup's working tile in LDS (wt: the row).
+template <bool COMP>
+__device__ __forceinline__ void load_tile_row(RowRegs<COMP>& R, const float* wt, int q) {
+#pragma unroll
+  for (int m = 0; m < CPL; ++m) R.w[m] = wt[QL * m + q];
+}
+
+// The block for this lane's row again, from the working copy (memory, or wt: the row of the
+// LDS tile), with IEEE division, then
 // the row's outputs.  Runs only for a wave whose fast pass met an error quotient outside
 // the reciprocal iteration's exact range; it reloads the fast pass's register state R
 // (dead once the wave has decided to run again) instead of holding a second copy.
@@ -320,8 +334,10 @@ __device__ void gptq_rows_exact(RowRegs<COMP>& R, const float* __restrict__ wc, 
                                 const float* __restrict__ lo, const float* __restrict__ st,
                                 int64_t ldp, const float* su, int q, float nm,
                                 float* __restrict__ err1, int64_t lde,
-                                uint8_t* __restrict__ codes, float* __restrict__ comp) {
+                                uint8_t* __restrict__ codes, float* __restrict__ comp,
+                                const float* wt = nullptr) {
   load_row<COMP>(R, wc, K, i1, L, rbase, nrows, lr, blk, gspan, gsel, lo, st, ldp, su, q);
+  if (wt != nullptr) load_tile_row<COMP>(R, wt, q);
   exact_groups<COMP>(std::make_integer_sequence<int, CPL>{}, R, L, q, nm, su + lane_off(q),
                      (int)(threadIdx.x & 63));
   store_row<COMP>(R, K, i1, L, r, q, err1, lde, codes, comp);
@@ -415,8 +431,8 @@ __global__ __launch_bounds__(RPG * QL, 2) void gptq_block_kernel(
     const float* suq = su + lane_off(q);
     float ub[2][CPL];
     load_urow<0>(ub[0], suq);
-    gptq_steps<FULL, COMP, false>(std::make_integer_sequence<int, LMAX>{}, R, L, q, nm, suq, ub);
-    if (R.inexact != 0) {
+    gptq_steps<FULL, COMP>(std::make_integer_sequence<int, LMAX>{}, R, L, q, nm, suq, ub);
+    if (__builtin_amdgcn_ballot_w64(!row_exact(R)) != 0) {
       // some row of this wave met an error quotient outside the iteration's exact range
       // (subnormal or negative-zero numerators, extreme magnitudes): the wave runs the
       // block again from the working copy with IEEE division
@@ -541,6 +557,226 @@ __global__ __launch_bounds__(256, T == MG_T ? 2 : 4) void gptq_trailing_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------------
+// The column loops of a whole super-block in one launch, for batches of few rows.
+//
+// A workgroup keeps its 16 rows through the super-block's blocks.  Before block b's column
+// loop it applies the products of the super-block's earlier blocks to its 16 x 128 tile of
+// block b itself (the near updates, which are launches of their own otherwise): wave v takes
+// columns [32v, 32v + 32) on v_mfma_f32_16x16x4_f32, the errors from LDS, U from L2 a 64-rank
+// chunk ahead, each block's product from zero in k order and subtracted in block order, so the
+// bits are the separate launches'.  The tile goes to the column loop through LDS.
+//
+// What bounds it is latency: a block is its 128-step loop (7 us) and the loads around it.  As
+// launches of their own a column loop takes 16 us (10 of them its start: block map, ladders, U
+// block, reciprocals) and a near update 9-12 us on a grid too small for the chip; here the next
+// block's U, block map and working tile are in flight during the loop.  Alone, the super-blocks of
+// 1024 x 4096 take 58 us of four blocks (897 us of column loops and near updates for the
+// matrix as separate launches, 465 here), those of 4096 x 14336 150 us of eight (2997 and
+// 2100); the whole encode of these 1086 -> 908 and 10480 -> 9520 us.
+// One workgroup per CU (its errors stay in LDS), so it is for batches that fill no more than
+// one round of the CUs: FUSED_ROWS rows.  Beyond, two workgroups per CU of the separate column
+// loops hide each other's latency, and the near updates read each U tile once per 64 rows
+// instead of once per 16 (encode of 4608 x 4096: 2031 us separately, 2133 fused; 9216 x 2560:
+// 1847 and 1987; 4096 x 4096: 1554 fused, 1800 separately).
+// ---------------------------------------------------------------------------------
+constexpr int64_t FUSED_ROWS = 4096;
+constexpr int WSTR = LMAX + 4;  // LDS row stride of the working tile (floats)
+typedef float f32x4g __attribute__((ext_vector_type(4)));
+
+// FULL: every block has LMAX columns (K a multiple of it).
+template <bool FULL, bool COMP, int SB>
+__global__ __launch_bounds__(RPG * QL, 1) void gptq_super_kernel(
+    const float* __restrict__ wc, int64_t N, int64_t K, int64_t i0, int nblk,
+    float* __restrict__ err1, int64_t lde, uint8_t* __restrict__ codes,
+    const float* __restrict__ lo, const float* __restrict__ st, int64_t ldp,
+    const int32_t* __restrict__ row_grp, const int64_t* __restrict__ u_ptrs,
+    const int32_t* __restrict__ blk, const float* __restrict__ nmax,
+    float* __restrict__ comp) {
+  constexpr int ESTR = SB * LMAX + 4;
+  __shared__ float su[LMAX * USTR];
+  __shared__ float et[RPG * ESTR];
+  __shared__ float wt[RPG * WSTR];
+  const int tid = threadIdx.x, lane = tid & 63, q = lane & (QL - 1), g4 = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t rbase = (int64_t)blockIdx.x * RPG;
+  const int lr = wave * RPW + lane / QL;
+  const int64_t r = rbase + lr;
+  const bool live = r < N;
+  const int64_t rend = ((rbase + RPG < N) ? rbase + RPG : N) - 1;
+  const int nrows = (int)(rend - rbase + 1);
+  const int gl0 = row_grp[rbase], gl1 = row_grp[rend];
+  const int gr = live ? row_grp[r] : -1;
+  constexpr int NV = LMAX * LMAX / 4 / (RPG * QL);  // 16-byte vectors of U per thread
+  for (int g = gl0, ge = gl0; g <= gl1; g = ge + 1) {
+    ge = factor_run_end(u_ptrs, g, gl1, K);
+    const bool mine = gr >= g && gr <= ge;
+    const int gsel = mine ? gr - g : 0;
+    const float nm = mine ? nmax[gr] : 0.0f;
+    const float* U = reinterpret_cast<const float*>(u_ptrs[g]);
+    const int32_t* bg = blk + (int64_t)g * K;
+    RowRegs<COMP> R;
+    int bix[CPL];
+    f32x4 uv[NV];
+    float2 tv[4];  // working tile, C layout: rows 4 g4 + i, columns 32 wave + 2q, + 1
+    const int tc = 32 * wave + 2 * q;
+    // block b's U block, block map and working tile
+    auto fetch = [&](int b) {
+      const int64_t i1 = i0 + (int64_t)b * LMAX;
+      const int L = (int)((K - i1 < LMAX) ? K - i1 : LMAX);
+      load_row_a<COMP>(R, bix, nullptr, K, i1, L, rbase, nrows, lr, bg, ge - g, gsel, q);
+      const __amdgpu_buffer_rsrc_t ur = mg_rsrc(U + i1 * K + i1, (int64_t)(L - 1) * K + L);
+#pragma unroll
+      for (int t = 0; t < NV; ++t) {
+        const int idx = tid + RPG * QL * t, i = idx / (LMAX / 4), c = 4 * (idx % (LMAX / 4));
+        uv[t] = mg_load4(ur, i < L ? (uint32_t)(((int64_t)i * K + c) * 4) : MG_OOB);
+      }
+      const __amdgpu_buffer_rsrc_t wr = mg_rsrc(wc + rbase * K + i1, (int64_t)(nrows - 1) * K + L);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        tv[i] = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(
+            wr, (int)(tc < L ? (uint32_t)(((int64_t)(4 * g4 + i) * K + tc) * 4) : MG_OOB), 0, 0));
+    };
+    fetch(0);
+#pragma unroll 1
+    for (int b = 0; b < nblk; ++b) {
+      const int64_t i1 = i0 + (int64_t)b * LMAX;
+      const int L = (int)((K - i1 < LMAX) ? K - i1 : LMAX);
+      // near updates: blocks 0 .. b - 1 of the super-block (whole ones) on this tile, 64 ranks
+      // of U at a time, the next 64 in flight; lane l holds U[k][tc], U[k][tc + 1] for
+      // k = 4s + l / 16 (columns past L are never stored)
+      if (b > 0) {
+        const __amdgpu_buffer_rsrc_t br =
+            mg_rsrc(U + i0 * K + i1, (int64_t)(b * LMAX - 1) * K + L);
+        const uint32_t bo = (uint32_t)(((int64_t)g4 * K + tc) * 4);
+        const uint32_t k4 = (uint32_t)(16 * K);  // bytes of four rows of U
+        float2 bv[2][16];
+        float ev[2][16];
+        const float* ea = &et[q * ESTR + g4];
+        auto chunk = [&](float2 (&v)[16], float (&e)[16], int ch) {
+#pragma unroll
+          for (int s = 0; s < 16; ++s) {
+            v[s] = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(
+                br, (int)(bo + (uint32_t)(16 * ch + s) * k4), 0, 0));
+            e[s] = ea[64 * ch + 4 * s];
+          }
+        };
+        auto mma = [&](f32x4g (&a)[2], const float2 (&v)[16], const float (&e)[16]) {
+          __builtin_amdgcn_sched_barrier(0);  // the next chunk's reads stay ahead of these
+#pragma unroll
+          for (int s = 0; s < 16; ++s) {
+            a[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(e[s], v[s].x, a[0], 0, 0, 0);
+            a[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(e[s], v[s].y, a[1], 0, 0, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        chunk(bv[0], ev[0], 0);
+#pragma unroll 1
+        for (int t = 0; t < b; ++t) {
+          f32x4g a[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+          chunk(bv[1], ev[1], 2 * t + 1);
+          mma(a, bv[0], ev[0]);
+          // (the last block reads the first chunk again: no branch around the loads)
+          chunk(bv[0], ev[0], t + 1 < b ? 2 * t + 2 : 0);
+          mma(a, bv[1], ev[1]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            tv[i].x = tv[i].x - a[0][i];
+            tv[i].y = tv[i].y - a[1][i];
+          }
+        }
+      }
+      load_row_b<COMP>(R, bix, rbase, nrows, lr, lo, st, ldp);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<float2*>(&wt[(4 * g4 + i) * WSTR + tc]) = tv[i];
+#pragma unroll
+      for (int t = 0; t < NV; ++t) {
+        const int idx = tid + RPG * QL * t, i = idx / (LMAX / 4), c = 4 * (idx % (LMAX / 4));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int cc = c + e;
+          const float v = uv[t][e];
+          su[i * USTR + lane_off(cc % QL) + cc / QL] = (cc < L) ? v : 0.0f;
+        }
+      }
+      __syncthreads();
+      load_tile_row<COMP>(R, wt + lr * WSTR, q);
+      load_row_c<COMP>(R, L, su, q);
+      if (b + 1 < nblk) fetch(b + 1);
+      // the U panel of the next near update, rows of blocks 0 .. b, into this XCD's L2 while the
+      // loop runs: each of its workgroups (blockIdx % 8) touches its share of the 128-byte lines
+      // (values unused; without it every chunk of the panel waits for a first touch)
+      float touch[4];
+      {
+        const __amdgpu_buffer_rsrc_t pr = mg_rsrc(U + i0 * K + i1 + LMAX,
+                                                  (int64_t)((b + 1) * LMAX - 1) * K + LMAX);
+        const uint32_t nl = b + 1 < nblk && i1 + 2 * LMAX <= K ? 4u * (b + 1) * LMAX : 0u;
+        const uint32_t step = ((gridDim.x + 7) >> 3) * (RPG * QL);
+        const uint32_t at = (blockIdx.x >> 3) * (RPG * QL) + tid;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const uint32_t li = at + t * step;
+          const uint32_t off = li < nl ? ((li >> 2) * (uint32_t)K + 32u * (li & 3)) * 4u : MG_OOB;
+          touch[t] = __builtin_bit_cast(
+              float, __builtin_amdgcn_raw_buffer_load_b32(pr, (int)off, 0, 0));
+        }
+      }
+      const float* suq = su + lane_off(q);
+      float ub[2][CPL];
+      load_urow<0>(ub[0], suq);
+      if (FULL || L == LMAX)
+        gptq_steps<true, COMP>(std::make_integer_sequence<int, LMAX>{}, R, L, q, nm, suq, ub);
+      else
+        gptq_steps<false, COMP>(std::make_integer_sequence<int, LMAX>{}, R, L, q, nm, suq, ub);
+      asm volatile("" ::"v"(touch[0]), "v"(touch[1]), "v"(touch[2]), "v"(touch[3]));
+      float* eb = err1 + b * LMAX;
+      if (mine) {
+        if (__builtin_amdgcn_ballot_w64(!row_exact(R)) != 0)
+          gptq_rows_exact<COMP>(R, nullptr, K, i1, L, rbase, nrows, lr, r, bg, ge - g, gsel, lo, st,
+                                ldp, su, q, nm, eb, lde, codes, comp, wt + lr * WSTR);
+        else
+          store_row<COMP>(R, K, i1, L, r, q, eb, lde, codes, comp);
+      }
+#pragma unroll
+      for (int m = 0; m < CPL; ++m) et[lr * ESTR + b * LMAX + QL * m + q] = R.er[m];
+      __syncthreads();
+    }
+  }
+}
+
+int launch_super(const float* wc, int64_t n, int64_t k, int64_t i0, int nblk, float* err1,
+                 int64_t lde, uint8_t* codes, const float* lo, const float* st, int64_t ldp,
+                 const int32_t* row_grp, const int64_t* u_ptrs, const int32_t* blk,
+                 const float* nmax, float* comp, hipStream_t s) {
+  const dim3 grid((unsigned)((n + RPG - 1) / RPG));
+  double work = 0.0;
+  for (int b = 0; b < nblk; ++b) {
+    const double len = (double)std::min<int64_t>(LMAX, k - (i0 + (int64_t)b * LMAX));
+    work += n * len * (len - 1) + 2.0 * n * len * b * LMAX;  // the loop and its near updates
+  }
+  LaunchTimer timer(HI2X_TIME_GPTQ_BLOCK, work, s);
+  const bool full = i0 + (int64_t)nblk * LMAX <= k;
+#define HI2X_SUPER_LAUNCH(F, C, SB)                                                          \
+  hipLaunchKernelGGL((gptq_super_kernel<F, C, SB>), grid, dim3(RPG * QL), 0, s, wc, n, k, i0, \
+                     nblk, err1, lde, codes, lo, st, ldp, row_grp, u_ptrs, blk, nmax, comp)
+#define HI2X_SUPER_SB(F, C)                \
+  if (nblk <= 4) HI2X_SUPER_LAUNCH(F, C, 4); \
+  else HI2X_SUPER_LAUNCH(F, C, 8)
+  if (full && comp) {
+    HI2X_SUPER_SB(true, true);
+  } else if (full) {
+    HI2X_SUPER_SB(true, false);
+  } else if (comp) {
+    HI2X_SUPER_SB(false, true);
+  } else {
+    HI2X_SUPER_SB(false, false);
+  }
+#undef HI2X_SUPER_SB
+#undef HI2X_SUPER_LAUNCH
+  return launch_status("gptq_super_kernel");
+}
+
 int launch_block(const float* wc, int64_t n, int64_t k, int64_t i1, int64_t len, float* err1,
                  int64_t lde, uint8_t* codes, const float* lo, const float* st, int64_t ldp,
                  const int32_t* row_grp, const int64_t* u_ptrs, const int32_t* blk,
@@ -659,7 +895,13 @@ extern "C" int hi2x_gptq_run(float* wc, int64_t n, int64_t k, uint8_t* codes, co
   for (int64_t sb = 0; sb < nblocks; sb += super_blocks) {
     const int64_t sb_end = (sb + super_blocks < nblocks) ? sb + super_blocks : nblocks;
     const int64_t cs_end = (sb_end * LMAX < k) ? sb_end * LMAX : k;
-    for (int64_t b = sb; b < sb_end; ++b) {
+    const bool fused = n <= FUSED_ROWS && super_blocks > 1 && super_blocks <= 8;
+    if (fused) {
+      const int rc = launch_super(wc, n, k, sb * LMAX, (int)(sb_end - sb), err_ws, lde, codes, lo,
+                                  st, ldp, row_grp, u_ptrs, blk, nmax, comp, s);
+      if (rc) return rc;
+    }
+    for (int64_t b = sb; b < sb_end && !fused; ++b) {
       const int64_t i1 = b * LMAX;
       const int64_t len = (k - i1 < LMAX) ? k - i1 : LMAX;
       float* eb = err_ws + (b - sb) * LMAX;
