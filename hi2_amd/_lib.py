@@ -70,6 +70,8 @@ SIGNATURES = {
     "hi2x_qad_decode_fwd": [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I, _F, _P],
     "hi2x_qad_decode_bwd": [_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I, _F, _P, _P,
                             _P],
+    "hi2x_qad_weights_fwd": [_P, _P, _P, _I64, _I64, _I64, _P, _P, _P, _P],
+    "hi2x_qad_weights_bwd": [_P, _P, _P, _P, _I64, _I64, _I64, _P, _P, _P, _P],
     "hi2x_qad_wht_scale": [_P, _I64, _I64, _P, _P, _I, _P],
 }
 class Piece(ctypes.Structure):
@@ -79,6 +81,13 @@ class Piece(ctypes.Structure):
                 ("k", _I64), ("nbits", ctypes.c_int32), ("pad_", ctypes.c_int32),
                 ("block", _I64), ("code_off", _P), ("param_off", _P), ("out_codes", _P),
                 ("out_params", _P), ("out_consts", _P)]
+
+
+class QadGroup(ctypes.Structure):
+    """hi2x_qad_group (include/hi2x.h): one group of hi2x_qad_weights_fwd / _bwd."""
+
+    _fields_ = [("lo_u", _P), ("st_u", _P), ("consts", _P), ("rows", _P), ("n_rows", _I64),
+                ("block", ctypes.c_int32), ("nmax", _F), ("g_lo", _P), ("g_st", _P)]
 
 
 SIGNATURES["hi2x_assemble_batch"] = [_P, _I64, _P, _P]
@@ -284,6 +293,9 @@ def workspace(dev: torch.device, size_fn: str, *args) -> torch.Tensor:
 def call(name: str, dev: torch.device, *args) -> None:
     """Call ``name`` with ``args`` + the current stream of ``dev`` (device made current)."""
     fn = getattr(lib(), name)
-    with torch.cuda.device(dev):
+    if torch.cuda.current_device() == dev.index:  # the usual case, without the guard's cost
         rc = fn(*args, stream(dev))
+    else:
+        with torch.cuda.device(dev):
+            rc = fn(*args, stream(dev))
     check(rc, name)

@@ -55,8 +55,61 @@ __device__ __forceinline__ float at(const float4& v, int i) {
   return i == 0 ? v.x : (i == 1 ? v.y : (i == 2 ? v.z : v.w));
 }
 
+// One cross-lane level of the butterfly: partner lane ^ M of the 4-lane group (CTRL its
+// DPP quad_perm), the upper lane keeping the difference.
+template <int M, int CTRL>
+__device__ __forceinline__ void butterfly_step(float4& v, int lane) {
+  const bool upper = (lane & M) != 0;
+  float4 p;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    at(p, e) = __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, at(v, e)), CTRL, 0xf, 0xf,
+                                           true));
+#pragma unroll
+  for (int e = 0; e < 4; ++e) at(v, e) = upper ? at(p, e) - at(v, e) : at(v, e) + at(p, e);
+}
+
+// H16 of a 16-column group (without the factor 0.25) held by four consecutive lanes, 4 columns
+// each: y[t] = (t & h) ? y[t ^ h] - y[t] : y[t] + y[t ^ h] for h = 1, 2 inside the lane, then 4
+// and 8 between the lanes (aligned in the wave).
+__device__ __forceinline__ float4 butterfly16(float4 v, int lane) {
+  float4 y;
+  y.x = v.x + v.y; y.y = v.x - v.y; y.z = v.z + v.w; y.w = v.z - v.w;
+  v.x = y.x + y.z; v.z = y.x - y.z; v.y = y.y + y.w; v.w = y.y - y.w;
+  butterfly_step<1, 0xB1>(v, lane);  // DPP quad_perm [1,0,3,2]: lane ^ 1
+  butterfly_step<2, 0x4E>(v, lane);  // [2,3,0,1]: lane ^ 2
+  return v;
+}
+
+// H16(v) on a flagged group, v elsewhere, then / scale (PRE: / scale first), columns c0 .. c0 + 3.
+template <bool PRE>
+__device__ __forceinline__ float4 wht_scale4(float4 v, int64_t c0,
+                                             const uint8_t* __restrict__ flags,
+                                             const uint16_t* __restrict__ scale) {
+  float4 s = make_float4(1.f, 1.f, 1.f, 1.f);
+  if (scale) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) at(s, e) = f16_from_bits(scale[c0 + e]);
+    if (PRE) {
+      v.x = v.x / s.x; v.y = v.y / s.y; v.z = v.z / s.z; v.w = v.w / s.w;
+    }
+  }
+  const float4 h = butterfly16(v, threadIdx.x & 63);
+  float4 o = flags[c0 >> 4] != 0
+                 ? make_float4(h.x * 0.25f, h.y * 0.25f, h.z * 0.25f, h.w * 0.25f)
+                 : v;
+  if (!PRE && scale) {
+    o.x = o.x / s.x; o.y = o.y / s.y; o.z = o.z / s.z; o.w = o.w / s.w;
+  }
+  return o;
+}
+
 // out[rows[r], :] = fp16(lo + q * step) (the sum in f64), for the group's
-// rows r; v = latent (times unit when given).
+// rows r; v = latent (times unit when given).  With flags, the rotation of the flagged groups
+// and the division by scale follow in registers (H16(out) / scale, qad_wht_scale_kernel's
+// operations): the weights of a 4096 x 4096 Linear in one pass over latent, unit and out
+// instead of two (40 us of kernels for forward, 62 for backward; 60 and 76 as two passes).
 // The block's divisions by safe (the fp32 divisions of the torch graph) as div_rcp
 // through one reciprocal per thread: bit-identical to IEEE division for every numerator.
 template <int SHIFT>
@@ -64,7 +117,8 @@ __global__ __launch_bounds__(QT) void qad_decode_fwd_kernel(
     const float* __restrict__ latent, const float* __restrict__ unit,
     const float* __restrict__ lo_u, const float* __restrict__ st_u,
     const uint16_t* __restrict__ consts, const int64_t* __restrict__ rows, int64_t n_rows,
-    int64_t r_total, int64_t k, float nmax, float* __restrict__ out) {
+    int64_t r_total, int64_t k, float nmax, const uint8_t* __restrict__ flags,
+    const uint16_t* __restrict__ scale, float* __restrict__ out) {
   constexpr int shift = SHIFT;
   // thread (row, column quad); the host keeps n_rows * k / 4 below 2^31, so the index
   // arithmetic is 32-bit (a 64-bit division is a long emulated sequence on the SIMD)
@@ -95,6 +149,8 @@ __global__ __launch_bounds__(QT) void qad_decode_fwd_kernel(
     const double val = (double)l.lo + (double)q * (double)l.st;
     at(o, e) = f16_round((float)val);
   }
+  // (a row's threads come in whole groups of four lanes, so a group's lanes are all here)
+  if (flags) o = wht_scale4<false>(o, c0, flags, scale);
   st4(out + off, o);
 }
 
@@ -102,7 +158,8 @@ __global__ __launch_bounds__(QT) void qad_decode_fwd_kernel(
 //   gz = G * step inside the clamp range [0, nmax] of z, else 0;  d latent = gz / safe
 //   (times unit);  d lo_byte = lo_scale * sum_block(G - gz / safe);
 //   d step_byte = step_scale * sum_block(G * q - [step != 0] gz * (z / safe)).
-// The block sums are the pairwise tree s[i] += s[i + h] for h = B/2 .. 1: the levels
+// With flags, G is H16(grad / scale) of the gradient given (the transform's backward), formed in
+// registers as in the forward.  The block sums are the pairwise tree s[i] += s[i + h] for h = B/2 .. 1: the levels
 // h >= 4 are shuffles between the block's lanes, h = 2 and 1 inside the lane.
 // Lane j + D of this lane's row of 16 (DPP row_shl; past the row's end 0: such lanes'
 // sums are never read).  Written as update_dpp so that the add folds it in.
@@ -133,8 +190,8 @@ __global__ __launch_bounds__(QT) void qad_decode_bwd_kernel(
     const float* __restrict__ unit, const float* __restrict__ lo_u,
     const float* __restrict__ st_u, const uint16_t* __restrict__ consts,
     const int64_t* __restrict__ rows, int64_t n_rows, int64_t r_total, int64_t k,
-    float nmax, float* __restrict__ g_latent, float* __restrict__ g_lo,
-    float* __restrict__ g_st) {
+    float nmax, const uint8_t* __restrict__ flags, const uint16_t* __restrict__ scale,
+    float* __restrict__ g_latent, float* __restrict__ g_lo, float* __restrict__ g_st) {
   constexpr int shift = SHIFT;
   const uint32_t k4 = (uint32_t)(k >> 2);
   const uint32_t i = blockIdx.x * QT + threadIdx.x;
@@ -162,7 +219,8 @@ __global__ __launch_bounds__(QT) void qad_decode_bwd_kernel(
       u = ld4(unit + off);
       v.x *= u.x; v.y *= u.y; v.z *= u.z; v.w *= u.w;
     }
-    const float4 g = ld4(grad + off);
+    float4 g = ld4(grad + off);
+    if (flags) g = wht_scale4<true>(g, c0, flags, scale);
     float4 gl;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -194,62 +252,18 @@ __global__ __launch_bounds__(QT) void qad_decode_bwd_kernel(
 }
 
 // out = H16(x) / scale over the flagged 16-column groups (x / scale elsewhere), or with
-// pre_div the division first: H16(x / scale).  H16 is the butterfly
-// y[t] = (t & h) ? y[t ^ h] - y[t] : y[t] + y[t ^ h] for h = 1, 2, 4, 8, then * 0.25.
-// h = 1, 2 act inside a lane's 4 columns, h = 4, 8 between the group's 4 lanes.
-// One cross-lane level of the butterfly: partner lane ^ M of the 4-lane group (CTRL its
-// DPP quad_perm), the upper lane keeping the difference.
-template <int M, int CTRL>
-__device__ __forceinline__ void butterfly_step(float4& v, int lane) {
-  const bool upper = (lane & M) != 0;
-  float4 p;
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-    at(p, e) = __builtin_bit_cast(
-        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, at(v, e)), CTRL, 0xf, 0xf,
-                                           true));
-#pragma unroll
-  for (int e = 0; e < 4; ++e) at(v, e) = upper ? at(p, e) - at(v, e) : at(v, e) + at(p, e);
-}
-
+// pre_div the division first: H16(x / scale).
 __global__ __launch_bounds__(QT) void qad_wht_scale_kernel(
     const float* __restrict__ x, int64_t n_rows, int64_t k, const uint8_t* __restrict__ flags,
     const uint16_t* __restrict__ scale, int pre_div, float* __restrict__ out) {
   const uint32_t k4 = (uint32_t)(k >> 2);
   const uint32_t i = blockIdx.x * QT + threadIdx.x;
-  const bool valid = i < (uint32_t)n_rows * k4;
-  float4 v = make_float4(0.f, 0.f, 0.f, 0.f), s = make_float4(1.f, 1.f, 1.f, 1.f);
-  int64_t c0 = 0, r = 0;
-  if (valid) {
-    const uint32_t r32 = i / k4;
-    r = r32;
-    c0 = (int64_t)(i - r32 * k4) << 2;
-    v = ld4(x + r * k + c0);
-    if (scale) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) at(s, e) = f16_from_bits(scale[c0 + e]);
-      if (pre_div) {
-        v.x = v.x / s.x; v.y = v.y / s.y; v.z = v.z / s.z; v.w = v.w / s.w;
-      }
-    }
-  }
-  const float4 orig = v;
-  // h = 1
-  float4 y;
-  y.x = v.x + v.y; y.y = v.x - v.y; y.z = v.z + v.w; y.w = v.z - v.w;
-  // h = 2
-  v.x = y.x + y.z; v.z = y.x - y.z; v.y = y.y + y.w; v.w = y.y - y.w;
-  // h = 4, 8: partner lane j ^ 1, j ^ 2 of the group (lanes 4-aligned in the wave)
-  const int lane = threadIdx.x & 63;
-  butterfly_step<1, 0xB1>(v, lane);  // DPP quad_perm [1,0,3,2]: lane ^ 1
-  butterfly_step<2, 0x4E>(v, lane);  // [2,3,0,1]: lane ^ 2
-  if (!valid) return;
-  const bool flagged = flags[c0 >> 4] != 0;
-  float4 o = flagged ? make_float4(v.x * 0.25f, v.y * 0.25f, v.z * 0.25f, v.w * 0.25f) : orig;
-  if (scale && !pre_div) {
-    o.x = o.x / s.x; o.y = o.y / s.y; o.z = o.z / s.z; o.w = o.w / s.w;
-  }
-  st4(out + r * k + c0, o);
+  if (i >= (uint32_t)n_rows * k4) return;  // whole groups of four lanes
+  const uint32_t r32 = i / k4;
+  const int64_t r = r32, c0 = (int64_t)(i - r32 * k4) << 2;
+  const float4 v = ld4(x + r * k + c0);
+  st4(out + r * k + c0, pre_div ? wht_scale4<true>(v, c0, flags, scale)
+                                : wht_scale4<false>(v, c0, flags, scale));
 }
 
 int block_shift(int block) { return block == 16 ? 4 : (block == 32 ? 5 : (block == 64 ? 6 : -1)); }
@@ -261,24 +275,24 @@ bool aligned16(const void* p) { return p == nullptr || ((uintptr_t)p & 15) == 0;
 
 using namespace hi2x;
 
-extern "C" int hi2x_qad_decode_fwd(const float* latent, const float* unit, const float* lo_u,
-                                   const float* st_u, const uint16_t* consts,
-                                   const int64_t* rows, int64_t n_rows, int64_t r_total,
-                                   int64_t k, int block, float nmax, float* out, void* stream) {
+static int decode_fwd(const char* what, const float* latent, const float* unit, const float* lo_u,
+                      const float* st_u, const uint16_t* consts, const int64_t* rows,
+                      int64_t n_rows, int64_t r_total, int64_t k, int block, float nmax,
+                      const uint8_t* flags, const uint16_t* scale, float* out, void* stream) {
   clear_error();
   const int shift = block_shift(block);
-  HI2X_REQUIRE(shift > 0, "qad_decode_fwd: block %d must be 16, 32 or 64", block);
+  HI2X_REQUIRE(shift > 0, "%s: block %d must be 16, 32 or 64", what, block);
   HI2X_REQUIRE(n_rows >= 0 && r_total >= 0 && k > 0 && k % block == 0,
-               "qad_decode_fwd: K=%lld must be a positive multiple of the block", (long long)k);
+               "%s: K=%lld must be a positive multiple of the block", what, (long long)k);
   HI2X_REQUIRE(aligned16(latent) && aligned16(unit) && aligned16(out),
-               "qad_decode_fwd: latent, unit and out must be 16-byte aligned");
+               "%s: latent, unit and out must be 16-byte aligned", what);
   if (n_rows == 0) return HI2X_OK;
   const int64_t total = n_rows * (k / 4);
-  HI2X_REQUIRE(total < (int64_t(1) << 31), "qad_decode_fwd: %lld rows x K too large", (long long)n_rows);
+  HI2X_REQUIRE(total < (int64_t(1) << 31), "%s: %lld rows x K too large", what, (long long)n_rows);
   const dim3 grid((unsigned)((total + QT - 1) / QT));
 #define HI2X_QAD_FWD(S)                                                                     \
   hipLaunchKernelGGL(qad_decode_fwd_kernel<S>, grid, dim3(QT), 0, as_stream(stream), latent, \
-                     unit, lo_u, st_u, consts, rows, n_rows, r_total, k, nmax, out)
+                     unit, lo_u, st_u, consts, rows, n_rows, r_total, k, nmax, flags, scale, out)
   if (shift == 4) HI2X_QAD_FWD(4);
   else if (shift == 5) HI2X_QAD_FWD(5);
   else HI2X_QAD_FWD(6);
@@ -286,31 +300,79 @@ extern "C" int hi2x_qad_decode_fwd(const float* latent, const float* unit, const
   return launch_status("qad_decode_fwd_kernel");
 }
 
-extern "C" int hi2x_qad_decode_bwd(const float* grad, const float* latent, const float* unit,
-                                   const float* lo_u, const float* st_u, const uint16_t* consts,
-                                   const int64_t* rows, int64_t n_rows, int64_t r_total,
-                                   int64_t k, int block, float nmax, float* g_latent, float* g_lo,
-                                   float* g_st, void* stream) {
+static int decode_bwd(const char* what, const float* grad, const float* latent, const float* unit,
+                      const float* lo_u, const float* st_u, const uint16_t* consts,
+                      const int64_t* rows, int64_t n_rows, int64_t r_total, int64_t k, int block,
+                      float nmax, const uint8_t* flags, const uint16_t* scale, float* g_latent,
+                      float* g_lo, float* g_st, void* stream) {
   clear_error();
   const int shift = block_shift(block);
-  HI2X_REQUIRE(shift > 0, "qad_decode_bwd: block %d must be 16, 32 or 64", block);
+  HI2X_REQUIRE(shift > 0, "%s: block %d must be 16, 32 or 64", what, block);
   HI2X_REQUIRE(n_rows >= 0 && r_total >= 0 && k > 0 && k % block == 0,
-               "qad_decode_bwd: K=%lld must be a positive multiple of the block", (long long)k);
+               "%s: K=%lld must be a positive multiple of the block", what, (long long)k);
   HI2X_REQUIRE(aligned16(grad) && aligned16(latent) && aligned16(unit) && aligned16(g_latent),
-               "qad_decode_bwd: grad, latent, unit and g_latent must be 16-byte aligned");
+               "%s: grad, latent, unit and g_latent must be 16-byte aligned", what);
   if (n_rows == 0) return HI2X_OK;
   const int64_t total = n_rows * (k / 4);
-  HI2X_REQUIRE(total < (int64_t(1) << 31), "qad_decode_bwd: %lld rows x K too large", (long long)n_rows);
+  HI2X_REQUIRE(total < (int64_t(1) << 31), "%s: %lld rows x K too large", what, (long long)n_rows);
   const dim3 grid((unsigned)((total + QT - 1) / QT));
 #define HI2X_QAD_BWD(S)                                                                    \
   hipLaunchKernelGGL(qad_decode_bwd_kernel<S>, grid, dim3(QT), 0, as_stream(stream), grad, \
                      latent, unit, lo_u, st_u, consts, rows, n_rows, r_total, k, nmax,     \
-                     g_latent, g_lo, g_st)
+                     flags, scale, g_latent, g_lo, g_st)
   if (shift == 4) HI2X_QAD_BWD(4);
   else if (shift == 5) HI2X_QAD_BWD(5);
   else HI2X_QAD_BWD(6);
 #undef HI2X_QAD_BWD
   return launch_status("qad_decode_bwd_kernel");
+}
+
+extern "C" int hi2x_qad_decode_fwd(const float* latent, const float* unit, const float* lo_u,
+                                   const float* st_u, const uint16_t* consts,
+                                   const int64_t* rows, int64_t n_rows, int64_t r_total,
+                                   int64_t k, int block, float nmax, float* out, void* stream) {
+  return decode_fwd("qad_decode_fwd", latent, unit, lo_u, st_u, consts, rows, n_rows, r_total, k,
+                    block, nmax, nullptr, nullptr, out, stream);
+}
+
+extern "C" int hi2x_qad_decode_bwd(const float* grad, const float* latent, const float* unit,
+                                   const float* lo_u, const float* st_u, const uint16_t* consts,
+                                   const int64_t* rows, int64_t n_rows, int64_t r_total,
+                                   int64_t k, int block, float nmax, float* g_latent, float* g_lo,
+                                   float* g_st, void* stream) {
+  return decode_bwd("qad_decode_bwd", grad, latent, unit, lo_u, st_u, consts, rows, n_rows,
+                    r_total, k, block, nmax, nullptr, nullptr, g_latent, g_lo, g_st, stream);
+}
+
+extern "C" int hi2x_qad_weights_fwd(const float* latent, const float* unit,
+                                    const hi2x_qad_group* groups, int64_t n_groups,
+                                    int64_t r_total, int64_t k, const uint8_t* flags,
+                                    const uint16_t* scale, float* out, void* stream) {
+  clear_error();
+  HI2X_REQUIRE(n_groups >= 0 && (groups || n_groups == 0), "qad_weights_fwd: bad groups");
+  for (int64_t i = 0; i < n_groups; ++i) {
+    const hi2x_qad_group& g = groups[i];
+    const int rc = decode_fwd("qad_weights_fwd", latent, unit, g.lo_u, g.st_u, g.consts, g.rows,
+                              g.n_rows, r_total, k, g.block, g.nmax, flags, scale, out, stream);
+    if (rc) return rc;
+  }
+  return HI2X_OK;
+}
+
+extern "C" int hi2x_qad_weights_bwd(const float* grad, const float* latent, const float* unit,
+                                    const hi2x_qad_group* groups, int64_t n_groups,
+                                    int64_t r_total, int64_t k, const uint8_t* flags,
+                                    const uint16_t* scale, float* g_latent, void* stream) {
+  clear_error();
+  HI2X_REQUIRE(n_groups >= 0 && (groups || n_groups == 0), "qad_weights_bwd: bad groups");
+  for (int64_t i = 0; i < n_groups; ++i) {
+    const hi2x_qad_group& g = groups[i];
+    const int rc = decode_bwd("qad_weights_bwd", grad, latent, unit, g.lo_u, g.st_u, g.consts,
+                              g.rows, g.n_rows, r_total, k, g.block, g.nmax, flags, scale,
+                              g_latent, g.g_lo, g.g_st, stream);
+    if (rc) return rc;
+  }
+  return HI2X_OK;
 }
 
 extern "C" int hi2x_qad_wht_scale(const float* x, int64_t n_rows, int64_t k,

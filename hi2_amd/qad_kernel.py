@@ -1,9 +1,9 @@
 """Fused ladder decode of QAD's fake-quantised Linears on MI355X, forward and backward.
 
 Mirror of the reference's ``hi2/qad_kernel.py`` (``load`` 229-258, ``available`` 261-268,
-``failure`` 271-272, ``_StoredDecode`` 275-318, ``_Transform`` 321-336, ``original``
-339-348, ``stored`` 351-370), backed by ``hi2x_qad_decode_fwd``, ``hi2x_qad_decode_bwd``
-and ``hi2x_qad_wht_scale`` of ``libhi2x.so``.  ``load()`` returns an object with the
+``failure`` 271-272, ``_StoredDecode`` 275-318, ``_Transform`` 321-336, ``original`` 339-348,
+``stored`` 351-370), backed by ``hi2x_qad_decode_fwd/bwd``, ``hi2x_qad_weights_fwd/bwd`` (the
+decode with the transform) and ``hi2x_qad_wht_scale`` of ``libhi2x.so``.  ``load()`` returns an object with the
 extension's three functions (``decode_fwd``, ``decode_bwd``, ``wht_scale``, same
 arguments), so code written against the reference's extension runs unchanged.  The
 calls never wait for the device: a group row outside the latent is skipped by the
@@ -17,6 +17,7 @@ kernel's pairwise-tree order, and the transform is the reference kernel's butter
 torch graph, as in the reference); ``=kernel`` makes a missing library an error.
 """
 
+import ctypes
 import os
 
 import torch
@@ -52,6 +53,36 @@ def _group_args(latent, unit, lo_u, st_u, consts, rows, block):
     if tuple(consts.shape) != (n, 3):
         raise RuntimeError("consts must be [rows, 3]")
     return k, n
+
+
+def _transform_args(flags, scale, k):
+    """The rotation flags and smoothing vector as pointers, checked as ``wht_scale`` checks
+    them (None without a transform)."""
+    if flags is None:
+        return None, None
+    _check(flags, torch.uint8, "flags")
+    if k % 16 or flags.numel() != k // 16:
+        raise RuntimeError("K must be a multiple of 16 with one flag per 16 columns")
+    if scale is not None and scale.numel():
+        _check(scale, torch.float16, "scale")
+        if scale.numel() != k:
+            raise RuntimeError("scale must have K entries")
+    return _lib.ptr(flags), _opt(scale)
+
+
+def _group_table(latent, unit, meta, params, grads=None):
+    """The groups of a tensor as the library's array (and its width), each checked as
+    ``decode_fwd`` checks it; ``grads``: the byte gradients ``[lo, st]`` of every group."""
+    tab = (_lib.QadGroup * max(len(meta), 1))()
+    for gi, (rows, consts, nbits, block) in enumerate(meta):
+        lo_u, st_u = params[2 * gi], params[2 * gi + 1]
+        _lib.require_gpu(latent, lo_u, st_u, consts, rows)
+        _, n = _group_args(latent, unit, lo_u, st_u, consts, rows, block)
+        tab[gi] = _lib.QadGroup(
+            lo_u.data_ptr(), st_u.data_ptr(), consts.data_ptr(), rows.data_ptr(), n, int(block),
+            float(2 ** nbits - 1), *((g.data_ptr() for g in grads[2 * gi:2 * gi + 2])
+                                     if grads else (None, None)))
+    return tab
 
 
 class _Kernels:
@@ -140,33 +171,52 @@ def _mod():
     return mod
 
 
+def _decode(latent, unit, meta, flags, scale, params, out) -> None:
+    """Every group's rows of ``out``: the stored values, or with ``flags`` the weights in the
+    model's basis, in one call."""
+    _mod()
+    if not meta:
+        return
+    tab = _group_table(latent, unit, meta, params)
+    fl, sc = _transform_args(flags, scale, latent.shape[1])
+    _lib.call("hi2x_qad_weights_fwd", _lib.require_gpu(latent, out, flags, scale),
+              _lib.ptr(latent), _opt(unit), ctypes.cast(tab, ctypes.c_void_p), len(meta),
+              latent.shape[0], latent.shape[1], fl, sc, _lib.ptr(out))
+
+
+def _decode_grads(ctx, grad, flags, scale):
+    """The latent's gradient and every group's byte gradients."""
+    latent, unit, *params = ctx.saved_tensors
+    _mod()
+    grad = grad.contiguous()
+    g_latent = torch.empty_like(latent)
+    grads = [torch.empty_like(p) for p in params]
+    if ctx.meta:
+        _check(grad, torch.float32, "grad")
+        if grad.shape != latent.shape:
+            raise RuntimeError("grad must have the latent's shape")
+        tab = _group_table(latent, unit, ctx.meta, params, grads)
+        fl, sc = _transform_args(flags, scale, latent.shape[1])
+        _lib.call("hi2x_qad_weights_bwd", _lib.require_gpu(grad, latent, flags, scale),
+                  _lib.ptr(grad), _lib.ptr(latent), _opt(unit), ctypes.cast(tab, ctypes.c_void_p),
+                  len(ctx.meta), latent.shape[0], latent.shape[1], fl, sc, _lib.ptr(g_latent))
+    return g_latent, grads
+
+
 class _StoredDecode(torch.autograd.Function):
     """``stored = decode(latent, unit, ladder bytes)`` over all groups of one tensor."""
 
     @staticmethod
     def forward(ctx, latent, unit, meta, *params):
         out = torch.empty_like(latent)
-        mod = _mod()
-        for gi, (rows, consts, nbits, block) in enumerate(meta):
-            mod.decode_fwd(latent, unit, params[2 * gi], params[2 * gi + 1], consts, rows, block,
-                           float(2 ** nbits - 1), out)
+        _decode(latent, unit, meta, None, None, params, out)
         ctx.meta = meta
         ctx.save_for_backward(latent, unit, *params)
         return out
 
     @staticmethod
     def backward(ctx, grad):
-        latent, unit, *params = ctx.saved_tensors
-        grad = grad.contiguous()
-        g_latent = torch.empty_like(latent)
-        grads = []
-        mod = _mod()
-        for gi, (rows, consts, nbits, block) in enumerate(ctx.meta):
-            g_lo = torch.empty_like(params[2 * gi])
-            g_st = torch.empty_like(params[2 * gi])
-            mod.decode_bwd(grad, latent, unit, params[2 * gi], params[2 * gi + 1], consts, rows,
-                           block, float(2 ** nbits - 1), g_latent, g_lo, g_st)
-            grads += [g_lo, g_st]
+        g_latent, grads = _decode_grads(ctx, grad, None, None)
         return (g_latent, None, None, *grads)
 
 
@@ -187,28 +237,53 @@ class _Transform(torch.autograd.Function):
         return out, None, None
 
 
+class _Weights(torch.autograd.Function):
+    """``_Transform`` of ``_StoredDecode`` in one pass per group and direction."""
+
+    @staticmethod
+    def forward(ctx, latent, unit, meta, flags, scale, *params):
+        out = torch.empty_like(latent)
+        _decode(latent, unit, meta, flags, scale, params, out)
+        ctx.meta, ctx.flags, ctx.scale = meta, flags, scale
+        ctx.save_for_backward(latent, unit, *params)
+        return out
+
+    @staticmethod
+    def backward(ctx, grad):
+        g_latent, grads = _decode_grads(ctx, grad, ctx.flags, ctx.scale)
+        return (g_latent, None, None, None, None, *grads)
+
+
+def _groups(fq):
+    return ([(g.rows, g.consts, g.nbits, g.block) for g in fq.groups],
+            [p for g in fq.groups for p in (g.lo_u, g.step_u)])
+
+
+def _values(fq, meta, params, flags, scale) -> torch.Tensor:
+    with torch.no_grad():
+        out = torch.empty_like(fq.latent)
+        _decode(fq.latent.detach(), fq.unit, meta, flags, scale, [p.detach() for p in params],
+                out)
+        return out
+
+
 def original(fq) -> torch.Tensor:
     """The weights of a fake-quantised Linear in the model's own basis, with the STE graph:
     the stored values, then the rotation of the flagged groups and the division by the
-    smoothing vector, fused."""
-    w = stored(fq, True)
+    smoothing vector, fused with the decode."""
     if not fq.has_had and not fq.has_scale:
-        return w
-    return _Transform.apply(w, fq.had, fq.col_scale if fq.has_scale else fq.col_scale[:0])
+        return stored(fq, True)
+    meta, params = _groups(fq)
+    scale = fq.col_scale if fq.has_scale else fq.col_scale[:0]
+    if torch.is_grad_enabled():
+        return _Weights.apply(fq.latent, fq.unit, meta, fq.had, scale, *params)
+    return _values(fq, meta, params, fq.had, scale)
 
 
 def stored(fq, grad: bool) -> torch.Tensor:
     """The stored-basis weights of a fake-quantised Linear (rows in the tensor's own order),
     with the STE graph when ``grad``."""
-    meta = [(g.rows, g.consts, g.nbits, g.block) for g in fq.groups]
-    params = [p for g in fq.groups for p in (g.lo_u, g.step_u)]
-    latent = fq.latent
+    meta, params = _groups(fq)
     if grad and torch.is_grad_enabled():
-        return _StoredDecode.apply(latent, fq.unit, meta, *params)
-    with torch.no_grad():
-        out = torch.empty_like(latent)
-        mod = _mod()
-        for (rows, consts, nbits, block), lo_u, st_u in zip(meta, params[::2], params[1::2]):
-            mod.decode_fwd(latent.detach(), fq.unit, lo_u.detach(), st_u.detach(), consts, rows,
-                           block, float(2 ** nbits - 1), out)
-        return out
+        return _StoredDecode.apply(fq.latent, fq.unit, meta, *params)
+    return _values(fq, meta, params, None, None)

@@ -475,6 +475,34 @@ int hi2x_qad_decode_bwd(const float* grad, const float* latent, const float* uni
                         int block, float nmax, float* g_latent, float* g_lo, float* g_st,
                         void* stream);
 
+/* One group of rows of a fake-quantised tensor: the arguments of hi2x_qad_decode_fwd / _bwd that
+ * differ between groups (g_lo and g_st for the backward only). */
+typedef struct hi2x_qad_group {
+  const float* lo_u;
+  const float* st_u;
+  const uint16_t* consts;
+  const int64_t* rows;
+  int64_t n_rows;
+  int32_t block;
+  float nmax;
+  float* g_lo;
+  float* g_st;
+} hi2x_qad_group;
+
+/* hi2x_qad_decode_fwd / _bwd of every group of a tensor in turn (groups: a host array), with
+ * flags [k / 16] u8 together with the transform of hi2x_qad_wht_scale in the same pass, for
+ * hi2.qad_kernel.original (hi2/qad_kernel.py:321-348): the decoded values go through
+ * H16(.) / scale on the flagged groups before they are written (scale [k] fp16 or NULL); the
+ * backward takes the gradient of that result, G = H16(grad / scale) being formed in registers.
+ * Bit for bit the separate entries one after the other; flags NULL: the decode alone. */
+int hi2x_qad_weights_fwd(const float* latent, const float* unit, const hi2x_qad_group* groups,
+                         int64_t n_groups, int64_t r_total, int64_t k, const uint8_t* flags,
+                         const uint16_t* scale, float* out, void* stream);
+int hi2x_qad_weights_bwd(const float* grad, const float* latent, const float* unit,
+                         const hi2x_qad_group* groups, int64_t n_groups, int64_t r_total,
+                         int64_t k, const uint8_t* flags, const uint16_t* scale,
+                         float* g_latent, void* stream);
+
 /* wht_scale (hi2/qad_kernel.py:165-189, Python side hi2/qad_kernel.py:321-336): out =
  * H16(x) / scale over the flagged 16-column groups (x / scale elsewhere), or with pre_div
  * H16(x / scale); H16 the normalised order-16 Walsh-Hadamard butterfly.  x/out [n_rows, k]
