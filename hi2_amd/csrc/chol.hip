@@ -34,6 +34,25 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_u16(const uint16_t* base,
                                            0x00020000);
 }
 
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2v __attribute__((ext_vector_type(2)));
+
+// Three bf16 planes of a pair of values, x1 = bf16(x), x2 = bf16(x - x1), x3 = bf16(x - x1 - x2)
+// (the differences are exact in fp32; bf16 has fp32's exponent range, so no scale is needed):
+// v_cvt_pk_bf16_f32 makes a plane of the pair, and a bf16 back to fp32 is its bits in the upper
+// half.
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t (&o)[3]) {
+#pragma unroll
+  for (int pl = 0; pl < 3; ++pl) {
+    o[pl] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2v){a, b}, bf16x2));
+    if (pl < 2) {
+      a = a - __builtin_bit_cast(float, o[pl] << 16);
+      b = b - __builtin_bit_cast(float, o[pl] & 0xffff0000u);
+    }
+  }
+}
+
 // ---- triangular GEMM ----------------------------------------------------------------
 // C[M, N] = alpha * A[M, Kd] * op(B) + beta * C (beta 0 or 1).
 // AMODE 1: A lower triangular.  BMODE 1 / 2: op(B) lower / upper triangular.
@@ -75,9 +94,185 @@ __host__ __device__ inline void tri_krange(int64_t r0, int64_t c0, int64_t T, in
   if (BMODE == 2) kend = (c0 + T < kend) ? c0 + T : kend;
 }
 
+// ---- 64-tiles of the deep recursion levels on bf16 planes ----------------------------------
+// A chunk of 32 ranks is split into its three bf16 planes as it goes from registers to LDS
+// (each element once per tile), and the tile runs six of the nine plane products on the bf16
+// MFMA, small ones first: 384 cycles of the matrix core per chunk and wave where the fp32 MFMA
+// takes 1024.  fp32-level rounding.  These products are a few workgroups whose operands other
+// XCDs have just written: four chunks are in flight in registers (one in flight cost 3-4 % of
+// a whole factor).  Measured against the fp32 MFMA tiles: a rank-256 product of one round of
+// tiles 15-18 -> 10 us, a K=4096 factor 1777 -> 1692 us, 32 experts of K=1024 697 -> 656 us;
+// factor error against 64 bits 4.2e-6 (fp32: 4.8e-6) at K=4096, 2.1e-6 (3.6e-6) at K=1024.
+// What is left at 10 us is the launch, the chunks' load latency and the strided C.
+constexpr int TS_D = 4;    // chunks in flight
+constexpr int TS_P = 40;   // LDS pitch of a plane's row (32 k; 16-byte reads on distinct banks)
+struct TriSplitSmem {
+  uint16_t A[2][3][64][TS_P];
+  uint16_t B[2][3][64][TS_P];
+};
+typedef uint16_t TriPlanes[3][64][TS_P];
+
+// Row-major X[r][k] as rows of the tile: thread (row tid / 4, 8 consecutive k).
+template <class Mask>
+struct SplitRows {
+  const float* p;
+  int64_t ld, nrows, kend;
+  Mask mask;
+  __device__ __forceinline__ void load(int64_t r0, int64_t k0, int tid, f32x4 (&st)[2],
+                                       bool live) const {
+    const int64_t rows = (nrows - r0 < 64) ? nrows - r0 : 64;
+    const __amdgpu_buffer_rsrc_t rs = mg_rsrc(p + r0 * ld + k0, (rows - 1) * ld + kend - k0);
+    const int rr = tid >> 2;
+    const uint32_t off = live && rr < rows ? (uint32_t)((rr * ld + 8 * (tid & 3)) * 4) : MG_OOB;
+#pragma unroll
+    for (int v = 0; v < 2; ++v) st[v] = mg_load4(rs, off + 16 * v);
+  }
+  // elements at k >= kend of rows before the last are real memory of the next columns
+  __device__ __forceinline__ void store(TriPlanes& S, int64_t r0, int64_t k0, int tid,
+                                        const f32x4 (&st)[2]) const {
+    const int m = tid >> 2, h = tid & 3;
+    const int64_t kb = k0 + 8 * h;
+    const bool edge = Mask::kElem || k0 + MG_KC > kend;
+    uint32_t w[3][4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float x[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int j = 2 * e + i;
+        const bool keep = !edge || (kb + j < kend && mask.elem(r0 + m, kb + j));
+        x[i] = keep ? st[j >> 2][j & 3] : 0.0f;
+      }
+      uint32_t o[3];
+      split_pair(x[0], x[1], o);
+#pragma unroll
+      for (int pl = 0; pl < 3; ++pl) w[pl][e] = o[pl];
+    }
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl)
+      *reinterpret_cast<uint4*>(&S[pl][m][8 * h]) = make_uint4(w[pl][0], w[pl][1], w[pl][2], w[pl][3]);
+  }
+};
+
+// Row-major X[k][c] as the B operand of a plain product: thread (k pair tid % 16, 4 columns).
+template <class Mask>
+struct SplitCols {
+  const float* p;
+  int64_t ld, ncols, kend;
+  Mask mask;
+  __device__ __forceinline__ void load(int64_t c0, int64_t k0, int tid, f32x4 (&st)[2],
+                                       bool live) const {
+    const int64_t kv = (kend - k0 < MG_KC) ? kend - k0 : MG_KC;
+    const __amdgpu_buffer_rsrc_t rs = mg_rsrc(p + k0 * ld + c0, (kv - 1) * ld + (ncols - c0));
+    const int kk = 2 * (tid & 15), cb = 4 * (tid >> 4);
+#pragma unroll
+    for (int v = 0; v < 2; ++v)
+      st[v] = mg_load4(rs, live && kk + v < kv ? (uint32_t)(((kk + v) * ld + cb) * 4) : MG_OOB);
+  }
+  __device__ __forceinline__ void store(TriPlanes& S, int64_t c0, int64_t k0, int tid,
+                                        const f32x4 (&st)[2]) const {
+    const int kk = 2 * (tid & 15), cb = 4 * (tid >> 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bool k0ok = !Mask::kElem || mask.elem(k0 + kk, c0 + cb + e);
+      const bool k1ok = !Mask::kElem || mask.elem(k0 + kk + 1, c0 + cb + e);
+      uint32_t o[3];
+      split_pair(k0ok ? st[0][e] : 0.0f, k1ok ? st[1][e] : 0.0f, o);
+#pragma unroll
+      for (int pl = 0; pl < 3; ++pl) *reinterpret_cast<uint32_t*>(&S[pl][cb + e][kk]) = o[pl];
+    }
+  }
+};
+
+// acc += A[r0:r0+64, kbeg:kend] * op(B)[kbeg:kend, c0:c0+64], one 32 x 32 accumulator per wave.
+// Every chunk issues the same loads (past the end they read nothing).
+template <class AL, class BL>
+__device__ __forceinline__ void tri_split_mainloop(f32x16& acc, TriSplitSmem& sm, const AL& al,
+                                                   const BL& bl, int64_t r0, int64_t c0,
+                                                   int64_t kbeg, int64_t kend) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (kend <= kbeg) return;
+  const int nch = (int)((kend - kbeg + MG_KC - 1) / MG_KC);
+  f32x4 sa[TS_D][2], sb[TS_D][2];
+  auto load = [&](int ch, f32x4(&a)[2], f32x4(&b)[2]) {
+    const bool live = ch < nch;
+    const int64_t k = kbeg + (int64_t)(live ? ch : 0) * MG_KC;
+    al.load(r0, k, tid, a, live);
+    bl.load(c0, k, tid, b, live);
+  };
+#pragma unroll
+  for (int d = 0; d < TS_D; ++d) load(d, sa[d], sb[d]);
+  __syncthreads();  // the previous use of the LDS buffers is over
+  al.store(sm.A[0], r0, kbeg, tid, sa[0]);
+  bl.store(sm.B[0], c0, kbeg, tid, sb[0]);
+  __syncthreads();
+  const int ra = (wave >> 1) * 32 + (lane & 31), rb = (wave & 1) * 32 + (lane & 31);
+  const int kh = 8 * (lane >> 5);
+  constexpr int PA[6] = {2, 0, 1, 1, 0, 0}, PB[6] = {0, 2, 1, 0, 1, 0};
+  f32x16 acc2;  // the second k-step's chain
+#pragma unroll
+  for (int j = 0; j < 16; ++j) acc2[j] = 0.0f;
+  for (int c4 = 0; c4 < nch; c4 += TS_D) {
+#pragma unroll
+    for (int d = 0; d < TS_D; ++d) {
+      const int ch = c4 + d;
+      if (ch >= nch) break;
+      load(ch + TS_D, sa[d], sb[d]);
+      bf16x8 a[2][3], b[2][3];
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int pl = 0; pl < 3; ++pl) {
+          a[ks][pl] = *reinterpret_cast<const bf16x8*>(&sm.A[d & 1][pl][ra][16 * ks + kh]);
+          b[ks][pl] = *reinterpret_cast<const bf16x8*>(&sm.B[d & 1][pl][rb][16 * ks + kh]);
+        }
+#pragma unroll
+      for (int t = 0; t < 6; ++t) {
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][PA[t]], b[0][PB[t]], acc, 0, 0, 0);
+        acc2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1][PA[t]], b[1][PB[t]], acc2, 0, 0, 0);
+      }
+      if (ch + 1 < nch) {  // the other buffer was last read before the previous barrier
+        const int64_t kn = kbeg + (int64_t)(ch + 1) * MG_KC;
+        al.store(sm.A[(d + 1) & 1], r0, kn, tid, sa[(d + 1) % TS_D]);
+        bl.store(sm.B[(d + 1) & 1], c0, kn, tid, sb[(d + 1) % TS_D]);
+      }
+      __syncthreads();
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 16; ++j) acc[j] = acc[j] + acc2[j];
+}
+
+// LDS of an output tile, and its product: bf16 planes for 64-tiles (SPLIT), else fp32 MFMA.
+template <int T, bool SPLIT>
+struct TriTile {
+  using Smem = MgSmemT<T>;
+  template <class M> using Rows = RowsLoader<M, T>;
+  template <class M> using Cols = ColsLoader<M, T>;
+  template <int NA, class AL, class BL>
+  static __device__ __forceinline__ void run(f32x16 (&acc)[NA][NA], Smem& sm, const AL& al,
+                                             const BL& bl, int64_t r0, int64_t c0, int64_t kbeg,
+                                             int64_t kend) {
+    mg_mainloop<NA, T>(acc, sm, al, bl, r0, c0, kbeg, kend);
+  }
+};
+template <>
+struct TriTile<64, true> {
+  using Smem = TriSplitSmem;
+  template <class M> using Rows = SplitRows<M>;
+  template <class M> using Cols = SplitCols<M>;
+  template <int NA, class AL, class BL>
+  static __device__ __forceinline__ void run(f32x16 (&acc)[NA][NA], Smem& sm, const AL& al,
+                                             const BL& bl, int64_t r0, int64_t c0, int64_t kbeg,
+                                             int64_t kend) {
+    tri_split_mainloop(acc[0][0], sm, al, bl, r0, c0, kbeg, kend);
+  }
+};
+
 // One output tile of the product (workgroup bid of the launch's tile mapping).
-template <int AMODE, int BMODE, bool TB, bool CLOW, int T>
-__device__ __forceinline__ void tri_gemm_tile(const GemmArgs& g0, MgSmemT<T>& sm, int64_t tm,
+template <int AMODE, int BMODE, bool TB, bool CLOW, int T, bool SPLIT>
+__device__ __forceinline__ void tri_gemm_tile(const GemmArgs& g0,
+                                              typename TriTile<T, SPLIT>::Smem& sm, int64_t tm,
                                               int64_t tn, int super, const MgSched& sched,
                                               int64_t bid) {
   constexpr int NA = T / 64;
@@ -103,19 +298,20 @@ __device__ __forceinline__ void tri_gemm_tile(const GemmArgs& g0, MgSmemT<T>& sm
   f32x16 acc[NA][NA];
   mg_zero<NA>(acc);
   using AMask = typename std::conditional<AMODE == 1, MaskLower, NoMask>::type;
-  RowsLoader<AMask, T> al{g.A, g.lda, g.M, kend, AMask{}};
+  using Tile = TriTile<T, SPLIT>;
+  typename Tile::template Rows<AMask> al{g.A, g.lda, g.M, kend, AMask{}};
   if (TB) {
     // op(B)[k][j] = B[j][k]: lower op(B) keeps k >= j, upper keeps k <= j
     using BMask = typename std::conditional<
         BMODE == 1, MaskUpper, typename std::conditional<BMODE == 2, MaskLower, NoMask>::type>::type;
-    RowsLoader<BMask, T> bl{g.B, g.ldb, g.N, kend, BMask{}};
-    mg_mainloop<NA, T>(acc, sm, al, bl, r0, c0, kbeg, kend);
+    typename Tile::template Rows<BMask> bl{g.B, g.ldb, g.N, kend, BMask{}};
+    Tile::template run<NA>(acc, sm, al, bl, r0, c0, kbeg, kend);
   } else {
     // op(B)[k][c] = B[k][c]: lower keeps c <= k (mask(k, c)), upper keeps c >= k
     using BMask = typename std::conditional<
         BMODE == 1, MaskLower, typename std::conditional<BMODE == 2, MaskUpper, NoMask>::type>::type;
-    ColsLoader<BMask, T> bl{g.B, g.ldb, g.N, kend, BMask{}};
-    mg_mainloop<NA, T>(acc, sm, al, bl, r0, c0, kbeg, kend);
+    typename Tile::template Cols<BMask> bl{g.B, g.ldb, g.N, kend, BMask{}};
+    Tile::template run<NA>(acc, sm, al, bl, r0, c0, kbeg, kend);
   }
   const CTile<T> ct(g.C, g.ldc, g.M, g.N, r0, c0);
   f32x16 cv[NA][NA];
@@ -140,27 +336,27 @@ __device__ __forceinline__ void tri_gemm_tile(const GemmArgs& g0, MgSmemT<T>& sm
   });
 }
 
-template <int AMODE, int BMODE, bool TB, bool CLOW, int T>
+template <int AMODE, int BMODE, bool TB, bool CLOW, int T, bool SPLIT>
 __global__ __launch_bounds__(256) void tri_gemm_kernel(GemmArgs g0, int64_t tm, int64_t tn,
                                                        int super, MgSched sched) {
-  __shared__ MgSmemT<T> sm;
-  tri_gemm_tile<AMODE, BMODE, TB, CLOW, T>(g0, sm, tm, tn, super, sched, blockIdx.x);
+  __shared__ typename TriTile<T, SPLIT>::Smem sm;
+  tri_gemm_tile<AMODE, BMODE, TB, CLOW, T, SPLIT>(g0, sm, tm, tn, super, sched, blockIdx.x);
 }
 
 // Two independent small products in one launch (64-tiles, xcd-spread tiles): workgroups
 // [0, grid1) run the first, the rest the second.  The recursion pairs A22 -= T1 T1^T with
 // T2 = T1 A11, which needs the same inputs and none of the other's output.
-template <int A1, int B1, bool TB1, bool C1, int A2, int B2, bool TB2, bool C2>
+template <int A1, int B1, bool TB1, bool C1, int A2, int B2, bool TB2, bool C2, bool SPLIT>
 __global__ __launch_bounds__(256) void tri_gemm_pair_kernel(GemmArgs g1, int64_t tm1,
                                                             int64_t tn1, int64_t grid1,
                                                             GemmArgs g2, int64_t tm2,
                                                             int64_t tn2) {
-  __shared__ MgSmemT<64> sm;
+  __shared__ typename TriTile<64, SPLIT>::Smem sm;
   const int64_t bid = blockIdx.x;
   if (bid < grid1)
-    tri_gemm_tile<A1, B1, TB1, C1, 64>(g1, sm, tm1, tn1, 0, MgSched{}, bid);
+    tri_gemm_tile<A1, B1, TB1, C1, 64, SPLIT>(g1, sm, tm1, tn1, 0, MgSched{}, bid);
   else
-    tri_gemm_tile<A2, B2, TB2, C2, 64>(g2, sm, tm2, tn2, 0, MgSched{}, bid - grid1);
+    tri_gemm_tile<A2, B2, TB2, C2, 64, SPLIT>(g2, sm, tm2, tn2, 0, MgSched{}, bid - grid1);
 }
 
 // ---- products of the big levels on fp16 MFMA through a scaled two-way split ----------
@@ -1016,15 +1212,20 @@ int gemm3x(const G3Args& a, hipStream_t s, int batch) {
 }
 
 // A22 -= T1 T1^T (lower) and T2 = T1 A11 in one launch, on 64-tiles (pair_small).
+static bool chol_split();
 int tri_gemm_pair(GemmArgs a1, GemmArgs a2, hipStream_t s, int batch) {
   const int64_t tm1 = (a1.M + 63) / 64, tn1 = (a1.N + 63) / 64;
   const int64_t tm2 = (a2.M + 63) / 64, tn2 = (a2.N + 63) / 64;
   const int64_t grid1 = (tm1 * tn1 + 7) / 8 * 8, grid2 = (tm2 * tn2 + 7) / 8 * 8;
   LaunchTimer timer(HI2X_TIME_CHOL_GEMM,
                     ((double)a1.M * a1.N * a1.Kd + (double)a2.M * a2.N * a2.Kd) * batch, s);
-  hipLaunchKernelGGL((tri_gemm_pair_kernel<0, 0, true, true, 0, 1, false, false>),
-                     dim3((unsigned)(grid1 + grid2), 1, (unsigned)batch), dim3(256), 0, s, a1,
-                     tm1, tn1, grid1, a2, tm2, tn2);
+  const dim3 grid((unsigned)(grid1 + grid2), 1, (unsigned)batch);
+  if (chol_split())
+    hipLaunchKernelGGL((tri_gemm_pair_kernel<0, 0, true, true, 0, 1, false, false, true>), grid,
+                       dim3(256), 0, s, a1, tm1, tn1, grid1, a2, tm2, tn2);
+  else
+    hipLaunchKernelGGL((tri_gemm_pair_kernel<0, 0, true, true, 0, 1, false, false, false>), grid,
+                       dim3(256), 0, s, a1, tm1, tn1, grid1, a2, tm2, tn2);
   return launch_status("tri_gemm_pair_kernel");
 }
 
@@ -1124,9 +1325,13 @@ int tri_gemm(const GemmArgs& a, hipStream_t s, int batch = 1) {
     // a small grid: 64-tiles, four times the workgroups for a quarter of the work each
     const int64_t tm6 = (a.M + 63) / 64, tn6 = (a.N + 63) / 64;
     const int64_t grid = (tm6 * tn6 + 7) / 8 * 8;
-    hipLaunchKernelGGL((tri_gemm_kernel<AMODE, BMODE, TB, CLOW, 64>),
-                       dim3((unsigned)grid, 1, (unsigned)batch), dim3(256), 0, s, a, tm6, tn6, 0,
-                       MgSched{});
+    const dim3 g((unsigned)grid, 1, (unsigned)batch);
+    if (chol_split())
+      hipLaunchKernelGGL((tri_gemm_kernel<AMODE, BMODE, TB, CLOW, 64, true>), g, dim3(256), 0, s, a,
+                         tm6, tn6, 0, MgSched{});
+    else
+      hipLaunchKernelGGL((tri_gemm_kernel<AMODE, BMODE, TB, CLOW, 64, false>), g, dim3(256), 0, s,
+                         a, tm6, tn6, 0, MgSched{});
     return launch_status("tri_gemm_kernel");
   }
   // big grids (several rounds of the 512 workgroup slots): super-tiles balanced over the
@@ -1150,7 +1355,7 @@ int tri_gemm(const GemmArgs& a, hipStream_t s, int batch = 1) {
   const int64_t grid = sched.per_xcd > 0 ? mg_sched_grid(sched)
                        : super            ? mg_super_grid(tm, tn, CLOW)
                                           : (ntiles + 7) / 8 * 8;
-  hipLaunchKernelGGL((tri_gemm_kernel<AMODE, BMODE, TB, CLOW, MG_T>),
+  hipLaunchKernelGGL((tri_gemm_kernel<AMODE, BMODE, TB, CLOW, MG_T, false>),
                      dim3((unsigned)grid, 1, (unsigned)batch), dim3(256), 0, s, a, tm, tn, super,
                      sched);
   return launch_status("tri_gemm_kernel");
@@ -1437,26 +1642,11 @@ __device__ __forceinline__ f32x4v tile_mma(const f32x4v& a, const f32x4v& b) {
   return p;
 }
 
-// Three bf16 planes of four values, x1 = bf16(x), x2 = bf16(x - x1), x3 = bf16(x - x1 - x2)
-// (the differences are exact in fp32; bf16 has fp32's exponent range, so no scale is needed).
-// Pairs go through v_cvt_pk_bf16_f32; a bf16 back to fp32 is its bits in the upper half.
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2v __attribute__((ext_vector_type(2)));
+// The planes of four values, two pairs each.
 __device__ __forceinline__ void split4(const f32x4v& x, uint2 (&o)[3]) {
   uint32_t u[2][3];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    float a = x[2 * h], b = x[2 * h + 1];
-#pragma unroll
-    for (int pl = 0; pl < 3; ++pl) {
-      u[h][pl] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2v){a, b}, bf16x2));
-      if (pl < 2) {
-        a = a - __builtin_bit_cast(float, u[h][pl] << 16);
-        b = b - __builtin_bit_cast(float, u[h][pl] & 0xffff0000u);
-      }
-    }
-  }
+  for (int h = 0; h < 2; ++h) split_pair(x[2 * h], x[2 * h + 1], u[h]);
 #pragma unroll
   for (int pl = 0; pl < 3; ++pl) o[pl] = make_uint2(u[0][pl], u[1][pl]);
 }

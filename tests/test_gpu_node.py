@@ -1,14 +1,15 @@
 """The factor of one recursion node (``node_kernel``, up to 256 columns in one workgroup) on
 the MI355X against float64: sizes at the edges of its 16-column tiles and 128-column halves,
-several matrices per launch, and pivots that fail in either half."""
+several matrices per launch, and pivots that fail in either half; and the products that join two
+nodes and more, at ranks and widths that end inside a 64-tile and a 32-rank chunk."""
 
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
-# one workgroup (<= 256 columns) and the smallest sizes of two
-SIZES = [4, 12, 16, 20, 60, 124, 128, 132, 240, 252, 256, 260, 388]
+# one workgroup (<= 256 columns), the smallest sizes of two, and several joined by products
+SIZES = [4, 12, 16, 20, 60, 124, 128, 132, 240, 252, 256, 260, 388, 516, 772, 1020, 1156]
 
 
 def _hessian(k, dev, seed):
