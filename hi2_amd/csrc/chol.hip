@@ -1681,14 +1681,6 @@ __device__ __forceinline__ void sub_comp(f32x4v& d, f32x4v& dc, const f32x4v& q)
   d = t;
 }
 
-// A workgroup barrier that orders LDS accesses only: __syncthreads() would also wait for the
-// wave's stores of finished blocks to reach memory, about a microsecond each time.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 struct NodeSmem {
   uint4 A[ND_N][64];   // planes 2 and 1 of P_j of the current block column
   uint2 A3[ND_N][64];  // its plane 3

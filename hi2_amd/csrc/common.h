@@ -117,6 +117,14 @@ __device__ __forceinline__ float f16_from_bits(uint16_t b) {
 
 #include "divrcp.h"
 
+// A workgroup barrier that orders LDS accesses only: __syncthreads() would also wait for the
+// wave's stores of finished blocks to reach memory, about a microsecond each time.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // torch.clamp(q, 0, n - 1): NaN propagates through both compares.
 __device__ __forceinline__ float clamp_code(float q, float nm) {
   q = (q < 0.0f) ? 0.0f : q;

@@ -3,6 +3,8 @@
 // Reference: hi2/encode.py:18-119 (EFFORT, _recon, _lsq, fit_ladder, quantize_params),
 // hi2/ladder_kernel.py:44-86 (the grid search), hi2/format.py:45-69 (decode_params,
 // ladder_dequantize), hi2/hessian.py:318-345 (_finish).
+#include <algorithm>
+
 #include "common.h"
 
 namespace hi2x {
@@ -450,6 +452,77 @@ __global__ void unpermute_kernel(const uint8_t* __restrict__ codes_ro, const flo
   if (comp && comp_ro) comp[r * k + c] = comp_ro[i];
 }
 
+// The same, a row at a time through LDS, for rows that fit there and that 16-byte accesses can
+// move: scattered stores of one element each, and 8 bytes of perm read for every 5 moved, held
+// the kernel above at 1.0 TB/s; here only LDS is written out of order, perm is read once per
+// workgroup (16-bit copies in LDS), and the next row's loads are in flight while this one is
+// turned.  The whole finish (its sse included) of 9216 x 2560: 327 -> 75 us with comp,
+// 83 -> 38 without; of 4096 x 14336 with comp 922 -> 189.  One row of 4096 to 16384 columns
+// takes as long either way (15-16 us, 43-46 us), so the row count does not choose.
+constexpr int UP_NV = 4;  // float4 of comp a thread: rows of up to 16 T columns
+template <int T>
+__global__ __launch_bounds__(T) void unpermute_rows_kernel(
+    const uint8_t* __restrict__ codes_ro, const float* __restrict__ comp_ro,
+    const int64_t* __restrict__ perm, int64_t n, int k, uint8_t* __restrict__ codes,
+    float* __restrict__ comp) {
+  // up to 56 KB as the launch asks for, so that short rows share a CU; 112 KB declared
+  extern __shared__ __align__(16) uint8_t up_dyn[];
+  __shared__ __align__(16) uint8_t up_static[T > 512 ? 7 * 4 * UP_NV * T : 16];
+  uint8_t* up_smem = T > 512 ? up_static : up_dyn;
+  float* f = reinterpret_cast<float*>(up_smem);  // k floats
+  uint16_t* p = reinterpret_cast<uint16_t*>(f + k);
+  uint8_t* c = reinterpret_cast<uint8_t*>(p + k);
+  const int t = threadIdx.x;
+  for (int j = t; j < k; j += T) p[j] = (uint16_t)perm[j];
+  uint32_t vc[UP_NV];
+  float4 vf[UP_NV];
+  auto load = [&](int64_t r) {
+    const uint32_t* cr = reinterpret_cast<const uint32_t*>(codes_ro + r * k);
+    const float4* fr = reinterpret_cast<const float4*>(comp_ro + r * k);
+#pragma unroll
+    for (int q = 0; q < UP_NV; ++q) {
+      const int j = t + q * T;
+      if (j * 4 < k) {
+        vc[q] = cr[j];
+        if (comp) vf[q] = fr[j];
+      }
+    }
+  };
+  int64_t r = blockIdx.x;
+  if (r < n) load(r);
+  for (; r < n; r += gridDim.x) {
+    __syncthreads();  // perm is there; the row before has been read
+#pragma unroll
+    for (int q = 0; q < UP_NV; ++q) {
+      const int j = t + q * T;
+      if (j * 4 < k) {
+        const uint2 pp = reinterpret_cast<const uint2*>(p)[j];
+        const uint32_t i0 = pp.x & 0xffffu, i1 = pp.x >> 16, i2 = pp.y & 0xffffu, i3 = pp.y >> 16;
+        c[i0] = (uint8_t)vc[q];
+        c[i1] = (uint8_t)(vc[q] >> 8);
+        c[i2] = (uint8_t)(vc[q] >> 16);
+        c[i3] = (uint8_t)(vc[q] >> 24);
+        if (comp) {
+          f[i0] = vf[q].x;
+          f[i1] = vf[q].y;
+          f[i2] = vf[q].z;
+          f[i3] = vf[q].w;
+        }
+      }
+    }
+    if (r + gridDim.x < n) load(r + gridDim.x);
+    lds_barrier();
+#pragma unroll
+    for (int q = 0; q < UP_NV; ++q) {
+      const int j = t + q * T;
+      if (j * 4 < k) {
+        reinterpret_cast<uint32_t*>(codes + r * k)[j] = reinterpret_cast<uint32_t*>(c)[j];
+        if (comp) reinterpret_cast<float4*>(comp + r * k)[j] = reinterpret_cast<float4*>(f)[j];
+      }
+    }
+  }
+}
+
 // sse[r] = sum_c d_c (fp16(lo + code*step) - w)^2 in torch's CPU sum order for a
 // contiguous row of k floats: 8 vector lanes x 4 vector accumulators, the 4-level
 // cascade over rows of 32 floats (base 2^max(4, ceil_log2(rows)/4)), the extra vectors
@@ -729,8 +802,21 @@ extern "C" int hi2x_finish(const uint8_t* codes_ro, const float* comp_ro, const 
                     (double)n * k * (5 + (moves ? 2 + (comp ? 8 : 0) : 0)), s);
   // without a permutation the outputs may alias the inputs: nothing to move then
   if (!(perm == nullptr && codes == codes_ro && comp == comp_ro)) {
-    hipLaunchKernelGGL(unpermute_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
-                       codes_ro, comp_ro, perm, n, k, codes, comp);
+    float* const cm = comp_ro ? comp : nullptr;
+    // rows that 4-byte (codes) and 16-byte (comp) accesses can move and that fit the LDS
+    if (perm && k % 4 == 0 && k <= 16 * 1024 && (((uintptr_t)codes_ro | (uintptr_t)codes) & 3) == 0 &&
+        (!cm || (((uintptr_t)comp_ro | (uintptr_t)cm) & 15) == 0)) {
+      if (k <= 16 * 512)
+        hipLaunchKernelGGL(unpermute_rows_kernel<512>, dim3((unsigned)std::min<int64_t>(n, 1024)),
+                           dim3(512), (unsigned)(k * 7), s, codes_ro, comp_ro, perm, n, (int)k,
+                           codes, cm);
+      else
+        hipLaunchKernelGGL(unpermute_rows_kernel<1024>, dim3((unsigned)std::min<int64_t>(n, 256)),
+                           dim3(1024), 0, s, codes_ro, comp_ro, perm, n, (int)k, codes, cm);
+    } else {
+      hipLaunchKernelGGL(unpermute_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
+                         codes_ro, comp_ro, perm, n, k, codes, comp);
+    }
     const int rc = launch_status("unpermute_kernel");
     if (rc) return rc;
   }
