@@ -98,7 +98,8 @@ class HessianStats:
             raise RuntimeError(
                 f"hi2_amd.HessianStats accumulates on the MI355X; got device {dev}"
             )
-        self._dev = dev
+        # the device current now, wherever the first update runs
+        self._dev = torch.device("cuda", torch.cuda.current_device()) if dev.index is None else dev
         self._sum: torch.Tensor | None = None  # made by the first update (or read as zeros)
         self._upper_only = False
         self.n = 0
@@ -141,13 +142,15 @@ class HessianStats:
         if t:
             first = self._sum is None  # nothing to add to: neither cleared nor read
             if first:
-                self._sum = torch.empty(self.k, self.k, dtype=torch.float32, device=dev)
-            elif self._sum.dtype != torch.float32 or not self._sum.is_contiguous():
-                self._S = self.S.to(torch.float32).contiguous()
-            s = self._sum
+                s = torch.empty(self.k, self.k, dtype=torch.float32, device=dev)
+            else:
+                if self._sum.dtype != torch.float32 or not self._sum.is_contiguous():
+                    self._S = self.S.to(torch.float32).contiguous()
+                s = self._sum
             ws = _lib.workspace(dev, "hi2x_hessian_accumulate_workspace_bytes", dtype, t, self.k)
             _lib.call("hi2x_hessian_accumulate", dev, _lib.ptr(x), dtype, t, self.k, _lib.ptr(s),
                       int(first), _lib.ptr(ws), ws.numel())
+            self._sum = s  # a first update that raised leaves the sum unmade
             self._upper_only = True
         self.n += t
 

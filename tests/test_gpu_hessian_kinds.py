@@ -100,3 +100,25 @@ def test_sum_without_an_update_is_zero(dev):
     assert st.n == 0 and not bool(st.S.any())
     had = torch.ones(3, dtype=torch.uint8, device=dev)
     assert not bool(HessianStats(48, dev).transformed(None, had).any())
+
+
+def test_first_update_that_raises_leaves_the_sum_unmade(dev, monkeypatch):
+    """A caller that catches the error and updates again adds to zero, not to unset memory."""
+    from hi2_amd import _lib
+    from hi2_amd.hessian import HessianStats
+
+    x = _x(64, 48, torch.float32, dev, 5)
+    want = HessianStats(48, dev)
+    want.update(x)
+    st = HessianStats(48, "cuda")
+
+    def fail(*a):
+        raise RuntimeError("no workspace")
+
+    with monkeypatch.context() as m:
+        m.setattr(_lib, "workspace", fail)
+        with pytest.raises(RuntimeError):
+            st.update(x)
+    assert st.n == 0 and not st._upper_only and st._sum is None
+    st.update(x)
+    assert torch.equal(st.S, want.S)
