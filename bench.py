@@ -775,7 +775,7 @@ class StageTimer:
 # kernel families timed by the library (hi2x_timing_*), with the peak that bounds each
 KERNELS = {  # kind -> (kernel, bound, peak FLOP/s, work unit)
     0: ("gptq_trailing_kernel", "mfma", PEAK_F32, "2*rows*rank*cols"),
-    1: ("syrk2_bf16_kernel", "mfma", PEAK_BF16, "T*K*(K+1) (upper triangle, 2 flops per product)"),
+    1: ("syrk2_kernel", "mfma", PEAK_BF16, "T*K*(K+1) (upper triangle, 2 flops per product)"),
     2: ("tri_gemm_kernel", "mfma", PEAK_F32, "M*N*rank (one triangular operand; the "
         "factor's fp32 MFMA products)"),
     11: ("gemm3_kernel/gemm3x_kernel (split planes)", "mfma", PEAK_BF16,

@@ -1304,8 +1304,9 @@ int g3_pair(const G3Args& a1, const G3Args& a2, hipStream_t s, int batch) {
   }
 }
 
-// Products of the big grids: fp16 MFMA on the two scaled split planes (default), or the
-// fp32 MFMA GEMM when HI2X_CHOL_FP32 is set to a nonzero value (read once per process).
+// Products of the big grids: fp16 MFMA on the two scaled split planes (default); of the small
+// ones: bf16 MFMA on three planes.  HI2X_CHOL_FP32 set to a nonzero value runs all of them on
+// the fp32 MFMA (read once per process).
 static bool chol_split() {
   static const bool split = [] {
     const char* e = getenv("HI2X_CHOL_FP32");
