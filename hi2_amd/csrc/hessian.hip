@@ -55,9 +55,10 @@ __device__ __forceinline__ void store_sym(float* __restrict__ s, int64_t K, int6
 // either are exact in fp32; K=2560, 3 x 1777 fp16 tokens 197 us with the transform, 1715 us
 // converted to fp32 and multiplied on the fp32 MFMA), and
 // fp32 tokens as three bf16 planes x1 = bf16(x), x2 = bf16(x - x1), x3 = bf16(x - x1 - x2)
-// (the differences are exact in fp32, so the planes hold x to 2^-24 of itself whatever the
-// other tokens are), six of the nine plane products on the bf16 MFMA, small ones first: 96
-// cycles of the matrix core per 16 tokens of a 32 x 32 tile where the fp32 MFMA takes 512.
+// (the differences are exact in fp32, and from 2^-110 up the planes are all of x, whatever the
+// other tokens are; PLANE_MIN and PLANE_MAX below), six of the nine plane products on the bf16
+// MFMA, small ones first: 96 cycles of the matrix core per 16 tokens of a 32 x 32 tile where the
+// fp32 MFMA takes 512.
 // K=4096, 2 x 2048 fp32 tokens: 558 us with the transform, 2750 us on the fp32 MFMA (263
 // against 1250 us a batch); error against float64 2.6e-7 and 7.3e-7.
 // X [T, K] is first transposed once (one HBM pass) so that every MFMA operand (8
@@ -192,10 +193,19 @@ __global__ __launch_bounds__(256) void transpose8_bf16_kernel(const uint16_t* __
   }
 }
 
+// What the planes' products need of a value that is not zero, as bits of its magnitude.  From
+// 2^-110 up its last bit is at least 2^-133, the least bf16, so the third plane holds what the
+// first two leave; below, bits are lost (up to 4 units of 2^-24 at 2^-112).
+// Below 2^53 no sum of plane products over a call's tokens (fewer than 2^21) reaches the largest
+// fp32; above, products and sums of one sign may pass it where the rest would bring them back
+// (1e22 is 1.0035e22 - 3.5e19 - 9e15: its square is inf, and the planes' inf - inf).
+constexpr uint32_t PLANE_MIN = 0x08800000u;  // 2^-110
+constexpr uint32_t PLANE_MAX = 0x5a000000u;  // 2^53
+
 // The three bf16 planes of f32 X [T, K], transposed: row k of xt [K, 3 Tp] is plane 1, 2, 3 of
-// feature k, zeros from T on.  One pass: 4 bytes read and 6 written per element.  A value whose
-// first plane would round to infinity (or is not finite) sets *bad, and the caller's products
-// run on the fp32 MFMA instead.  VEC: K a multiple of 4 and x 16-byte aligned.
+// feature k, zeros from T on.  One pass: 4 bytes read and 6 written per element.  A value outside
+// the range above (or not finite) sets *bad, and the caller's products run on the fp32 MFMA
+// instead.  VEC: K a multiple of 4 and x 16-byte aligned.
 template <bool VEC>
 __global__ __launch_bounds__(256) void transpose_planes_kernel(const float* __restrict__ x,
                                                                int64_t T, int64_t K, int64_t Tp,
@@ -205,10 +215,10 @@ __global__ __launch_bounds__(256) void transpose_planes_kernel(const float* __re
   const int64_t t0 = (int64_t)blockIdx.y * 64, k0 = (int64_t)blockIdx.x * 64;
   const int tid = threadIdx.x;
   bool wide = false;
-  // the largest fp32 magnitude that rounds to a finite bf16 is below 0x7f7f8000
   auto put = [&](int r, int c, float v) {
     tile[r][c] = v;
-    wide = wide || (__float_as_uint(v) & 0x7fffffffu) >= 0x7f7f8000u;
+    const uint32_t a = __float_as_uint(v) & 0x7fffffffu;
+    wide = wide || (a != 0 && a - PLANE_MIN >= PLANE_MAX - PLANE_MIN);
   };
   if constexpr (VEC) {
 #pragma unroll

@@ -279,7 +279,7 @@ int64_t hi2x_hessian_accumulate_workspace_bytes(int dtype, int64_t t, int64_t k)
  * 2 = bf16 (at most 4M f16 rows per call).  first != 0 takes s as zero instead of reading
  * it.  f16 and bf16 products are exact on their own MFMA with f32 accumulation; f32 rows run as
  * three bf16 planes each (fp32-level rounding, also element by element), or on the f32 MFMA
- * where a value is not finite or within half a bf16 step of the largest fp32. */
+ * where a value is not zero and not in [2^-110, 2^53) in magnitude (infinities and NaN too). */
 int hi2x_hessian_accumulate(const void* x, int dtype, int64_t t, int64_t k, float* s, int first,
                             void* ws, int64_t ws_bytes, void* stream);
 

@@ -57,7 +57,7 @@ def test_fp32_elements_keep_their_own_precision(dev):
 @pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.4e38])
 @pytest.mark.parametrize("first", [True, False])
 def test_fp32_values_beyond_the_planes(value, first, dev):
-    """Infinities, NaN and the largest fp32 values give what fp32 products and sums give."""
+    """Infinities, NaN and the largest fp32 values, first and later updates."""
     from hi2_amd.hessian import HessianStats
 
     t, k = 96, 300
@@ -74,6 +74,55 @@ def test_fp32_values_beyond_the_planes(value, first, dev):
     assert torch.equal(torch.isnan(s), torch.isnan(want))
     assert torch.equal(s[torch.isinf(want)], want[torch.isinf(want)])
     assert torch.allclose(s[fin], want[fin], rtol=1e-4, atol=1e-4 * 400 * t)
+
+
+def _fp32_kernel(x, dev):
+    """Both triangles of ``x^T x`` on the fp32 MFMA (the C entry without a workspace)."""
+    from hi2_amd import _lib
+
+    s = torch.zeros(x.shape[1], x.shape[1], device=dev)
+    _lib.call("hi2x_hessian_syrk", x.device, _lib.ptr(x), 0, x.shape[0], x.shape[1], _lib.ptr(s),
+              None, 0)
+    return s
+
+
+# squares that pass the largest fp32 (their planes' products of unlike sign too), and magnitudes
+# whose planes cannot hold them; alone and beside their negative, K for both load widths
+@pytest.mark.parametrize("value", [2.0 ** 53, 1e20, 1.5e21, 1e22, 7e25, 3e30, 2.0 ** -111, 1e-36,
+                                   1e-40])
+@pytest.mark.parametrize("pair", [False, True])
+@pytest.mark.parametrize("k", [300, 301])
+def test_fp32_values_outside_the_planes_range(value, pair, k, dev):
+    """They give the bits of fp32 products and sums."""
+    from hi2_amd.hessian import HessianStats
+
+    x = _x(96, k, torch.float32, dev, 12)
+    x[5, 7] = value
+    if pair:
+        x[9, 20] = x[9, 7] = -value
+    st = HessianStats(k, dev)
+    print(f"outside the planes {value} k={k}", flush=True)
+    st.update(x)
+    want = _fp32_kernel(x, dev)
+    nan = torch.isnan(want)
+    assert torch.equal(torch.isnan(st.S), nan)
+    assert torch.equal(st.S[~nan], want[~nan])
+
+
+@pytest.mark.parametrize("value", [2.0 ** -110 * (1 + 2.0 ** -23), 1.7e-30, 2.0 ** 53 * (1 - 2.0 ** -24)])
+def test_fp32_values_at_the_ends_of_the_planes_range(value, dev):
+    """A feature of such magnitudes only, against float64: the bound of the other magnitudes."""
+    from hi2_amd.hessian import HessianStats
+
+    t, k = 96, 64
+    x = _x(t, k, torch.float32, dev, 13)
+    x[:, 3] = value * (1 + 2.0 ** -12) ** torch.arange(t, device=dev) if value < 1 else value
+    st = HessianStats(k, dev)
+    st.update(x)
+    xd = x.double()
+    ok = (st.S.double() - xd.T @ xd).abs() <= (t + 4) * 2.0 ** -24 * (xd.abs().T @ xd.abs())
+    ok[3, 3] |= value ** 2 < 2.0 ** -126  # the square of the feature is below the normal fp32
+    assert bool(ok.all())
 
 
 def test_fp16_specials(dev):
