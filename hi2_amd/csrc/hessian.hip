@@ -196,7 +196,7 @@ __global__ __launch_bounds__(256) void transpose8_bf16_kernel(const uint16_t* __
 // What the planes' products need of a value that is not zero, as bits of its magnitude.  From
 // 2^-110 up its last bit is at least 2^-133, the least bf16, so the third plane holds what the
 // first two leave; below, bits are lost (up to 4 units of 2^-24 at 2^-112).
-// Below 2^53 no sum of plane products over a call's tokens (fewer than 2^21) reaches the largest
+// Below 2^53 no sum of plane products over a pass's tokens (at most 2^18) reaches the largest
 // fp32; above, products and sums of one sign may pass it where the rest would bring them back
 // (1e22 is 1.0035e22 - 3.5e19 - 9e15: its square is inf, and the planes' inf - inf).
 constexpr uint32_t PLANE_MIN = 0x08800000u;  // 2^-110
@@ -1258,9 +1258,35 @@ int launch_syrk(const void* x, int dtype, int64_t t, int64_t k, float* s, char* 
   return !rc && mirror ? launch_mirror(s, k, st) : rc;
 }
 
-// fp32 tokens run as planes unless a 256-feature panel of them would pass 32-bit offsets (1.4 M
-// tokens in one call).
-bool f32_planes(int64_t t, int64_t k) { return (t + 63) / 64 * 64 * 3 <= (int64_t(1) << 22); }
+// Tokens of one pass (a multiple of 64): fp32 calls run in passes whose planes take at most
+// 512 MiB, each added to S in turn: 16384 tokens at K=14336 take 18.8 ms in three passes (23.2
+// in one), 65536 at K=4096 9.4 (8.9), 2^20 at K=256 2.1 (2.6).  2^18 tokens keep a 256-feature panel of three planes below
+// the 2^31 bytes of a buffer's offsets.
+int64_t syrk_pass(int kind, int64_t t, int64_t k) {
+  if (kind != SYRK_PLANES) return t;
+  const int64_t most =
+      std::min<int64_t>(int64_t(1) << 18, std::max<int64_t>(64, (int64_t(512) << 20) / (6 * k) / 64 * 64));
+  const int64_t passes = (t + most - 1) / most;
+  return passes <= 1 ? t : ((t + passes - 1) / passes + 63) / 64 * 64;
+}
+
+size_t syrk_bytes(int kind, int64_t t, int64_t k) {
+  if (t == 0) return 0;
+  const int64_t per = syrk_pass(kind, t, k), last = t - (t - 1) / per * per;
+  return std::max(syrk_plan(kind, per, k).total(), syrk_plan(kind, last, k).total());
+}
+
+// S += X^T X (first: S = X^T X) over t > 0 tokens, upper triangle, in passes; ws of syrk_bytes.
+template <int KIND>
+int launch_passes(const void* x, int64_t t, int64_t k, float* s, int first, char* ws,
+                  hipStream_t st) {
+  const int64_t per = syrk_pass(KIND, t, k), row = k * (KIND == SYRK_PLANES ? 4 : 2);
+  int rc = HI2X_OK;
+  for (int64_t t0 = 0; t0 < t && !rc; t0 += per)
+    rc = launch_syrk16<KIND>(static_cast<const char*>(x) + t0 * row, std::min(per, t - t0), k, s,
+                             first != 0 && t0 == 0, ws, st);
+  return rc;
+}
 
 // Workspace of the grouped accumulation: xt [k, cap] bf16 (cap = tokens + 64 per group,
 // the windows' worst case) and the plan tables.
@@ -1323,8 +1349,7 @@ extern "C" int hi2x_hessian_syrk_upper(const void* x, int dtype, int64_t t, int6
 
 extern "C" int64_t hi2x_hessian_accumulate_workspace_bytes(int dtype, int64_t t, int64_t k) {
   if (dtype < 0 || dtype > 2 || k <= 0 || t < 0) return -1;
-  if (dtype == 0) return f32_planes(t, k) ? (int64_t)syrk_plan(SYRK_PLANES, t, k).total() : 0;
-  return (int64_t)syrk_plan(SYRK_BF16, t, k).total();
+  return (int64_t)syrk_bytes(dtype == 0 ? SYRK_PLANES : SYRK_BF16, t, k);
 }
 
 extern "C" int hi2x_hessian_accumulate(const void* x, int dtype, int64_t t, int64_t k, float* s,
@@ -1341,11 +1366,9 @@ extern "C" int hi2x_hessian_accumulate(const void* x, int dtype, int64_t t, int6
                                 (size_t)hi2x_hessian_accumulate_workspace_bytes(dtype, t, k), st,
                                 "hessian_accumulate");
   if (rc) return rc;
-  if (dtype == 2) return launch_syrk16<SYRK_BF16>(x, t, k, s, first, w.p, st);
-  if (dtype == 1) return launch_syrk16<SYRK_F16>(x, t, k, s, first, w.p, st);
-  if (f32_planes(t, k)) return launch_syrk16<SYRK_PLANES>(x, t, k, s, first, w.p, st);
-  LaunchTimer timer(HI2X_TIME_HESSIAN_SYRK, (double)t * k * (k + 1), st);
-  return launch_syrk_f32((const float*)x, t, k, s, first, nullptr, st);
+  if (dtype == 2) return launch_passes<SYRK_BF16>(x, t, k, s, first, w.p, st);
+  if (dtype == 1) return launch_passes<SYRK_F16>(x, t, k, s, first, w.p, st);
+  return launch_passes<SYRK_PLANES>(x, t, k, s, first, w.p, st);
 }
 
 extern "C" int hi2x_hessian_mirror(float* s, int64_t k, void* stream) {

@@ -129,7 +129,9 @@ class HessianStats:
     @torch.no_grad()
     def update(self, x: torch.Tensor, chunk: int = 4096) -> None:
         """``S += x^T x`` over all rows of ``x[..., K]`` (``chunk`` is accepted for
-        interface compatibility; the kernel streams the rows itself)."""
+        interface compatibility).  Scratch: a transposed copy of 16-bit rows, 2 bytes an
+        element; at most 512 MiB of planes for fp32 rows, which run in passes; and partial
+        sums where the tiles of ``S`` are few."""
         x = x.reshape(-1, self.k)
         dev = self._dev if self._sum is None else self._sum.device
         t = x.shape[0]

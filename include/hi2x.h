@@ -271,7 +271,8 @@ int hi2x_hessian_syrk(const void* x, int dtype, int64_t t, int64_t k, float* s, 
 int hi2x_hessian_syrk_upper(const void* x, int dtype, int64_t t, int64_t k, float* s,
                             void* ws, int64_t ws_bytes, void* stream);
 
-/* Workspace of hi2x_hessian_accumulate for t rows of width k. */
+/* Workspace of hi2x_hessian_accumulate for t rows of width k: the transposed copy, three bf16
+ * planes for f32 rows, which run in passes that hold those to 512 MiB; and partial sums. */
 int64_t hi2x_hessian_accumulate_workspace_bytes(int dtype, int64_t t, int64_t k);
 
 /* HessianStats.update (hi2/hessian.py:35-40) on the upper triangle (i <= j) of s, the lower one

@@ -125,6 +125,34 @@ def test_fp32_values_at_the_ends_of_the_planes_range(value, dev):
     assert bool(ok.all())
 
 
+def _integers(t, k, dtype, dev, seed):
+    """Tokens whose sums of products are whole numbers below 2^24 for up to 2^22 / 2 tokens."""
+    g = torch.Generator(device=dev).manual_seed(seed)
+    return torch.randint(-2, 3, (t, k), generator=g, device=dev).to(dtype)
+
+
+@pytest.mark.parametrize("t,k", [(1 << 18, 16), ((1 << 18) + 1, 260), ((1 << 19) + 70, 37)])
+@pytest.mark.parametrize("outside", [False, True])
+def test_fp32_passes(t, k, outside, dev):
+    """More tokens than one pass's planes hold: exact sums, first and later update, also where a
+    value outside the planes' range sends one of the passes to the fp32 kernel."""
+    from hi2_amd.hessian import HessianStats
+
+    x = _integers(t, k, torch.float32, dev, t + k)
+    if outside:
+        x[t - 3, 2] = 2.0 ** 60  # its own row and column of the sum are not compared
+    st = HessianStats(k, dev)
+    print(f"fp32 passes t={t} k={k}", flush=True)
+    st.update(x)
+    st.update(x[:70])
+    xd = x.double()
+    want = xd.T @ xd + xd[:70].T @ xd[:70]
+    keep = torch.ones(k, dtype=torch.bool, device=dev)
+    keep[2] = not outside
+    assert torch.equal(st.S.double()[keep][:, keep], want[keep][:, keep])
+    assert st.n == t + 70
+
+
 def test_fp16_specials(dev):
     """fp16 infinities, NaN and subnormals multiply as their fp32 values do."""
     from hi2_amd.hessian import HessianStats
