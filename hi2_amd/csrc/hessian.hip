@@ -1246,26 +1246,14 @@ int launch_syrk16(const void* x, int64_t t, int64_t k, float* s, int first, char
   return rc;
 }
 
-// The accumulations without a choice of workspace: bf16 through the transposed copy, f32 on
-// the fp32 MFMA (no workspace; both triangles).
-int launch_syrk(const void* x, int dtype, int64_t t, int64_t k, float* s, char* ws,
-                hipStream_t st, bool mirror = true) {
-  if (dtype != 2) {
-    LaunchTimer timer(HI2X_TIME_HESSIAN_SYRK, (double)t * k * (k + 1), st);  // upper triangle
-    return launch_syrk_f32((const float*)x, t, k, s, 0, nullptr, st);
-  }
-  const int rc = launch_syrk16<SYRK_BF16>(x, t, k, s, 0, ws, st);
-  return !rc && mirror ? launch_mirror(s, k, st) : rc;
-}
-
-// Tokens of one pass (a multiple of 64): fp32 calls run in passes whose planes take at most
-// 512 MiB, each added to S in turn: 16384 tokens at K=14336 take 18.8 ms in three passes (23.2
-// in one), 65536 at K=4096 9.4 (8.9), 2^20 at K=256 2.1 (2.6).  2^18 tokens keep a 256-feature panel of three planes below
-// the 2^31 bytes of a buffer's offsets.
+// Tokens of one pass (a multiple of 64).  A 256-feature panel of a pass stays below the 2^31 bytes
+// of a buffer's offsets: 2^21 tokens of 16 bits, 2^18 of three planes.  fp32 calls run in passes
+// whose planes take at most 512 MiB, each added to S in turn: 16384 tokens at K=14336 take
+// 18.8 ms in three passes (23.2 in one), 65536 at K=4096 9.4 (8.9), 2^20 at K=256 2.1 (2.6).
 int64_t syrk_pass(int kind, int64_t t, int64_t k) {
-  if (kind != SYRK_PLANES) return t;
-  const int64_t most =
+  const int64_t planes =
       std::min<int64_t>(int64_t(1) << 18, std::max<int64_t>(64, (int64_t(512) << 20) / (6 * k) / 64 * 64));
+  const int64_t most = kind == SYRK_PLANES ? planes : int64_t(1) << 21;
   const int64_t passes = (t + most - 1) / most;
   return passes <= 1 ? t : ((t + passes - 1) / passes + 63) / 64 * 64;
 }
@@ -1286,6 +1274,18 @@ int launch_passes(const void* x, int64_t t, int64_t k, float* s, int first, char
     rc = launch_syrk16<KIND>(static_cast<const char*>(x) + t0 * row, std::min(per, t - t0), k, s,
                              first != 0 && t0 == 0, ws, st);
   return rc;
+}
+
+// The accumulations without a choice of workspace: bf16 through the transposed copy, f32 on
+// the fp32 MFMA (no workspace; both triangles).
+int launch_syrk(const void* x, int dtype, int64_t t, int64_t k, float* s, char* ws,
+                hipStream_t st, bool mirror = true) {
+  if (dtype != 2) {
+    LaunchTimer timer(HI2X_TIME_HESSIAN_SYRK, (double)t * k * (k + 1), st);  // upper triangle
+    return launch_syrk_f32((const float*)x, t, k, s, 0, nullptr, st);
+  }
+  const int rc = launch_passes<SYRK_BF16>(x, t, k, s, 0, ws, st);
+  return !rc && mirror ? launch_mirror(s, k, st) : rc;
 }
 
 // Workspace of the grouped accumulation: xt [k, cap] bf16 (cap = tokens + 64 per group,
@@ -1313,7 +1313,7 @@ using namespace hi2x;
 
 extern "C" int64_t hi2x_hessian_workspace_bytes(int dtype, int64_t t, int64_t k) {
   if ((dtype != 0 && dtype != 2) || k <= 0 || t < 0) return -1;
-  return dtype == 2 ? (int64_t)syrk_plan(SYRK_BF16, t, k).total() : 0;
+  return dtype == 2 ? (int64_t)syrk_bytes(SYRK_BF16, t, k) : 0;
 }
 
 extern "C" int hi2x_hessian_syrk(const void* x, int dtype, int64_t t, int64_t k, float* s,
@@ -1325,7 +1325,7 @@ extern "C" int hi2x_hessian_syrk(const void* x, int dtype, int64_t t, int64_t k,
   hipStream_t st = as_stream(stream);
   Workspace w;
   const int rc = take_workspace(w, ws, ws_bytes,
-                                dtype == 2 ? syrk_plan(SYRK_BF16, t, k).total() : 0, st,
+                                dtype == 2 ? syrk_bytes(SYRK_BF16, t, k) : 0, st,
                                 "hessian_syrk");
   if (rc) return rc;
   return launch_syrk(x, dtype, t, k, s, w.p, st);
@@ -1341,7 +1341,7 @@ extern "C" int hi2x_hessian_syrk_upper(const void* x, int dtype, int64_t t, int6
   hipStream_t st = as_stream(stream);
   Workspace w;
   const int rc = take_workspace(w, ws, ws_bytes,
-                                dtype == 2 ? syrk_plan(SYRK_BF16, t, k).total() : 0, st,
+                                dtype == 2 ? syrk_bytes(SYRK_BF16, t, k) : 0, st,
                                 "hessian_syrk_upper");
   if (rc) return rc;
   return launch_syrk(x, dtype, t, k, s, w.p, st, false);
@@ -1358,8 +1358,6 @@ extern "C" int hi2x_hessian_accumulate(const void* x, int dtype, int64_t t, int6
   HI2X_REQUIRE(dtype >= 0 && dtype <= 2, "hessian_accumulate: dtype %d (0 = f32, 1 = f16, 2 = bf16)",
                dtype);
   HI2X_REQUIRE(k > 0 && t > 0 && x && s, "hessian_accumulate: bad arguments");
-  HI2X_REQUIRE(dtype != 1 || t <= (int64_t(1) << 22), "hessian_accumulate: %lld f16 tokens exceed 4M",
-               (long long)t);
   hipStream_t st = as_stream(stream);
   Workspace w;
   const int rc = take_workspace(w, ws, ws_bytes,

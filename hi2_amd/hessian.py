@@ -130,14 +130,12 @@ class HessianStats:
     def update(self, x: torch.Tensor, chunk: int = 4096) -> None:
         """``S += x^T x`` over all rows of ``x[..., K]`` (``chunk`` is accepted for
         interface compatibility).  Scratch: a transposed copy of 16-bit rows, 2 bytes an
-        element; at most 512 MiB of planes for fp32 rows, which run in passes; and partial
-        sums where the tiles of ``S`` are few."""
+        element and 2M rows at a time; at most 512 MiB of planes for fp32 rows, which run in
+        passes too; and partial sums where the tiles of ``S`` are few."""
         x = x.reshape(-1, self.k)
         dev = self._dev if self._sum is None else self._sum.device
         t = x.shape[0]
         dtype = _SYRK_DTYPE.get(x.dtype, 0)
-        if dtype == 1 and t > 1 << 22:
-            dtype = 0
         if not dtype and x.dtype != torch.float32:
             x = x.to(torch.float32)
         x = x.to(dev).contiguous()

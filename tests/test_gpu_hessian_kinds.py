@@ -153,6 +153,30 @@ def test_fp32_passes(t, k, outside, dev):
     assert st.n == t + 70
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("t,k", [((1 << 21) + 1, 24), ((1 << 23) + 70, 16)])
+def test_16_bit_passes(t, k, dtype, dev):
+    """More tokens than a pass takes (2^23 rows of a 256-feature panel no longer fit 32-bit
+    offsets): exact sums, through ``HessianStats`` and for bf16 through the other entries."""
+    from hi2_amd import _lib
+    from hi2_amd.hessian import HessianStats
+
+    g = torch.Generator(device=dev).manual_seed(k)
+    x = torch.randint(-1, 2, (t, k), generator=g, device=dev, dtype=torch.int8).to(dtype)
+    st = HessianStats(k, dev)
+    print(f"16-bit passes {dtype} t={t} k={k}", flush=True)
+    st.update(x)
+    want = sum(c.double().T @ c.double() for c in x.split(1 << 20))
+    assert torch.equal(st.S.double(), want)
+    if dtype == torch.bfloat16:
+        ws = _lib.workspace(dev, "hi2x_hessian_workspace_bytes", 2, t, k)
+        assert ws.numel() < 2 * k * (1 << 22)  # one pass of the copy, and partial sums
+        for name in ("hi2x_hessian_syrk", "hi2x_hessian_syrk_upper"):
+            s = torch.zeros(k, k, device=dev)
+            _lib.call(name, x.device, _lib.ptr(x), 2, t, k, _lib.ptr(s), _lib.ptr(ws), ws.numel())
+            assert torch.equal(s.double().triu(), want.triu())
+
+
 def test_fp16_specials(dev):
     """fp16 infinities, NaN and subnormals multiply as their fp32 values do."""
     from hi2_amd.hessian import HessianStats
