@@ -749,9 +749,9 @@ __global__ __launch_bounds__(256) void mirror_kernel(float* __restrict__ s, int6
   }
 }
 
-// f32 X [T, K] on v_mfma_f32_32x32x2_f32, 128 x 128 tiles: for callers without a workspace and
-// for tokens that the bf16 planes cannot hold (only: when not null, the launch does nothing
-// unless the word there is nonzero).  Writes both triangles; first: S is taken as zero.
+// f32 X [T, K] on v_mfma_f32_32x32x2_f32, 128 x 128 tiles: for callers without a workspace, for
+// few tokens (f32_few) and for tokens that the bf16 planes cannot hold (only: when not null, the
+// launch does nothing unless the word there is nonzero).  Writes both triangles; first: S is taken as zero.
 __global__ __launch_bounds__(256) void syrk_f32_kernel(const float* __restrict__ x, int64_t T,
                                                        int64_t K, int nT, float* __restrict__ s,
                                                        int first,
@@ -1156,6 +1156,11 @@ SyrkPlan syrk_plan(int kind, int64_t t, int64_t k) {
       if (c < cost - 1e-9) cost = c, best = sp;
     }
   }
+  // few fp16 or fp32 tokens: writing and summing partials takes longer than the workgroups that
+  // they occupy save (K = 2048: 64 fp16 tokens 28 us split, 20 whole; 160 fp32 tokens 58 and
+  // 45; K = 6144: 128 fp32 tokens 209 and 86; from 256 fp32 tokens at K = 1536 on, splits win:
+  // 54 and 55).  bf16 sums keep their order.
+  if (kind != SYRK_BF16 && t <= std::min<int64_t>(192, 13 * p.ntiles)) best = 1;
   syrk_chunk(p.tv, best, p.tchunk, p.splits);
   p.parts_bytes = p.splits > 1 ? (size_t)p.splits * k * k * sizeof(float) : 0;
   return p;
@@ -1264,6 +1269,16 @@ size_t syrk_bytes(int kind, int64_t t, int64_t k) {
   return std::max(syrk_plan(kind, per, k).total(), syrk_plan(kind, last, k).total());
 }
 
+// fp32 tokens that go to the fp32 kernel, one launch, instead of the planes' five: up to 64
+// where its 128-tiles are at most 136 (K <= 2048: 20-32 us, the planes 27-33), fewer as the tiles
+// fill a round of the CUs (K = 2304: 50; 28 us at 32, the planes 33); past a round its tiles take
+// longer (K = 4096: 58 us and 37).  Up to three tokens at any K: a product of planes is rounded
+// up to six times where an fp32 product is rounded once, and sums of so few do not hide it.
+bool f32_few(int64_t t, int64_t k) {
+  const int64_t nT = (k + HT - 1) / HT, tiles = nT * (nT + 1) / 2;
+  return t <= 3 || (t <= 64 && tiles <= 256 && t * tiles <= 64 * 136);
+}
+
 // S += X^T X (first: S = X^T X) over t > 0 tokens, upper triangle, in passes; ws of syrk_bytes.
 template <int KIND>
 int launch_passes(const void* x, int64_t t, int64_t k, float* s, int first, char* ws,
@@ -1349,7 +1364,8 @@ extern "C" int hi2x_hessian_syrk_upper(const void* x, int dtype, int64_t t, int6
 
 extern "C" int64_t hi2x_hessian_accumulate_workspace_bytes(int dtype, int64_t t, int64_t k) {
   if (dtype < 0 || dtype > 2 || k <= 0 || t < 0) return -1;
-  return (int64_t)syrk_bytes(dtype == 0 ? SYRK_PLANES : SYRK_BF16, t, k);
+  if (dtype == 0) return f32_few(t, k) ? 0 : (int64_t)syrk_bytes(SYRK_PLANES, t, k);
+  return (int64_t)syrk_bytes(dtype == 1 ? SYRK_F16 : SYRK_BF16, t, k);
 }
 
 extern "C" int hi2x_hessian_accumulate(const void* x, int dtype, int64_t t, int64_t k, float* s,
@@ -1366,7 +1382,9 @@ extern "C" int hi2x_hessian_accumulate(const void* x, int dtype, int64_t t, int6
   if (rc) return rc;
   if (dtype == 2) return launch_passes<SYRK_BF16>(x, t, k, s, first, w.p, st);
   if (dtype == 1) return launch_passes<SYRK_F16>(x, t, k, s, first, w.p, st);
-  return launch_passes<SYRK_PLANES>(x, t, k, s, first, w.p, st);
+  if (!f32_few(t, k)) return launch_passes<SYRK_PLANES>(x, t, k, s, first, w.p, st);
+  LaunchTimer timer(HI2X_TIME_HESSIAN_SYRK, (double)t * k * (k + 1), st);
+  return launch_syrk_f32((const float*)x, t, k, s, first, nullptr, st);
 }
 
 extern "C" int hi2x_hessian_mirror(float* s, int64_t k, void* stream) {

@@ -85,7 +85,8 @@ _SYRK_DTYPE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 class HessianStats:
     """Full second moment ``sum x x^T`` of a Linear's input (fp32, ``[K, K]``) on a HIP
     device; ``update`` accumulates on MFMA (bf16 and fp16 inputs exactly, fp32 inputs as
-    three bf16 planes, other dtypes converted to fp32 first as the reference does).
+    three bf16 planes or, a few rows, on the fp32 MFMA, other dtypes converted to fp32 first as
+    the reference does).
 
     ``update`` brings only the upper triangle up to date; the lower one is mirrored when
     ``S`` is read (``S``, ``mean``, ``merge``), and ``transformed`` reads the upper

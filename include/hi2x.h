@@ -273,7 +273,7 @@ int hi2x_hessian_syrk_upper(const void* x, int dtype, int64_t t, int64_t k, floa
 
 /* Workspace of hi2x_hessian_accumulate for t rows of width k: the transposed copy of a pass over
  * the rows (16-bit rows: up to 2M rows a pass; f32 rows: up to 512 MiB of three bf16 planes) and
- * partial sums. */
+ * partial sums (few f32 rows: nothing). */
 int64_t hi2x_hessian_accumulate_workspace_bytes(int dtype, int64_t t, int64_t k);
 
 /* HessianStats.update (hi2/hessian.py:35-40) on the upper triangle (i <= j) of s, the lower one
@@ -281,7 +281,8 @@ int64_t hi2x_hessian_accumulate_workspace_bytes(int dtype, int64_t t, int64_t k)
  * 2 = bf16.  first != 0 takes s as zero instead of reading
  * it.  f16 and bf16 products are exact on their own MFMA with f32 accumulation; f32 rows run as
  * three bf16 planes each (fp32-level rounding, also element by element), or on the f32 MFMA
- * where a value is not zero and not in [2^-110, 2^53) in magnitude (infinities and NaN too). */
+ * where they are few (up to 64 rows, fewer from k = 2049 on) or a value is not zero and not in
+ * [2^-110, 2^53) in magnitude (infinities and NaN too). */
 int hi2x_hessian_accumulate(const void* x, int dtype, int64_t t, int64_t k, float* s, int first,
                             void* ws, int64_t ws_bytes, void* stream);
 

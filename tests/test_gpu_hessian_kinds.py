@@ -76,11 +76,12 @@ def test_fp32_values_beyond_the_planes(value, first, dev):
     assert torch.allclose(s[fin], want[fin], rtol=1e-4, atol=1e-4 * 400 * t)
 
 
-def _fp32_kernel(x, dev):
-    """Both triangles of ``x^T x`` on the fp32 MFMA (the C entry without a workspace)."""
+def _fp32_kernel(x, dev, s=None):
+    """Both triangles of ``x^T x`` (plus ``s``) on the fp32 MFMA (the C entry without a
+    workspace)."""
     from hi2_amd import _lib
 
-    s = torch.zeros(x.shape[1], x.shape[1], device=dev)
+    s = torch.zeros(x.shape[1], x.shape[1], device=dev) if s is None else s
     _lib.call("hi2x_hessian_syrk", x.device, _lib.ptr(x), 0, x.shape[0], x.shape[1], _lib.ptr(s),
               None, 0)
     return s
@@ -109,6 +110,54 @@ def test_fp32_values_outside_the_planes_range(value, pair, k, dev):
     assert torch.equal(st.S[~nan], want[~nan])
 
 
+def _integers(t, k, dtype, dev, seed):
+    """Tokens whose sums of products are whole numbers below 2^24 for up to 2^22 / 2 tokens."""
+    g = torch.Generator(device=dev).manual_seed(seed)
+    return torch.randint(-2, 3, (t, k), generator=g, device=dev).to(dtype)
+
+
+# both sides of each line of the rule, tiles of 128 that are whole and not
+@pytest.mark.parametrize("t,k,few", [(64, 48, True), (65, 48, False), (64, 2048, True),
+                                     (65, 2048, False), (56, 2049, True), (57, 2049, False),
+                                     (34, 2816, True), (4, 2817, False), (3, 2817, True),
+                                     (1, 4100, True), (4, 4100, False)])
+def test_few_fp32_tokens(t, k, few, dev):
+    """Few fp32 tokens run on the fp32 kernel, without scratch and with its bits, first and later
+    updates; past them, every element as the planes' bound has it."""
+    from hi2_amd import _lib
+    from hi2_amd.hessian import HessianStats
+
+    x = _x(t, k, torch.float32, dev, t + k)
+    f = _lib.lib().hi2x_hessian_accumulate_workspace_bytes
+    assert (f(0, t, k) == 0) == few
+    print(f"few fp32 tokens t={t} k={k}", flush=True)
+    st = HessianStats(k, dev)
+    st.update(x)
+    st.update(x[: t // 2])
+    if few:
+        assert torch.equal(st.S, _fp32_kernel(x[: t // 2], dev, _fp32_kernel(x, dev)))
+    x = torch.cat([x, x[: t // 2]]).double()
+    bound = (x.shape[0] + 4) * 2.0 ** -24
+    assert bool(((st.S.double() - x.T @ x).abs() <= bound * (x.abs().T @ x.abs())).all())
+
+
+@pytest.mark.parametrize("t", [13, 129, 192, 193])
+@pytest.mark.parametrize("k", [250, 1030, 1536])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_split_and_whole_token_ranges(t, k, dtype, dev):
+    """Either side of the line between one token range and several: whole numbers, so every
+    order of the sums is exact."""
+    from hi2_amd.hessian import HessianStats
+
+    x = _integers(t, k, dtype, dev, t + k)
+    st = HessianStats(k, dev)
+    print(f"token ranges {dtype} t={t} k={k}", flush=True)
+    st.update(x)
+    st.update(x)
+    xd = x.double()
+    assert torch.equal(st.S.double(), 2.0 * (xd.T @ xd))
+
+
 @pytest.mark.parametrize("value", [2.0 ** -110 * (1 + 2.0 ** -23), 1.7e-30, 2.0 ** 53 * (1 - 2.0 ** -24)])
 def test_fp32_values_at_the_ends_of_the_planes_range(value, dev):
     """A feature of such magnitudes only, against float64: the bound of the other magnitudes."""
@@ -123,12 +172,6 @@ def test_fp32_values_at_the_ends_of_the_planes_range(value, dev):
     ok = (st.S.double() - xd.T @ xd).abs() <= (t + 4) * 2.0 ** -24 * (xd.abs().T @ xd.abs())
     ok[3, 3] |= value ** 2 < 2.0 ** -126  # the square of the feature is below the normal fp32
     assert bool(ok.all())
-
-
-def _integers(t, k, dtype, dev, seed):
-    """Tokens whose sums of products are whole numbers below 2^24 for up to 2^22 / 2 tokens."""
-    g = torch.Generator(device=dev).manual_seed(seed)
-    return torch.randint(-2, 3, (t, k), generator=g, device=dev).to(dtype)
 
 
 @pytest.mark.parametrize("t,k", [(1 << 18, 16), ((1 << 18) + 1, 260), ((1 << 19) + 70, 37)])
