@@ -99,21 +99,22 @@ class HessianStats:
             raise RuntimeError(
                 f"hi2_amd.HessianStats accumulates on the MI355X; got device {dev}"
             )
-        # the device current now, wherever the first update runs
-        self._dev = torch.device("cuda", torch.cuda.current_device()) if dev.index is None else dev
-        self._sum: torch.Tensor | None = None  # made by the first update (or read as zeros)
+        # made now, so that a device or a lack of memory that refuses it does so here; written
+        # by the first update, or as zeros by a read before it
+        self._room: torch.Tensor | None = torch.empty(k, k, dtype=torch.float32, device=dev)
+        self._sum: torch.Tensor | None = None
         self._upper_only = False
         self.n = 0
 
     @property
     def _S(self) -> torch.Tensor:
         if self._sum is None:
-            self._sum = torch.zeros(self.k, self.k, dtype=torch.float32, device=self._dev)
+            self._S = self._room.zero_()
         return self._sum
 
     @_S.setter
     def _S(self, value: torch.Tensor) -> None:
-        self._sum = value
+        self._sum, self._room = value, None
 
     @property
     def S(self) -> torch.Tensor:
@@ -134,7 +135,7 @@ class HessianStats:
         element and 2M rows at a time; at most 512 MiB of planes for fp32 rows, which run in
         passes too; and partial sums where the tiles of ``S`` are few."""
         x = x.reshape(-1, self.k)
-        dev = self._dev if self._sum is None else self._sum.device
+        dev = (self._room if self._sum is None else self._sum).device
         t = x.shape[0]
         dtype = _SYRK_DTYPE.get(x.dtype, 0)
         if not dtype and x.dtype != torch.float32:
@@ -143,7 +144,7 @@ class HessianStats:
         if t:
             first = self._sum is None  # nothing to add to: neither cleared nor read
             if first:
-                s = torch.empty(self.k, self.k, dtype=torch.float32, device=dev)
+                s = self._room
             else:
                 if self._sum.dtype != torch.float32 or not self._sum.is_contiguous():
                     self._S = self.S.to(torch.float32).contiguous()
@@ -151,7 +152,7 @@ class HessianStats:
             ws = _lib.workspace(dev, "hi2x_hessian_accumulate_workspace_bytes", dtype, t, self.k)
             _lib.call("hi2x_hessian_accumulate", dev, _lib.ptr(x), dtype, t, self.k, _lib.ptr(s),
                       int(first), _lib.ptr(ws), ws.numel())
-            self._sum = s  # a first update that raised leaves the sum unmade
+            self._S = s  # a first update that raised leaves the sum unmade
             self._upper_only = True
         self.n += t
 

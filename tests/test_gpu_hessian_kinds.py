@@ -266,3 +266,17 @@ def test_first_update_that_raises_leaves_the_sum_unmade(dev, monkeypatch):
     assert st.n == 0 and not st._upper_only and st._sum is None
     st.update(x)
     assert torch.equal(st.S, want.S)
+
+
+def test_the_constructor_refuses(dev):
+    """A device that is not there and a sum that does not fit raise in the constructor."""
+    from hi2_amd.hessian import HessianStats
+
+    with pytest.raises(RuntimeError):
+        HessianStats(16, "cuda:99")
+    with pytest.raises(RuntimeError):
+        HessianStats(1 << 20, dev)  # 4 TiB
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    st = HessianStats(1024, dev)
+    assert torch.cuda.memory_allocated() - before >= 4 << 20 and not bool(st.S.any())
