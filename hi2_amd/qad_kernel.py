@@ -31,8 +31,13 @@ def _check(t: torch.Tensor, dtype: torch.dtype, name: str) -> None:
         raise RuntimeError(f"{name} must be contiguous {dtype}")
 
 
+def _full(t: torch.Tensor | None):
+    """None in the place of an empty tensor (an absent vector, on whatever device it is)."""
+    return None if t is None or t.numel() == 0 else t
+
+
 def _opt(t: torch.Tensor | None):
-    return None if t is None or t.numel() == 0 else _lib.ptr(t)
+    return _lib.ptr(_full(t))
 
 
 def _group_args(latent, unit, lo_u, st_u, consts, rows, block):
@@ -179,7 +184,7 @@ def _decode(latent, unit, meta, flags, scale, params, out) -> None:
         return
     tab = _group_table(latent, unit, meta, params)
     fl, sc = _transform_args(flags, scale, latent.shape[1])
-    _lib.call("hi2x_qad_weights_fwd", _lib.require_gpu(latent, out, flags, scale),
+    _lib.call("hi2x_qad_weights_fwd", _lib.require_gpu(latent, out, flags, _full(scale)),
               _lib.ptr(latent), _opt(unit), ctypes.cast(tab, ctypes.c_void_p), len(meta),
               latent.shape[0], latent.shape[1], fl, sc, _lib.ptr(out))
 
@@ -197,7 +202,7 @@ def _decode_grads(ctx, grad, flags, scale):
             raise RuntimeError("grad must have the latent's shape")
         tab = _group_table(latent, unit, ctx.meta, params, grads)
         fl, sc = _transform_args(flags, scale, latent.shape[1])
-        _lib.call("hi2x_qad_weights_bwd", _lib.require_gpu(grad, latent, flags, scale),
+        _lib.call("hi2x_qad_weights_bwd", _lib.require_gpu(grad, latent, flags, _full(scale)),
                   _lib.ptr(grad), _lib.ptr(latent), _opt(unit), ctypes.cast(tab, ctypes.c_void_p),
                   len(ctx.meta), latent.shape[0], latent.shape[1], fl, sc, _lib.ptr(g_latent))
     return g_latent, grads

@@ -56,3 +56,19 @@ def test_fused_equals_two_passes(n, k, unit, flags, scale, dev):
     assert all(torch.equal(x, y) for x, y in zip(a[1:], b[1:]))
     with torch.no_grad():
         assert torch.equal(original(fq)[rows], two[rows])
+
+
+def test_an_absent_smoothing_vector_may_be_anywhere(dev):
+    """Without smoothing, ``col_scale`` is not read and need not be on the device."""
+    from hi2_amd.qad_kernel import original
+
+    fq = _fq(7, 192, True, False, True, dev, 3)
+    rows = torch.cat([g.rows for g in fq.groups])
+    grad = torch.randn(7, 192, device=dev)
+    want = original(fq)
+    gw, = torch.autograd.grad(want, [fq.latent], grad)
+    for cs in (fq.col_scale.cpu(), torch.empty(0)):
+        fq.col_scale = cs
+        got = original(fq)
+        gg, = torch.autograd.grad(got, [fq.latent], grad)
+        assert torch.equal(got[rows], want[rows]) and torch.equal(gg[rows], gw[rows])
