@@ -1618,7 +1618,9 @@ __device__ __forceinline__ bool node_base(const f32x4v& d, f32x4v* xs, __amdgpu_
   base_steps(v, i, lg, pv, std::make_integer_sequence<int, 16>{});
   const bool bad = __builtin_amdgcn_ballot_w64(!(pv > 0.0f)) != 0;
   float r = __builtin_amdgcn_rsqf(pv);
-  r = __builtin_fmaf(0.5f * r, __builtin_fmaf(-pv * r, r, 1.0f), r);  // one Newton step
+  // one Newton step (an infinite pivot's r stays 0: a row of zeros, as 1 / sqrt gives it)
+  const float r1 = __builtin_fmaf(0.5f * r, __builtin_fmaf(-pv * r, r, 1.0f), r);
+  r = pv < __builtin_inff() ? r1 : r;
   // row i of L^-1: X[i][j] = M[i][j] r_i (j < i), X[i][i] = r_i, zeros above
   f32x4v x;
 #pragma unroll
@@ -1677,8 +1679,9 @@ __device__ __forceinline__ f32x4v plane_mma(const uint4& a, const uint2& a3, con
 // whole factor is as close to 64 bits as with one subtraction per 64 or 128 columns (K = 1024:
 // 3.6e-6 of U, 4.4e-6 without).
 __device__ __forceinline__ void sub_comp(f32x4v& d, f32x4v& dc, const f32x4v& q) {
-  const f32x4v y = -q - dc, t = d + y;
-  dc = (t - d) - y;
+  const f32x4v y = -q - dc, t = d + y, e = (t - d) - y;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) dc[j] = e[j] == e[j] ? e[j] : 0.0f;  // an infinite d stays one
   d = t;
 }
 

@@ -57,3 +57,15 @@ def test_node_reports_a_failing_pivot(at, dev):
     with pytest.raises(_lib.NotPositiveDefinite, match=f"block at {at // 128 * 128} "):
         _lib.call("hi2x_chol_inv_upper", h.device, _lib.ptr(h), k, 0.0, 0, _lib.ptr(u),
                   _lib.ptr(ws), ws.numel())
+
+
+@pytest.mark.parametrize("k", [16, 64, 260, 516])
+def test_an_overflowed_diagonal_gives_a_factor_of_zeros(k, dev):
+    """The damping is a share of the diagonal's mean: one infinite entry makes every pivot
+    infinite and its row 1 / sqrt of that."""
+    from hi2_amd.hessian import inverse_factor
+
+    h = _hessian(k, dev, 5).float()
+    h[k // 2, k // 2] = float("inf")
+    print(f"overflowed diagonal k={k}", flush=True)
+    assert not bool(inverse_factor(h, 0.01).any())
