@@ -587,7 +587,7 @@ typedef float f32x4g __attribute__((ext_vector_type(4)));
 // FULL: every block has LMAX columns (K a multiple of it).
 template <bool FULL, bool COMP, int SB>
 __global__ __launch_bounds__(RPG * QL, 1) void gptq_super_kernel(
-    const float* __restrict__ wc, int64_t N, int64_t K, int64_t i0, int nblk,
+    float* __restrict__ wc, int64_t N, int64_t K, int64_t i0, int nblk,
     float* __restrict__ err1, int64_t lde, uint8_t* __restrict__ codes,
     const float* __restrict__ lo, const float* __restrict__ st, int64_t ldp,
     const int32_t* __restrict__ row_grp, const int64_t* __restrict__ u_ptrs,
@@ -620,6 +620,13 @@ __global__ __launch_bounds__(RPG * QL, 1) void gptq_super_kernel(
     f32x4 uv[NV];
     float2 tv[4];  // working tile, C layout: rows 4 g4 + i, columns 32 wave + 2q, + 1
     const int tc = 32 * wave + 2 * q;
+    uint32_t own = 0;  // bit i: row 4 g4 + i is of this run
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int rr = 4 * g4 + i;
+      const int gi = row_grp[rbase + (rr < nrows ? rr : nrows - 1)];
+      own |= (rr < nrows && gi >= g && gi <= ge ? 1u : 0u) << i;
+    }
     // block b's U block, block map and working tile
     auto fetch = [&](int b) {
       const int64_t i1 = i0 + (int64_t)b * LMAX;
@@ -703,6 +710,17 @@ __global__ __launch_bounds__(RPG * QL, 1) void gptq_super_kernel(
       __syncthreads();
       load_tile_row<COMP>(R, wt + lr * WSTR, q);
       load_row_c<COMP>(R, L, su, q);
+      // the tile goes back to wc as the separate updates leave it (its stores and the next
+      // block's loads are in flight during the loop)
+      if (b > 0) {
+        const __amdgpu_buffer_rsrc_t wr = mg_rsrc(wc + rbase * K + i1, (int64_t)(nrows - 1) * K + L);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          __builtin_amdgcn_raw_buffer_store_b64(
+              __builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned, tv[i]), wr,
+              (int)(tc < L && (own >> i & 1) ? (uint32_t)(((int64_t)(4 * g4 + i) * K + tc) * 4)
+                                             : MG_OOB), 0, 0);
+      }
       if (b + 1 < nblk) fetch(b + 1);
       // the U panel of the next near update, rows of blocks 0 .. b, into this XCD's L2 while the
       // loop runs: each of its workgroups (blockIdx % 8) touches its share of the 128-byte lines
@@ -745,7 +763,7 @@ __global__ __launch_bounds__(RPG * QL, 1) void gptq_super_kernel(
   }
 }
 
-int launch_super(const float* wc, int64_t n, int64_t k, int64_t i0, int nblk, float* err1,
+int launch_super(float* wc, int64_t n, int64_t k, int64_t i0, int nblk, float* err1,
                  int64_t lde, uint8_t* codes, const float* lo, const float* st, int64_t ldp,
                  const int32_t* row_grp, const int64_t* u_ptrs, const int32_t* blk,
                  const float* nmax, float* comp, hipStream_t s) {

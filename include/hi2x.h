@@ -83,8 +83,8 @@ int hi2x_gptq_trailing(float* wc, int64_t n, int64_t k, int64_t i1, int64_t len,
  * of `super_blocks` consecutive blocks applied to the far columns in one pass
  * (each block's product still subtracted separately, in block order, so the result
  * is bit-identical to the per-block schedule).  Batches of up to 4096 rows run a
- * super-block of up to eight blocks as one launch.  wc is scratch: modified in place,
- * its contents afterwards unspecified.
+ * super-block of up to eight blocks as one launch.  wc is modified in place: every column
+ * holds afterwards what the blocks before its own left there.
  * err_ws: device workspace of n * 128 * super_blocks floats. */
 int hi2x_gptq_run(float* wc, int64_t n, int64_t k, uint8_t* codes, const float* lo,
                   const float* st, int64_t ldp, const int32_t* row_grp,

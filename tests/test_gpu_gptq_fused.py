@@ -72,6 +72,36 @@ def test_workgroups_of_two_factors(dev):
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
 
 
+@pytest.mark.parametrize("n,k,runs", [(1, 256, [1]), (17, 1088, [17]), (40, 640, [5, 14, 21]),
+                                      (64, 1168, [16, 48])])
+@pytest.mark.parametrize("sb", [4, 8])
+def test_working_copy_is_updated_in_place(n, k, runs, sb, dev):
+    """``hi2x_gptq_run`` leaves every column of ``wc`` with the updates of the blocks before its
+    own, whatever the schedule: the per-block one's bits."""
+    from hi2_amd import _lib
+
+    w, d, us = _inputs(n, k, dev, n + k, groups=2)
+    grp = torch.repeat_interleave(torch.arange(len(runs)), torch.tensor(runs)).int().to(dev)
+    ptrs = torch.tensor([us[i % 2].data_ptr() for i in range(len(runs))], dtype=torch.int64,
+                        device=dev)
+    blk = (torch.arange(k, device=dev, dtype=torch.int32) // 16).repeat(len(runs), 1).contiguous()
+    nmax = torch.full((len(runs),), 15.0, device=dev)
+    lo = w.reshape(n, -1, 16).amin(-1).half().float().contiguous()
+    st = ((w.reshape(n, -1, 16).amax(-1) - lo) / 15.0).half().float().contiguous()
+    out = []
+    for s in (1, sb):
+        wc, codes = w.clone(), torch.zeros(n, k, dtype=torch.uint8, device=dev)
+        ws = torch.empty(n, 128 * s, device=dev)
+        print(f"working copy n={n} k={k} sb={s}", flush=True)
+        _lib.call("hi2x_gptq_run", w.device, _lib.ptr(wc), n, k, _lib.ptr(codes), _lib.ptr(lo),
+                  _lib.ptr(st), k // 16, _lib.ptr(grp), _lib.ptr(ptrs), _lib.ptr(blk),
+                  _lib.ptr(nmax), None, _lib.ptr(ws), s)
+        out.append((wc, codes))
+    assert not torch.equal(out[0][0], w)
+    assert torch.equal(out[0][0].view(torch.int32), out[1][0].view(torch.int32))
+    assert torch.equal(out[0][1], out[1][1])
+
+
 @pytest.mark.parametrize("value", [0.0, -0.0, 1e-30, -1e-30, 3e20, float("inf"), float("nan")])
 def test_values_outside_the_fast_range(value, dev):
     from hi2_amd.hessian import GptqJob, encode_jobs_gptq
