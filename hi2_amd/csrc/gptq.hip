@@ -583,6 +583,7 @@ __global__ __launch_bounds__(256, T == MG_T ? 2 : 4) void gptq_trailing_kernel(
 constexpr int64_t FUSED_ROWS = 4096;
 constexpr int WSTR = LMAX + 4;  // LDS row stride of the working tile (floats)
 typedef float f32x4g __attribute__((ext_vector_type(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // wc is any float's address
 
 // FULL: every block has LMAX columns (K a multiple of it).
 template <bool FULL, bool COMP, int SB>
@@ -596,7 +597,7 @@ __global__ __launch_bounds__(RPG * QL, 1) void gptq_super_kernel(
   constexpr int ESTR = SB * LMAX + 4;
   __shared__ float su[LMAX * USTR];
   __shared__ float et[RPG * ESTR];
-  __shared__ float wt[RPG * WSTR];
+  __shared__ __attribute__((aligned(16))) float wt[RPG * WSTR];
   const int tid = threadIdx.x, lane = tid & 63, q = lane & (QL - 1), g4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t rbase = (int64_t)blockIdx.x * RPG;
@@ -620,13 +621,6 @@ __global__ __launch_bounds__(RPG * QL, 1) void gptq_super_kernel(
     f32x4 uv[NV];
     float2 tv[4];  // working tile, C layout: rows 4 g4 + i, columns 32 wave + 2q, + 1
     const int tc = 32 * wave + 2 * q;
-    uint32_t own = 0;  // bit i: row 4 g4 + i is of this run
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int rr = 4 * g4 + i;
-      const int gi = row_grp[rbase + (rr < nrows ? rr : nrows - 1)];
-      own |= (rr < nrows && gi >= g && gi <= ge ? 1u : 0u) << i;
-    }
     // block b's U block, block map and working tile
     auto fetch = [&](int b) {
       const int64_t i1 = i0 + (int64_t)b * LMAX;
@@ -710,17 +704,6 @@ __global__ __launch_bounds__(RPG * QL, 1) void gptq_super_kernel(
       __syncthreads();
       load_tile_row<COMP>(R, wt + lr * WSTR, q);
       load_row_c<COMP>(R, L, su, q);
-      // the tile goes back to wc as the separate updates leave it (its stores and the next
-      // block's loads are in flight during the loop)
-      if (b > 0) {
-        const __amdgpu_buffer_rsrc_t wr = mg_rsrc(wc + rbase * K + i1, (int64_t)(nrows - 1) * K + L);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          __builtin_amdgcn_raw_buffer_store_b64(
-              __builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned, tv[i]), wr,
-              (int)(tc < L && (own >> i & 1) ? (uint32_t)(((int64_t)(4 * g4 + i) * K + tc) * 4)
-                                             : MG_OOB), 0, 0);
-      }
       if (b + 1 < nblk) fetch(b + 1);
       // the U panel of the next near update, rows of blocks 0 .. b, into this XCD's L2 while the
       // loop runs: each of its workgroups (blockIdx % 8) touches its share of the 128-byte lines
@@ -755,6 +738,14 @@ __global__ __launch_bounds__(RPG * QL, 1) void gptq_super_kernel(
                                 ldp, su, q, nm, eb, lde, codes, comp, wt + lr * WSTR);
         else
           store_row<COMP>(R, K, i1, L, r, q, eb, lde, codes, comp);
+        // the row's tile goes back to wc as the separate updates leave it
+        if (b > 0) {
+#pragma unroll
+          for (int c = 4 * q; c < LMAX; c += 4 * QL)
+            if (c < L)
+              *reinterpret_cast<f32x4u*>(wc + r * K + i1 + c) =
+                  *reinterpret_cast<const f32x4g*>(wt + lr * WSTR + c);
+        }
       }
 #pragma unroll
       for (int m = 0; m < CPL; ++m) et[lr * ESTR + b * LMAX + QL * m + q] = R.er[m];
