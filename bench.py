@@ -344,6 +344,31 @@ def _encode_block(xs, ws, masks, timer=None, lanes=None, keep=None, cfg=CFG3):
     return out
 
 
+def cross_block_flops(shapes) -> float:
+    """Algorithmic flops of every cross-block update of rounding ``(rows, K)`` tensors, on the
+    real rows: per tensor, sum over 128-column blocks of 2 N 128 (K - i2)."""
+    total = 0.0
+    for n, k in shapes:
+        for i1 in range(0, k, 128):
+            i2 = min(i1 + 128, k)
+            total += 2.0 * n * (i2 - i1) * (k - i2)
+    return total
+
+
+def trailing_rate(n, ms, work, shapes) -> dict:
+    """The rate of the trailing update's ``n`` launches over their own flops (``work``, at most
+    those of the real rows: zero rows that align factor runs do not count) and durations, beside
+    all cross-block flops of the step: the difference, the near updates of batches of up to 4096
+    rows, runs inside gptq_super_kernel's launches."""
+    total = cross_block_flops(shapes)
+    work = min(work, total)
+    return {"bound": "mfma", "achieved": work / ms / 1e9, "peak": PEAK_F32 / 1e12,
+            "unit": "TFLOP/s", "frac": work / ms / 1e9 / (PEAK_F32 / 1e12),
+            "flops_per_step": work, "launches_per_step": n,
+            "cross_block_flops_per_step": total,
+            "flops_in_column_loops_per_step": total - work}
+
+
 def stage_breakdown(xs, ws, masks, cfg=CFG3):
     """One step run serially on one stream with every stage timed: per input its Hessian,
     transform and factor (stream events), per linear its rotation, ladder fit, column
@@ -456,8 +481,6 @@ def block_leg(cfg, dev, steps, warmup):
     sp = _lib.timing_query(11)
     _lib.timing_enable([])
     per_input, per_linear, rates = stage_breakdown(xs, ws, masks, cfg)
-    flops = tr[2]
-    trail_ms = tr[1]  # one step's launches
     res = {
         "workload": f"{cfg['name']}: " + ", ".join(f"{n} {r}x{k}" for n, r, k, _ in cfg["linears"])
                     + f"; {cfg['tokens']} tokens; "
@@ -465,14 +488,12 @@ def block_leg(cfg, dev, steps, warmup):
         "steps": steps,
         "ms_per_step": ms,
         "ms_per_linear": ms / len(cfg["linears"]),
-        "trailing_roofline": {"bound": "mfma", "achieved": flops / trail_ms / 1e9,
-                              "peak": PEAK_F32 / 1e12, "unit": "TFLOP/s",
-                              "frac": flops / trail_ms / 1e9 / (PEAK_F32 / 1e12),
-                              "flops_per_step": flops, "launches_per_step": tr[0],
-                              "timing": "event-timed launches in the last timed step (chains "
-                                        "concurrent)"},
+        "trailing_roofline": dict(trailing_rate(*tr, [(n, k) for _, n, k, _ in cfg["linears"]]),
+                                  timing="event-timed launches in the last timed step (chains "
+                                         "concurrent)"),
         "syrk_tflops_executed": sy[2] / sy[1] / 1e9 if sy[1] > 0 else None,
-        "factor_fp32_gemm_tflops": ch[2] / ch[1] / 1e9 if ch[1] > 0 else None,
+        "factor_planes_tflops_executed": small_products()[0] * ch[2] / ch[1] / 1e9
+        if ch[1] > 0 else None,
         "factor_split_fp16_tflops_executed": sp[2] / sp[1] / 1e9 if sp[1] > 0 else None,
         "stages_serial_ms": {"per_input": per_input, "per_linear": per_linear},
         "hbm_kernels": rates,
@@ -632,8 +653,6 @@ def moe_leg(dev, steps, warmup):
     encode_moe(*inp, timer=timer)
     stages = timer.summary()["moe"]
     counts = torch.bincount(inp[0].reshape(-1), minlength=E5).cpu().tolist()
-    flops = tr[2]
-    trail_ms = tr[1]  # one step's launches
     res = {
         "workload": "cfg5: OLMoE-shaped MoE layer, 64 experts (gate/up 1024x2048 sharing a "
                     "Hessian, down 2048x1024), top-8 of 16384 tokens routed by Zipf(1.1) "
@@ -645,10 +664,8 @@ def moe_leg(dev, steps, warmup):
                                      "max": max(counts)},
         "experts_below_floor": sum(c < int(FLOOR5 * H5) for c in counts),
         "stages_ms": stages,
-        "trailing_roofline": {"bound": "mfma", "achieved": flops / trail_ms / 1e9,
-                              "peak": PEAK_F32 / 1e12, "unit": "TFLOP/s",
-                              "frac": flops / trail_ms / 1e9 / (PEAK_F32 / 1e12),
-                              "flops_per_step": flops, "launches_per_step": tr[0]},
+        # per expert gate/up 2 x 1024 rows at K = 2048, down 2048 rows at K = 1024
+        "trailing_roofline": trailing_rate(*tr, [(E5 * 2 * I5, H5), (E5 * H5, I5)]),
         "grouped_syrk": {"launches_per_step": sy[0], "ms_per_step": sy[1],
                          "tflops_executed": sy[2] / sy[1] / 1e9 if sy[1] > 0 else None},
         "factor_ms_per_step_kernels": ch[1] + lf[1] + sp[1],
@@ -772,12 +789,20 @@ class StageTimer:
                 for n, h, e in self.points}
 
 
+def small_products():
+    """What the factor's small products execute per flop the library counts (M*N*rank, one
+    operand triangular): ``(factor, peak, work unit)``."""
+    if os.environ.get("HI2X_CHOL_FP32", "0") not in ("", "0"):
+        return 1.0, PEAK_F32, "M*N*rank fp32 MFMA flops"
+    return 6.0, PEAK_BF16, ("6*M*N*rank bf16 MFMA flops executed (six products of three bf16 "
+                            "planes per fp32-equivalent product of one triangular operand)")
+
+
 # kernel families timed by the library (hi2x_timing_*), with the peak that bounds each
 KERNELS = {  # kind -> (kernel, bound, peak FLOP/s, work unit)
     0: ("gptq_trailing_kernel", "mfma", PEAK_F32, "2*rows*rank*cols"),
     1: ("syrk2_kernel", "mfma", PEAK_BF16, "T*K*(K+1) (upper triangle, 2 flops per product)"),
-    2: ("tri_gemm_kernel", "mfma", PEAK_F32, "M*N*rank (one triangular operand; the "
-        "factor's fp32 MFMA products)"),
+    2: ("tri_gemm_kernel/tri_gemm_pair_kernel (64-tiles)", "mfma", *small_products()[1:]),
     11: ("gemm3_kernel/gemm3x_kernel (split planes)", "mfma", PEAK_BF16,
          "3*M*N*rank fp16 MFMA flops executed (three fp16 products per fp32-equivalent "
          "product of one triangular operand)"),
@@ -802,6 +827,8 @@ def kernel_stats(kind):
     n, ms, work = _lib.timing_query(kind)
     if n == 0 or ms <= 0.0:
         return None
+    if kind == 2:
+        work *= small_products()[0]
     rate = work / (ms / 1e3)
     out = {"kernel": name, "bound": bound, "launches": n, "avg_ms": ms / n,
            "total_ms": ms, "work_per_launch": work / n, "work_unit": unit,
@@ -814,18 +841,20 @@ def kernel_stats(kind):
     return out
 
 
-def pmc_traffic(kernel):
+def pmc_traffic(kernel, launches):
     """HBM bytes per launch of ``kernel`` (read + write) from the committed counter
     summary (profiles/traffic.json: rocprofv3 FETCH_SIZE and WRITE_SIZE passes over this
     bench's step, each scaled by what the counter reads for a 1 GiB device copy), with the
-    split; None when the summary or the kernel is absent."""
+    split; None when the summary or the kernel is absent, or when the summary was taken
+    with another number of launches per step than the ``launches`` of this run."""
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", "traffic.json")
     try:
         with open(path) as f:
-            e = json.load(f).get(kernel)
-    except (OSError, ValueError):
+            prof = json.load(f)
+            e, steps = prof.get(kernel), prof["_run"]["encodes"]
+    except (OSError, ValueError, KeyError):
         return None, None
-    if not e:
+    if not e or e["dispatches"] != launches * steps:
         return None, None
     rd, wr = e["fetch_bytes_per_launch"], e["write_bytes_per_launch"]
     return rd + wr, {"read_bytes": rd, "write_bytes": wr, "dispatches": e["dispatches"],
@@ -833,24 +862,19 @@ def pmc_traffic(kernel):
                                "WRITE_SIZE, averaged over the step's launches)"}
 
 
-def trailing_roofline(steps, basis):
-    """The trailing update's roofline over the last timing window: the algorithmic flops
-    of its launches (the near updates of batches of up to 4096 rows run inside the column
-    loops' launches and are not among them) divided by their summed event-timed durations;
-    ``traffic`` from the committed PMC summary."""
+def trailing_roofline(basis):
+    """The trailing update's roofline over one step (the last timing window): the flops of
+    its launches divided by their summed event-timed durations (trailing_rate); ``traffic``
+    from the committed PMC summary."""
     from hi2_amd import _lib
 
     n, ms, work = _lib.timing_query(DOMINANT)
-    flops = work
-    rate = flops / (ms / 1e3)
-    traffic, split = pmc_traffic(KERNELS[DOMINANT][0])
-    return {"bound": "mfma", "achieved": rate / 1e12, "peak": PEAK_F32 / 1e12,
-            "unit": "TFLOP/s", "frac": rate / PEAK_F32, "traffic": traffic,
-            "traffic_split": split,
-            "kernel": KERNELS[DOMINANT][0], "launches": n, "avg_ms": ms / n,
-            "flops_per_launch": flops / n,
-            "work": "2*rows*rank*cols summed over the cross-block update launches",
-            "timing": basis}
+    traffic, split = pmc_traffic(KERNELS[DOMINANT][0], n)
+    rate = trailing_rate(n, ms, work, [(r, k) for _, r, k, _ in LINEARS])
+    return dict(rate, traffic=traffic, traffic_split=split, kernel=KERNELS[DOMINANT][0],
+                launches=n, avg_ms=ms / n, flops_per_launch=rate["flops_per_step"] / n,
+                work="2*rows*rank*cols summed over the cross-block update launches",
+                timing=basis)
 
 
 def _cpu_info():
@@ -1121,6 +1145,7 @@ def micro(which, reps=3):
         for kd in kinds:
             n, kms, work = _lib.timing_query(kd)
             name, bound, peak, unit = KERNELS[kd]
+            work *= small_products()[0] if kd == 2 else 1.0
             stats[name] = {"launches": n // reps, "ms": kms / reps,
                            "tflops": work / kms / 1e9 if kms > 0 and work > 0 else None,
                            "frac_of_peak": work / kms / 1e9 / (peak / 1e12)
@@ -1351,7 +1376,7 @@ def main():
     ms_step = wall * 1e3 / args.steps
     stages = timer.summary()
     host_points = timer.host_points()
-    roof = trailing_roofline(1, "contended: event-timed launches of the last timed step, "
+    roof = trailing_roofline("contended: event-timed launches of the last timed step, "
                              "where the four input chains run concurrently")
     # one more, untimed step with every kernel family event-timed and the chains run one
     # after another on one stream: per-kernel rates without other chains sharing the GPU
@@ -1359,7 +1384,7 @@ def main():
     encode_block(xs, ws, masks, lanes=[CFG3["order"]])
     torch.cuda.synchronize()
     kernels = {KERNELS[k][0]: kernel_stats(k) for k in KERNELS}
-    roof_iso = trailing_roofline(1, "isolated: one step with the chains run one after "
+    roof_iso = trailing_roofline("isolated: one step with the chains run one after "
                                  "another on one stream")
     _lib.timing_enable([])
     per_input, per_linear, hbm = stage_breakdown(xs, ws, masks)
