@@ -1305,8 +1305,9 @@ int g3_pair(const G3Args& a1, const G3Args& a2, hipStream_t s, int batch) {
 }
 
 // Products of the big grids: fp16 MFMA on the two scaled split planes (default); of the small
-// ones: bf16 MFMA on three planes.  HI2X_CHOL_FP32 set to a nonzero value runs all of them on
-// the fp32 MFMA (read once per process).
+// ones: bf16 MFMA on three planes.  HI2X_CHOL_FP32 set to a nonzero value runs these products
+// between nodes on the fp32 MFMA (read once per process); the updates inside a node are on
+// three bf16 planes either way.
 static bool chol_split() {
   static const bool split = [] {
     const char* e = getenv("HI2X_CHOL_FP32");
@@ -1515,7 +1516,8 @@ __global__ __launch_bounds__(256) void reverse_damp4_kernel(const float* __restr
 // others apply the update.  A 256-column node takes 39 us and a 128-column one 27 (84-88
 // and 31 us as recursive 16/32/64/128-column halves in 135 KB of LDS, whose sweeps, small
 // products and barriers followed one another); with 26 KB of LDS it also finds a CU beside
-// another stream's GEMM workgroups.
+// another stream's GEMM workgroups, and beside gptq_super_kernel's of four blocks (107 KB), not
+// of eight (139 KB of a CU's 160).
 //
 // The 16 x 16 sweep is one wave's fused factor-and-invert of the symmetric tile, lane 16 g + i
 // holding columns 4g .. 4g + 3 of row i (the C layout, by symmetry).  For c = 0..15, with
@@ -1910,14 +1912,16 @@ struct Ctx {
 constexpr int split_mask_b(int bmode) { return bmode == 1 ? 2 : (bmode == 2 ? 1 : 0); }
 
 // Whether a product runs through the split planes: grids of at least 128 tiles of 128,
-// a lower-triangular output from 96 (14 x 14 tiles: the fp16 split's three MFMAs per 16 k
-// on 105 tiles beat the fp32 MFMA's 406 tiles of 64).
+// a lower-triangular output from 96 (14 x 14 tiles).  Against 64-tiles on bf16 planes, a whole
+// factor: K = 3584 1443 us, 1545 with a line of 121 for the triangle; K = 4096 1621, 1759 with
+// 257 and 137.  Below the lines it depends on the size: with 100 and 78, K = 3072 1331 -> 1250
+// and K = 6144 3278 -> 3113, K = 2560 956 -> 985.
 static bool split_worth(int64_t tm, int64_t tn, bool clow) {
   return clow ? tm * (tm + 1) / 2 >= 96 : tm * tn >= 128;
 }
 
-// One product of the recursion: the big grids through the split planes, the small ones
-// on the fp32 MFMA GEMM.
+// One product of the recursion: the big grids through the split planes, the small ones on
+// 64-tiles of three bf16 planes (tri_gemm).
 template <int AMODE, int BMODE, bool TB, bool CLOW>
 int product(const Ctx& c, GemmArgs a) {
   const int64_t tm = (a.M + MG_T - 1) / MG_T, tn = (a.N + MG_T - 1) / MG_T;
@@ -1945,7 +1949,7 @@ int product(const Ctx& c, GemmArgs a) {
 }
 
 // The split-plane tile edge a product runs on (as product() and gemm3() decide): 256,
-// 128, or 0 when it takes the fp32 path.
+// 128, or 0 when it is tri_gemm's.
 static int split_tile(const GemmArgs& a, bool clow) {
   const int64_t tm = (a.M + MG_T - 1) / MG_T, tn = (a.N + MG_T - 1) / MG_T;
   if (!chol_split() || !split_worth(tm, tn, clow)) return 0;

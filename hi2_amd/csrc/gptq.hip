@@ -573,7 +573,11 @@ __global__ __launch_bounds__(256, T == MG_T ? 2 : 4) void gptq_trailing_kernel(
 // block's U, block map and working tile are in flight during the loop.  Alone, the super-blocks of
 // 1024 x 4096 take 58 us of four blocks (897 us of column loops and near updates for the
 // matrix as separate launches, 465 here), those of 4096 x 14336 150 us of eight (2997 and
-// 2100); the whole encode of these 1086 -> 908 and 10480 -> 9520 us.
+// 2100); the whole encode of these 1088 -> 912 and 10454 -> 9492 us (906 and 9485 without
+// writing the tiles back to wc).
+// A lane holds 256 VGPRs, and 67-72 scalars of pointers and buffer descriptors past the 106 SGPRs
+// lie in VGPR lanes (no scratch memory); the launch takes 107 KB of LDS with four blocks' errors
+// and 139 KB with eight.
 // One workgroup per CU (its errors stay in LDS), so it is for batches that fill no more than
 // one round of the CUs: FUSED_ROWS rows.  Beyond, two workgroups per CU of the separate column
 // loops hide each other's latency, and the near updates read each U tile once per 64 rows

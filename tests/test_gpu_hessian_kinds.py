@@ -220,6 +220,23 @@ def test_16_bit_passes(t, k, dtype, dev):
             assert torch.equal(s.double().triu(), want.triu())
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("t,k", [(500, 1040), (70, 37), (0, 48)])
+def test_upper_entry(t, k, dtype, dev):
+    """``hi2x_hessian_syrk_upper`` leaves the upper triangle of ``hi2x_hessian_syrk``."""
+    from hi2_amd import _lib
+
+    x = _x(max(t, 1), k, dtype, dev, t + k)[:t].contiguous()
+    code = 2 if dtype == torch.bfloat16 else 0
+    ws = _lib.workspace(dev, "hi2x_hessian_workspace_bytes", code, t, k)
+    out = []
+    for name in ("hi2x_hessian_syrk", "hi2x_hessian_syrk_upper"):
+        s = torch.ones(k, k, device=dev)
+        _lib.call(name, x.device, _lib.ptr(x), code, t, k, _lib.ptr(s), _lib.ptr(ws), ws.numel())
+        out.append(s.triu())
+    assert torch.equal(*out)
+
+
 def test_fp16_specials(dev):
     """fp16 infinities, NaN and subnormals multiply as their fp32 values do."""
     from hi2_amd.hessian import HessianStats

@@ -779,7 +779,8 @@ def test_transformed_equals_transform_of_mean(dev, k, smooth):
 
 
 def test_upper_update_then_mirror_equals_full_update(dev):
-    """hi2x_hessian_syrk_upper + the mirror on first read of S == hi2x_hessian_syrk."""
+    """HessianStats.update (hi2x_hessian_accumulate, the upper triangle) + the mirror on first
+    read of S == hi2x_hessian_syrk."""
     from hi2_amd import _lib
     from hi2_amd.hessian import HessianStats
 
