@@ -226,7 +226,9 @@ class _StoredDecode(torch.autograd.Function):
 
 
 class _Transform(torch.autograd.Function):
-    """``H(x) / scale`` over the flagged 16-column groups; the backward is ``H(grad / scale)``."""
+    """``H(x) / scale`` over the flagged 16-column groups; the backward is ``H(grad / scale)``.
+    :func:`original` fuses it with the decode (``_Weights``); it is here for code written against
+    the reference's module."""
 
     @staticmethod
     def forward(ctx, x, flags, scale):
