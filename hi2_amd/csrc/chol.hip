@@ -39,7 +39,9 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2v __attribute__((ext_vector_type(2)));
 
 // Three bf16 planes of a pair of values, x1 = bf16(x), x2 = bf16(x - x1), x3 = bf16(x - x1 - x2)
-// (the differences are exact in fp32; bf16 has fp32's exponent range, so no scale is needed):
+// (the differences are exact in fp32, and the planes are all of x from 2^-110 up; bf16 has fp32's
+// exponent range, so no scale is needed: below, the third plane loses bits, which only a
+// Hessian of that size without damping can notice, damping keeping its diagonal above 1e-12 damp):
 // v_cvt_pk_bf16_f32 makes a plane of the pair, and a bf16 back to fp32 is its bits in the upper
 // half.
 __device__ __forceinline__ void split_pair(float a, float b, uint32_t (&o)[3]) {
